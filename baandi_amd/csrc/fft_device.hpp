@@ -55,10 +55,82 @@ __host__ __device__ constexpr int pass_mb(int R, int NT) {
                   : 2;  // R == 9
 }
 
+template <int R, bool INV, typename T>
+__host__ __device__ __forceinline__ void dft(c2<T>* v);
+
+// DFT of length A B for coprime A, B without twiddles (Good 1958, Thomas
+// 1963): input index B n1 + A n2, output index congruent to k1 mod A and to
+// k2 mod B, both mod A B.
+template <int A, int B, bool INV, typename T>
+__host__ __device__ __forceinline__ void dft_coprime(c2<T>* v) {
+  constexpr int N = A * B;
+  auto inverse = [](int x, int m) constexpr {
+    for (int i = 1; i < m; ++i)
+      if (x * i % m == 1) return i;
+    return 1;
+  };
+  constexpr int ka = B * inverse(B % A, A), kb = A * inverse(A % B, B);
+  c2<T> t[B][A];
+#pragma unroll
+  for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+    for (int n1 = 0; n1 < A; ++n1) t[n2][n1] = v[(B * n1 + A * n2) % N];
+    dft<A, INV>(t[n2]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < A; ++k1) {
+    c2<T> row[B];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) row[n2] = t[n2][k1];
+    dft<B, INV>(row);
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) v[(ka * k1 + kb * k2) % N] = row[k2];
+  }
+}
+
 // In-register DFT of length R with root e^{-2 pi i/R} (e^{+} for INV).
 template <int R, bool INV, typename T>
 __host__ __device__ __forceinline__ void dft(c2<T>* v) {
-  if constexpr (R == 2) {
+  if constexpr (R == 6) {
+    dft_coprime<2, 3, INV>(v);
+  } else if constexpr (R == 10) {
+    dft_coprime<2, 5, INV>(v);
+  } else if constexpr (R == 12) {
+    dft_coprime<4, 3, INV>(v);
+  } else if constexpr (R == 15) {
+    dft_coprime<3, 5, INV>(v);
+  } else if constexpr (R == 16) {
+    // 4 x 4: column DFTs over v[n1 + 4 n2], twiddles w^(n1 k1), row DFTs;
+    // X[k1 + 4 k2]. w = e^{-2 pi i/16} (e^{+} for INV).
+    const T h = T(0.70710678118654752440084436210484904);  // cos(pi/4)
+    const T c = T(0.92387953251128675612818318939678829);  // cos(pi/8)
+    const T s = T(0.38268343236508977172845998403039887);  // sin(pi/8)
+    const T sg = INV ? T(1) : T(-1);
+    c2<T> col[4][4];
+#pragma unroll
+    for (int n1 = 0; n1 < 4; ++n1) {
+#pragma unroll
+      for (int n2 = 0; n2 < 4; ++n2) col[n1][n2] = v[n1 + 4 * n2];
+      dft<4, INV>(col[n1]);
+    }
+    const c2<T> w1{c, sg * s}, w2{h, sg * h}, w3{s, sg * c}, w6{-h, sg * h}, w9{-c, -sg * s};
+    col[1][1] = cmul(col[1][1], w1);
+    col[1][2] = cmul(col[1][2], w2);
+    col[1][3] = cmul(col[1][3], w3);
+    col[2][1] = cmul(col[2][1], w2);
+    col[2][2] = rot_i<INV>(col[2][2]);
+    col[2][3] = cmul(col[2][3], w6);
+    col[3][1] = cmul(col[3][1], w3);
+    col[3][2] = cmul(col[3][2], w6);
+    col[3][3] = cmul(col[3][3], w9);
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+      c2<T> row[4] = {col[0][k1], col[1][k1], col[2][k1], col[3][k1]};
+      dft<4, INV>(row);
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = row[k2];
+    }
+  } else if constexpr (R == 2) {
     c2<T> a = v[0], b = v[1];
     v[0] = cadd(a, b);
     v[1] = csub(a, b);

@@ -362,6 +362,8 @@ extern "C" bd_status bd_gamma_op_autotune(bd_gamma_op* h, int32_t m, int32_t rep
           const bool useful = c == p.n1 || (c % 4 == 0) || c == 1;
           if (useful && o.plane_shape_valid(t, c)) cands.push_back({t, c});
         }
+      // The paired plane pass does not use the shape: only its time is taken.
+      if (o.pair.on && !o.kb) cands.assign(1, {o.plane_threads, p.chunk});
       if (cands.empty()) bd::fail(BD_ERR_APPLICATION, "no valid plane shape");
       BD_HIP(hipMemsetAsync(o.d_x.p, 0, size_t(o.n) * m * 8, o.stream));
       hipEvent_t a, z;

@@ -68,7 +68,7 @@ template <typename F>
 __global__ __launch_bounds__(kThreads) void k_stick_inverse(
     const double* __restrict__ x, int64_t ldx, int m, int n0, int T, int Spad,
     const int* __restrict__ tile_off, const int4* __restrict__ entries,
-    const c2<double>* __restrict__ roots_x, RadixPlan rx, c2<F>* __restrict__ sticks) {
+    const int* __restrict__ dst, const c2<double>* __restrict__ roots_x, RadixPlan rx, c2<F>* __restrict__ sticks) {
   extern __shared__ char smem[];
   c2<F>* L = reinterpret_cast<c2<F>*>(smem);
   c2<F>* rt = L + T * n0;
@@ -94,10 +94,11 @@ __global__ __launch_bounds__(kThreads) void k_stick_inverse(
   }
   __syncthreads();
   lds_fft<true>(L, T, n0, 1, rx, rt);
-  c2<F>* out = sticks + int64_t(t) * n0 * Spad + int64_t(tile) * T;
+  c2<F>* out = sticks + int64_t(t) * n0 * Spad;
+  dst += tile * T;
   for (int e = threadIdx.x; e < T * n0; e += blockDim.x) {
     const int xi = e / T, slot = e - xi * T;
-    out[int64_t(xi) * Spad + slot] = L[slot * n0 + xi];
+    out[int64_t(xi) * Spad + dst[slot]] = L[slot * n0 + xi];
   }
 }
 
@@ -106,16 +107,17 @@ template <typename F>
 __global__ __launch_bounds__(kThreads) void k_stick_forward(
     const double* __restrict__ x, int64_t ldx, double* __restrict__ y, int64_t ldy, int m,
     int n0, int T, int Spad, const int* __restrict__ tile_off, const int4* __restrict__ entries,
-    const c2<double>* __restrict__ roots_x, RadixPlan rx, const c2<F>* __restrict__ sticks,
+    const int* __restrict__ dst, const c2<double>* __restrict__ roots_x, RadixPlan rx, const c2<F>* __restrict__ sticks,
     const double* __restrict__ kinetic, double inv_n, int accumulate) {
   extern __shared__ char smem[];
   c2<F>* L = reinterpret_cast<c2<F>*>(smem);
   c2<F>* rt = L + T * n0;
   const int tile = blockIdx.x, t = blockIdx.y;
-  const c2<F>* in = sticks + int64_t(t) * n0 * Spad + int64_t(tile) * T;
+  const c2<F>* in = sticks + int64_t(t) * n0 * Spad;
+  dst += tile * T;
   for (int e = threadIdx.x; e < T * n0; e += blockDim.x) {
     const int xi = e / T, slot = e - xi * T;
-    L[slot * n0 + xi] = in[int64_t(xi) * Spad + slot];
+    L[slot * n0 + xi] = in[int64_t(xi) * Spad + dst[slot]];
   }
   stage_roots(rt, roots_x, n0);
   __syncthreads();
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kThreads) void k_stick_forward(
 template <typename F>
 __global__ __launch_bounds__(kThreads) void k_kstick_inverse(
     const double* __restrict__ x, int64_t ldx, int n0, int T, int Spad, const int* __restrict__ tile_off,
-    const int4* __restrict__ entries, const c2<double>* __restrict__ roots_x, RadixPlan rx,
+    const int4* __restrict__ entries, const int* __restrict__ dst, const c2<double>* __restrict__ roots_x, RadixPlan rx,
     c2<F>* __restrict__ sticks) {
   extern __shared__ char smem[];
   c2<F>* L = reinterpret_cast<c2<F>*>(smem);
@@ -194,10 +196,11 @@ __global__ __launch_bounds__(kThreads) void k_kstick_inverse(
   }
   __syncthreads();
   lds_fft<true>(L, T, n0, 1, rx, rt);
-  c2<F>* out = sticks + int64_t(t) * n0 * Spad + int64_t(tile) * T;
+  c2<F>* out = sticks + int64_t(t) * n0 * Spad;
+  dst += tile * T;
   for (int e = threadIdx.x; e < T * n0; e += blockDim.x) {
     const int xi = e / T, slot = e - xi * T;
-    out[int64_t(xi) * Spad + slot] = L[slot * n0 + xi];
+    out[int64_t(xi) * Spad + dst[slot]] = L[slot * n0 + xi];
   }
 }
 
@@ -205,16 +208,18 @@ __global__ __launch_bounds__(kThreads) void k_kstick_inverse(
 template <typename F>
 __global__ __launch_bounds__(kThreads) void k_kstick_forward(
     const double* __restrict__ x, int64_t ldx, double* __restrict__ y, int64_t ldy, int n0, int T, int Spad,
-    const int* __restrict__ tile_off, const int4* __restrict__ entries, const c2<double>* __restrict__ roots_x,
-    RadixPlan rx, const c2<F>* __restrict__ sticks, const double* __restrict__ kinetic, double inv_n) {
+    const int* __restrict__ tile_off, const int4* __restrict__ entries, const int* __restrict__ dst,
+    const c2<double>* __restrict__ roots_x, RadixPlan rx, const c2<F>* __restrict__ sticks,
+    const double* __restrict__ kinetic, double inv_n) {
   extern __shared__ char smem[];
   c2<F>* L = reinterpret_cast<c2<F>*>(smem);
   c2<F>* rt = L + T * n0;
   const int tile = blockIdx.x, t = blockIdx.y;
-  const c2<F>* in = sticks + int64_t(t) * n0 * Spad + int64_t(tile) * T;
+  const c2<F>* in = sticks + int64_t(t) * n0 * Spad;
+  dst += tile * T;
   for (int e = threadIdx.x; e < T * n0; e += blockDim.x) {
     const int xi = e / T, slot = e - xi * T;
-    L[slot * n0 + xi] = in[int64_t(xi) * Spad + slot];
+    L[slot * n0 + xi] = in[int64_t(xi) * Spad + dst[slot]];
   }
   stage_roots(rt, roots_x, n0);
   __syncthreads();
@@ -509,6 +514,49 @@ RadixPlan radix_plan(int n, bool big) {
   return rp;
 }
 
+// Order the occupied sticks (z, y) line by line, lines cyclically in z and
+// the sticks of a line cyclically in y, each from the first occupied index
+// after an empty one, and fill the plan's lines. Where the lines or the sticks
+// of a line are not one such run, the lines stay empty and the order is (z, y).
+static void order_sticks(StickPlan& p, std::vector<std::pair<int, int>>& sticks) {
+  // The start of the one cyclic run of `on`, -1 if there are several.
+  auto run_start = [](const std::vector<char>& on) {
+    const int n = int(on.size());
+    int start = -1, starts = 0;
+    for (int i = 0; i < n; ++i)
+      if (on[i] && !on[(i + n - 1) % n]) {
+        start = i;
+        ++starts;
+      }
+    return starts == 0 ? 0 : starts == 1 ? start : -1;
+  };
+  std::map<int, std::vector<char>> rows;
+  std::vector<char> zon(p.n2, 0);
+  for (auto& k : sticks) {
+    zon[k.first] = 1;
+    rows.emplace(k.first, std::vector<char>(p.n1, 0)).first->second[k.second] = 1;
+  }
+  const int zs = run_start(zon);
+  if (zs < 0) return;
+  std::vector<std::pair<int, int>> sorted;
+  std::vector<PlaneLine> lines;
+  for (int i = 0; i < p.n2; ++i) {
+    const int z = (zs + i) % p.n2;
+    if (!zon[z]) continue;
+    const auto& on = rows[z];
+    const int ys = run_start(on);
+    if (ys < 0) return;
+    PlaneLine l{int(sorted.size()), ys, 0, 0};
+    for (int j = 0; j < p.n1; ++j)
+      if (on[(ys + j) % p.n1]) sorted.push_back({z, (ys + j) % p.n1});
+    l.count = int(sorted.size()) - l.first;
+    lines.push_back(l);
+  }
+  sticks = std::move(sorted);
+  p.zs = zs;
+  p.lines = std::move(lines);
+}
+
 StickPlan build_stick_plan(const System& s) {
   StickPlan p{};
   p.n0 = s.dims[0];
@@ -531,6 +579,7 @@ StickPlan build_stick_plan(const System& s) {
       keys.insert({c, b});
     }
   std::vector<std::pair<int, int>> sticks(keys.begin(), keys.end());
+  order_sticks(p, sticks);
   p.S = int(sticks.size());
   std::map<std::pair<int, int>, int> index;
   for (int i = 0; i < p.S; ++i) index[sticks[i]] = i;
@@ -578,8 +627,14 @@ StickPlan build_stick_plan(const System& s) {
   p.ntiles = tile + 1;
   p.Spad = p.ntiles * p.T;
   p.stick_yz.assign(p.Spad, make_int2(-1, -1));
-  for (int i = 0; i < p.S; ++i)
-    p.stick_yz[tile_of[i] * p.T + slot_of[i]] = make_int2(sticks[i].second, zc_of[sticks[i].first]);
+  p.stick_dst.assign(p.Spad, -1);
+  for (int i = 0; i < p.S; ++i) {
+    p.stick_yz[i] = make_int2(sticks[i].second, zc_of[sticks[i].first]);
+    p.stick_dst[tile_of[i] * p.T + slot_of[i]] = i;
+  }
+  int pads = p.S;  // the padding slots behind the sticks
+  for (int& d : p.stick_dst)
+    if (d < 0) d = pads++;
   // Representative entries grouped by tile.
   std::vector<std::vector<int4>> per(p.ntiles);
   for (int64_t r = 0; r < s.nrep; ++r) {
@@ -621,6 +676,7 @@ StickPlan build_k_stick_plan(const System& s, const KBasis& kb) {
     keys.insert({c, b});
   }
   std::vector<std::pair<int, int>> sticks(keys.begin(), keys.end());
+  order_sticks(p, sticks);
   p.S = int(sticks.size());
   std::map<std::pair<int, int>, int> index;
   for (int i = 0; i < p.S; ++i) index[sticks[i]] = i;
@@ -644,6 +700,8 @@ StickPlan build_k_stick_plan(const System& s, const KBasis& kb) {
   p.Spad = p.ntiles * p.T;
   p.stick_yz.assign(p.Spad, make_int2(-1, -1));
   for (int i = 0; i < p.S; ++i) p.stick_yz[i] = make_int2(sticks[i].second, zc_of[sticks[i].first]);
+  p.stick_dst.resize(p.Spad);
+  std::iota(p.stick_dst.begin(), p.stick_dst.end(), 0);
   std::vector<std::vector<int4>> per(p.ntiles);
   for (int64_t g = 0; g < kb.nk; ++g) {
     int a, b, c;
@@ -702,7 +760,8 @@ void GammaOp::enable_split(int zb) {
   const int pairs = slots(capacity);
   int batch = int(std::max<size_t>(1, (size_t(2) << 30) / plane));
   batch = std::min(pairs, std::max(batch, kDensityGroups));
-  if (d_planes.n < (size_t(batch) * plane + 15) / 16) {
+  // (Gamma ops on the paired pass move no plane through HBM.)
+  if ((kb || !pair.on) && d_planes.n < (size_t(batch) * plane + 15) / 16) {
     DevBuf<c2<double>> fresh;
     fresh.alloc((size_t(batch) * plane + 15) / 16);
     std::swap(d_planes.p, fresh.p);
@@ -797,6 +856,15 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   d_entries.upload(plan.entries.data(), plan.entries.size(), stream);
   d_stick_yz.alloc(plan.stick_yz.size());
   d_stick_yz.upload(plan.stick_yz.data(), plan.stick_yz.size(), stream);
+  d_stick_dst.alloc(plan.stick_dst.size());
+  d_stick_dst.upload(plan.stick_dst.data(), plan.stick_dst.size(), stream);
+  if (!plan.lines.empty()) pair = pair_shape(plan.n1, plan.n2, plan.Z, elem);
+  if (pair.on) {
+    d_lines.alloc(plan.lines.size());
+    d_lines.upload(plan.lines.data(), plan.lines.size(), stream);
+    if (fft32()) pair_allow_lds<float>(pair);
+    else pair_allow_lds<double>(pair);
+  }
   d_zc.alloc(plan.z_of_zc.size());
   d_zc.upload(plan.z_of_zc.data(), plan.z_of_zc.size(), stream);
   d_kinetic.alloc(n);
@@ -816,6 +884,7 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   }
   const int pairs = slots(cap);
   d_sticks.alloc(size_t(pairs) * plan.n0 * plan.Spad);
+  if (pair.on && pair.split > 1 && !kb) d_sticks2.alloc(size_t(pairs) * plan.n0 * plan.Spad);
   // Planes that do not fit one workgroup go through the split pass.
   if (!fft_fits(plan.Z, plan.ry) || plane_lds(plan, elem) > lds_max) enable_split(0);
   // Host-pointer entry points stage through these (no allocation after create).
@@ -899,6 +968,24 @@ void GammaOp::split_pass(int pairs, const F* pot, const double* w, double* rho_p
 }
 
 template <typename F>
+PairArgs<F> GammaOp::pair_args(int pairs) const {
+  PairArgs<F> a{};
+  a.in = reinterpret_cast<const c2<F>*>(d_sticks.p);
+  a.out = reinterpret_cast<c2<F>*>(pair.split > 1 ? d_sticks2.p : d_sticks.p);
+  a.lines = d_lines.p;
+  a.roots = d_roots.p;
+  if constexpr (std::is_same_v<F, float>) a.potential = d_potential32.p;
+  else a.potential = d_potential.p;
+  a.inv_volume = 1.0 / sys->volume;
+  a.n0 = plan.n0;
+  a.Spad = plan.Spad;
+  a.Z = plan.Z;
+  a.zs = plan.zs;
+  a.pairs = pairs;
+  return a;
+}
+
+template <typename F>
 void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
   const StickPlan& p = plan;
   const int pairs = slots(m);
@@ -907,15 +994,22 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
   const F* pot;
   if constexpr (std::is_same_v<F, float>) pot = d_potential32.p;
   else pot = d_potential.p;
+  // k-point ops keep the radix passes of the fused one-workgroup kernel, whose
+  // bits the stick/plane path gives.
+  const bool paired = pair.on && !kb;
   if (profiling) BD_HIP(hipEventRecord(ev[0], stream));
   if (kb)
     hipLaunchKernelGGL(k_kstick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks);
+                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
   else
     hipLaunchKernelGGL(k_stick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks);
+                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
   if (profiling) BD_HIP(hipEventRecord(ev[1], stream));
-  if (p.zb > 0) {
+  if (paired) {
+    const PairArgs<F> a = pair_args<F>(pairs);
+    pair_launch<F>(stream, pair, 0, a, 1);
+    sticks = a.out;
+  } else if (p.zb > 0) {
     if (plane_threads == 512) split_pass<0, F, 512>(pairs, pot, nullptr, nullptr);
     else split_pass<0, F, 256>(pairs, pot, nullptr, nullptr);
   } else if (plane_threads == 512) {
@@ -930,11 +1024,11 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
   if (profiling) BD_HIP(hipEventRecord(ev[2], stream));
   if (kb)
     hipLaunchKernelGGL(k_kstick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, y, ldy, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks,
+                       ldx, y, ldy, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks,
                        d_kinetic.p, 1.0 / double(N));
   else
     hipLaunchKernelGGL(k_stick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, y, ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx,
+                       ldx, y, ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx,
                        sticks, d_kinetic.p, 1.0 / double(N), 0);
   if (profiling) BD_HIP(hipEventRecord(ev[3], stream));
 }
@@ -947,10 +1041,10 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
   if (kb)
     hipLaunchKernelGGL(k_kstick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks);
+                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
   else
     hipLaunchKernelGGL(k_stick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks);
+                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
   const int groups = std::min(pairs, kDensityGroups);
   // Warm start: keep the pairs' real-space fields (Gamma, fused plane pass).
   c2<F>* keep = kept_on ? reinterpret_cast<c2<F>*>(d_kept.p) : nullptr;
@@ -958,7 +1052,13 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
   kept_x = x;
   kept_ldx = ldx;
   kept_m = m;
-  if (p.zb > 0) {
+  if (pair.on) {
+    PairArgs<F> a = pair_args<F>(pairs);
+    a.kept_out = keep;
+    a.weights = w;
+    a.rho = d_rho_part.p;
+    pair_launch<F>(stream, pair, 1, a, groups);
+  } else if (p.zb > 0) {
     if (plane_threads == 512) split_pass<1, F, 512>(pairs, nullptr, w, d_rho_part.p);
     else split_pass<1, F, 256>(pairs, nullptr, w, d_rho_part.p);
   } else if (plane_threads == 512)
@@ -1000,14 +1100,20 @@ void GammaOp::kept_apply(const double* x, int64_t ldx, int m, const double* dv, 
     dvf = dv;
   }
   const c2<F>* kept = reinterpret_cast<const c2<F>*>(d_kept.p);
-  if (plane_threads == 512)
+  if (pair.on) {
+    PairArgs<F> a = pair_args<F>(pairs);
+    a.potential = dvf;
+    a.kept_in = kept;
+    pair_launch<F>(stream, pair, 2, a, 1);
+    sticks = a.out;
+  } else if (plane_threads == 512)
     hipLaunchKernelGGL((k_plane_kept<F, 512>), dim3(pairs, p.n0), dim3(512), plane_lds(p, e), stream, sticks, p.n0,
                        p.n1, p.n2, p.Spad, p.Z, p.chunk, d_stick_yz.p, d_zc.p, d_roots.p, p.ry, p.rz, dvf, kept);
   else
     hipLaunchKernelGGL((k_plane_kept<F, 256>), dim3(pairs, p.n0), dim3(256), plane_lds(p, e), stream, sticks, p.n0,
                        p.n1, p.n2, p.Spad, p.Z, p.chunk, d_stick_yz.p, d_zc.p, d_roots.p, p.ry, p.rz, dvf, kept);
   hipLaunchKernelGGL(k_stick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x, ldx, y,
-                     ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_roots.p, p.rx, sticks, d_kinetic.p,
+                     ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
                      1.0 / double(N), 1);
   if constexpr (std::is_same_v<F, float>) refresh_potential32();  // the float copy is V(r) again
 }

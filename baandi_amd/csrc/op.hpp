@@ -8,6 +8,7 @@
 
 #include "fft_device.hpp"
 #include "gemm.hpp"
+#include "plane.hpp"
 #include "system.hpp"
 
 namespace bd {
@@ -50,7 +51,13 @@ struct StickPlan {
   std::vector<int> tile_off;       // ntiles+1 offsets into entries
   std::vector<int4> entries;       // Gamma: (rep, plus slot*n0+x, minus slot*n0+x, 0)
                                    // k: (basis index, slot*n0+x, -1, 0)
-  std::vector<int2> stick_yz;      // per padded stick: (i1, zc), (-1,-1) pad
+  std::vector<int2> stick_yz;      // per stick buffer position: (i1, zc), (-1,-1) pad
+  std::vector<int> stick_dst;      // tile * T + slot -> stick buffer position
+  // The z lines of the sticks in cyclic order from z = zs, the buffer holding
+  // them one after the other; empty when a line (or the set of lines) is not
+  // one cyclic run, which the paired plane pass needs.
+  int zs = 0;
+  std::vector<PlaneLine> lines;
   std::vector<int> z_of_zc;        // Z
   std::vector<int> fpos;           // k only: stick * n0 + x per basis coefficient
 };
@@ -111,6 +118,10 @@ struct GammaOp {
   DevBuf<int> d_tile_off, d_zc;
   DevBuf<int4> d_entries;
   DevBuf<int2> d_stick_yz;
+  DevBuf<int> d_stick_dst;
+  DevBuf<PlaneLine> d_lines;
+  PairShape pair;  // the paired plane pass (plane.hpp), where it applies
+  DevBuf<c2<double>> d_sticks2;  // its output sticks where planes go by row parity
   DevBuf<c2<double>> d_roots;  // [n0 | n1 | n2]
   DevBuf<double> d_kinetic, d_potential, d_proj, d_blockd;
   DevBuf<float> d_potential32;  // mixed tier: V(r) in float
@@ -141,6 +152,8 @@ struct GammaOp {
   int kept_m = 0;
   void enable_kept(bool on);
   void apply_kept(const double* x, int64_t ldx, int m, const double* dv, double* y, int64_t ldy);
+  template <typename F>
+  PairArgs<F> pair_args(int pairs) const;
   template <typename F>
   void kept_apply(const double* x, int64_t ldx, int m, const double* dv, double* y, int64_t ldy);
   DevBuf<int> d_fpos;

@@ -231,7 +231,9 @@ bd_status bd_gamma_op_autotune(bd_gamma_op* op, int32_t m, int32_t reps, double*
 bd_status bd_gamma_op_fused_shape(bd_gamma_op* op, int32_t* inout4, int32_t set);
 /* Read (set = 0) or set the plane kernel's shape on the stick/plane path
  * (threads 256 or 512, y rows per z-FFT chunk); set accepts the shapes the
- * autotuner may pick. All shapes give the same bits. */
+ * autotuner may pick. All shapes give the same bits. Gamma ops whose plane has
+ * a kernel of the paired pass (both lengths a product of two radices) run that
+ * one whatever the shape says. */
 bd_status bd_gamma_op_plane_shape(bd_gamma_op* op, int32_t* inout2, int32_t set);
 /* Read (set = 0) or set the plane pass: 0 = one workgroup per y-z plane
  * (only where the Z x n1 plane fits the LDS), zb > 0 = the split pass, which
@@ -239,7 +241,9 @@ bd_status bd_gamma_op_plane_shape(bd_gamma_op* op, int32_t* inout2, int32_t set)
  * rows) at a time. The op picks the split pass at create when the plane does
  * not fit (the 144^3 grid of the Si512 cell in FP64); setting it on a smaller
  * cell allocates its plane buffer. Both give the same bits. Replaces the
- * plane stage of distributed_fft.rs:956-1080, which handles any plane size. */
+ * plane stage of distributed_fft.rs:956-1080, which handles any plane size.
+ * Gamma ops on the paired pass keep the setting (an op set to the split pass
+ * keeps no fields) and run the paired kernel either way. */
 bd_status bd_gamma_op_plane_split(bd_gamma_op* op, int32_t* inout, int32_t set);
 
 /* ------------------------------------------------------------------------
