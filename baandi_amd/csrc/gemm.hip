@@ -1,302 +1,19 @@
-// FP64 tiled GEMM kernels on the matrix cores: 64 x BN output tiles (BN 64;
-// 128 is built but slower here), 256 threads (4 waves, a 32 x BN/2 quadrant each), K
-// staged through LDS 16 at a time (the next slice loaded into registers while
-// the current one is multiplied), products by v_mfma_f64_16x16x4f64 (lane l
-// holds A[l%16][l/16], B[l/16][l%16] and D[l/16 + 4v][l%16], v = 0..3;
-// pinned by the probe below).
+// FP64 GEMMs: the choice of a tile and a split for each shape (the kernels are
+// in gemm_f64.hpp), and the C entry points.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "gemm_f64.hpp"
 
 namespace bd {
 
 namespace {
-constexpr int TM = 64, TK = 16;
-
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-// acc[bi][bj] += the wave's quadrant (rows wr*32 + [0, 32), cols wc*BN/2 +
-// [0, BN/2)) of As^T Bs for one TK slice.
-template <int BN>
-__device__ __forceinline__ void mfma_tile(const double (*As)[TM + 1], const double (*Bs)[BN + 1], int lane, int wr,
-                                          int wc, f64x4 (&acc)[2][BN / 32]) {
-  constexpr int NB = BN / 32;
-  const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for (int kk = 0; kk < TK; kk += 4) {
-    double a[2], b[NB];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) a[t] = As[kk + lk][wr * 32 + t * 16 + li];
-#pragma unroll
-    for (int t = 0; t < NB; ++t) b[t] = Bs[kk + lk][wc * (BN / 2) + t * 16 + li];
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-      for (int bj = 0; bj < NB; ++bj)
-        acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
-  }
-}
-
-// Slice loaders: every thread owns four consecutive elements of the A slice
-// and 4 * BN/64 of the B slice (consecutive along the contiguous index), so
-// the addresses are fixed per thread and advance by a constant per slice.
-// Interior slices load unchecked; edge slices check every element (zero
-// padding). The next slice is loaded into registers while the current one is
-// multiplied out of LDS.
-template <int BN>
-struct SliceRegs {
-  double a[4];
-  double b[4 * (BN / 64)];
-};
-
-// B slice (TK k x BN columns, k contiguous): thread t holds k = 4 (t & 3) + u
-// of column g * 64 + (t >> 2).
-template <int BN>
-__device__ __forceinline__ void load_b(SliceRegs<BN>& r, const double* __restrict__ B, int64_t ldb, int64_t k0,
-                                       int64_t kend, int64_t col0, int64_t N, bool interior) {
-  const int tid = threadIdx.x;
-  const int kb = (tid & 3) * 4;
-#pragma unroll
-  for (int g = 0; g < BN / 64; ++g) {
-    const int64_t gj = col0 + g * 64 + (tid >> 2);
-    const double* p = B + (k0 + kb) + gj * ldb;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      r.b[g * 4 + u] = interior ? p[u] : ((k0 + kb + u < kend && gj < N) ? p[u] : 0.0);
-  }
-}
-
-template <int BN>
-__device__ __forceinline__ void stash_b(const SliceRegs<BN>& r, double (*Bs)[BN + 1]) {
-  const int tid = threadIdx.x;
-  const int kb = (tid & 3) * 4;
-#pragma unroll
-  for (int g = 0; g < BN / 64; ++g)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Bs[kb + u][g * 64 + (tid >> 2)] = r.b[g * 4 + u];
-}
-
-// NN: C = alpha A B + beta C; 64 x BN output tile per workgroup.
-template <int BN>
-__global__ __launch_bounds__(256) void k_gemm_nn(int64_t M, int64_t N, int64_t K, double alpha,
-                                                 const double* __restrict__ A, int64_t lda,
-                                                 const double* __restrict__ B, int64_t ldb,
-                                                 double beta, double* __restrict__ C, int64_t ldc) {
-  constexpr int NB = BN / 32;
-  __shared__ double As[TK][TM + 1];
-  __shared__ double Bs[TK][BN + 1];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, wr = wave & 1, wc = wave >> 1;
-  const int64_t row0 = int64_t(blockIdx.x) * TM, col0 = int64_t(blockIdx.y) * BN;
-  f64x4 acc[2][NB];
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj) acc[bi][bj] = f64x4{0.0, 0.0, 0.0, 0.0};
-  // A slice (64 rows x TK k, rows contiguous): thread t holds rows
-  // 4 (t & 15) + u of k = t >> 4.
-  const int ka = tid >> 4, ia = (tid & 15) * 4;
-  const bool rows_in = row0 + TM <= M, cols_in = col0 + BN <= N;
-  SliceRegs<BN> r;
-  auto fetch = [&](int64_t k0) {
-    const bool interior = rows_in && cols_in && k0 + TK <= K;
-    const double* p = A + (row0 + ia) + (k0 + ka) * lda;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      r.a[u] = interior ? p[u] : ((row0 + ia + u < M && k0 + ka < K) ? p[u] : 0.0);
-    load_b<BN>(r, B, ldb, k0, K, col0, N, interior);
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) As[ka][ia + u] = r.a[u];
-    stash_b<BN>(r, Bs);
-  };
-  if (K > 0) {
-    fetch(0);
-    stash();
-    __syncthreads();
-  }
-  for (int64_t k0 = 0; k0 < K; k0 += TK) {
-    const bool more = k0 + TK < K;
-    if (more) fetch(k0 + TK);
-    mfma_tile<BN>(As, Bs, lane, wr, wc, acc);
-    __syncthreads();
-    if (more) {
-      stash();
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj) {
-      const int64_t gj = col0 + wc * (BN / 2) + bj * 16 + (lane & 15);
-      if (gj >= N) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int64_t gi = row0 + wr * 32 + bi * 16 + (lane >> 4) + 4 * v;
-        if (gi >= M) continue;
-        double* p = C + gi + gj * ldc;
-        *p = beta == 0.0 ? alpha * acc[bi][bj][v] : alpha * acc[bi][bj][v] + beta * *p;
-      }
-    }
-}
-
-// NN with 32 x 32 output tiles, for products whose 64-wide tiles would fill
-// only a fraction of the CUs (the subspace step's m x m and m x bands
-// products): four times the workgroups, each wave one 16 x 16 block, so the
-// K loop's MFMA chain runs on four times the SIMDs. Same operand layouts and
-// K slices as k_gemm_nn.
-constexpr int TS = 32;
-template <bool TRANS_A>
-__global__ __launch_bounds__(256) void k_gemm_s32(int64_t M, int64_t N, int64_t K, double alpha,
-                                                  const double* __restrict__ A, int64_t lda,
-                                                  const double* __restrict__ B, int64_t ldb, double beta,
-                                                  double* __restrict__ C, int64_t ldc) {
-  __shared__ double As[TK][TS + 1];
-  __shared__ double Bs[TK][TS + 1];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, wr = wave & 1, wc = wave >> 1;
-  const int li = lane & 15, lk = lane >> 4;
-  const int64_t row0 = int64_t(blockIdx.x) * TS, col0 = int64_t(blockIdx.y) * TS;
-  f64x4 acc = f64x4{0.0, 0.0, 0.0, 0.0};
-  // A slice (32 rows x TK k): thread t holds rows 2 (t & 15) + u of k = t >> 4.
-  // B slice (TK k x 32 columns): thread t holds k = 2 (t & 7) + u of column t >> 3.
-  const int ka = tid >> 4, ia = (tid & 15) * 2;
-  const int jb = tid >> 3, kb = (tid & 7) * 2;
-  double ra[2], rb[2];
-  // (TRANS_A: A is K x M, k contiguous; its slice is loaded like B's.)
-  auto fetch = [&](int64_t k0) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (TRANS_A) {
-        const int64_t gi = row0 + jb, gk = k0 + kb + u;
-        ra[u] = (gi < M && gk < K) ? A[gk + gi * lda] : 0.0;
-      } else {
-        const int64_t gi = row0 + ia + u, gk = k0 + ka;
-        ra[u] = (gi < M && gk < K) ? A[gi + gk * lda] : 0.0;
-      }
-      const int64_t gj = col0 + jb, gk2 = k0 + kb + u;
-      rb[u] = (gj < N && gk2 < K) ? B[gk2 + gj * ldb] : 0.0;
-    }
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (TRANS_A)
-        As[kb + u][jb] = ra[u];
-      else
-        As[ka][ia + u] = ra[u];
-      Bs[kb + u][jb] = rb[u];
-    }
-  };
-  if (K > 0) {
-    fetch(0);
-    stash();
-    __syncthreads();
-  }
-  for (int64_t k0 = 0; k0 < K; k0 += TK) {
-    const bool more = k0 + TK < K;
-    if (more) fetch(k0 + TK);
-#pragma unroll
-    for (int kk = 0; kk < TK; kk += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(As[kk + lk][wr * 16 + li], Bs[kk + lk][wc * 16 + li], acc, 0, 0,
-                                                 0);
-    __syncthreads();
-    if (more) {
-      stash();
-      __syncthreads();
-    }
-  }
-  const int64_t gj = col0 + wc * 16 + li;
-  if (gj >= N) return;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int64_t gi = row0 + wr * 16 + lk + 4 * v;
-    if (gi >= M) continue;
-    double* p = C + gi + gj * ldc;
-    *p = beta == 0.0 ? alpha * acc[v] : alpha * acc[v] + beta * *p;
-  }
-}
-
-// TN partial: part[s](MxN) = sum over k in chunk s of A[k,i] B[k,j].
-// Workgroups are dealt to the 8 XCDs round robin (id % 8); the logical
-// (tile, chunk) index puts the tiles of one K chunk on one XCD, one after the
-// other, where they share its L2 for the chunk's rows of A and B.
-constexpr int kXcds = 8;
-
-template <int BN>
-__global__ __launch_bounds__(256) void k_gemm_tn_part(int64_t M, int64_t N, int64_t K, int64_t chunk, int tiles_m,
-                                                      int tiles, int total, const double* __restrict__ A,
-                                                      int64_t lda, const double* __restrict__ B, int64_t ldb,
-                                                      double* __restrict__ part) {
-  constexpr int NB = BN / 32;
-  __shared__ double As[TK][TM + 1];
-  __shared__ double Bs[TK][BN + 1];
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int logical = (int(blockIdx.x) % kXcds) * per_xcd + int(blockIdx.x) / kXcds;
-  if (logical >= total) return;
-  const int tile = logical % tiles, kc = logical / tiles;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, wr = wave & 1, wc = wave >> 1;
-  const int64_t row0 = int64_t(tile % tiles_m) * TM, col0 = int64_t(tile / tiles_m) * BN;
-  const int64_t kbeg = int64_t(kc) * chunk, kend = std::min(K, kbeg + chunk);
-  f64x4 acc[2][NB];
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj) acc[bi][bj] = f64x4{0.0, 0.0, 0.0, 0.0};
-  // A slice (TK k x 64 columns i of A, k contiguous): thread t holds
-  // k = 4 (t & 3) + u of column i = t >> 2.
-  const int ia = tid >> 2, ka = (tid & 3) * 4;
-  const bool rows_in = row0 + TM <= M, cols_in = col0 + BN <= N;
-  SliceRegs<BN> r;
-  auto fetch = [&](int64_t k0) {
-    const bool interior = rows_in && cols_in && k0 + TK <= kend;
-    const double* p = A + (k0 + ka) + (row0 + ia) * lda;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      r.a[u] = interior ? p[u] : ((k0 + ka + u < kend && row0 + ia < M) ? p[u] : 0.0);
-    load_b<BN>(r, B, ldb, k0, kend, col0, N, interior);
-  };
-  auto stash = [&]() {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) As[ka + u][ia] = r.a[u];
-    stash_b<BN>(r, Bs);
-  };
-  if (kbeg < kend) {
-    fetch(kbeg);
-    stash();
-    __syncthreads();
-  }
-  for (int64_t k0 = kbeg; k0 < kend; k0 += TK) {
-    const bool more = k0 + TK < kend;
-    if (more) fetch(k0 + TK);
-    mfma_tile<BN>(As, Bs, lane, wr, wc, acc);
-    __syncthreads();
-    if (more) {
-      stash();
-      __syncthreads();
-    }
-  }
-  double* out = part + int64_t(kc) * M * N;
-#pragma unroll
-  for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj) {
-      const int64_t gj = col0 + wc * (BN / 2) + bj * 16 + (lane & 15);
-      if (gj >= N) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int64_t gi = row0 + wr * 32 + bi * 16 + (lane >> 4) + 4 * v;
-        if (gi < M) out[gi + gj * M] = acc[bi][bj][v];
-      }
-    }
-}
+using gemm64::f64x4;
 
 // Lane-layout probe: D (16x16, row-major) = A (16x4, row-major) B (4x16,
 // row-major) by one v_mfma_f64_16x16x4f64 with the operand layout above.
@@ -309,94 +26,146 @@ __global__ void k_mfma_f64_probe(const double* __restrict__ A, const double* __r
   for (int v = 0; v < 4; ++v) D[((lane >> 4) + 4 * v) * 16 + (lane & 15)] = d[v];
 }
 
-__global__ void k_gemm_tn_reduce(int64_t M, int64_t N, int splits, double alpha,
-                                 const double* __restrict__ part, double beta,
-                                 double* __restrict__ C, int64_t ldc) {
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= M * N) return;
-  const int64_t i = e % M, j = e / M;
-  // In chunk order; eight loads in flight at a time.
-  double s = 0.0;
-  int p = 0;
-  for (; p + 8 <= splits; p += 8) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = part[int64_t(p + u) * M * N + e];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u];
-  }
-  for (; p < splits; ++p) s += part[int64_t(p) * M * N + e];
-  double* c = C + i + j * ldc;
-  *c = beta == 0.0 ? alpha * s : alpha * s + beta * *c;
+// Tiles built: 64 rb x 16 nb.
+struct TileShape {
+  int rb, nb;
+};
+constexpr TileShape kTiles[] = {{1, 1}, {1, 2}, {1, 3}, {1, 5}, {1, 6}, {2, 2}, {2, 3}, {2, 4}, {2, 6}, {2, 8}};
+
+// Cycles a CU needs for `wgs` tiles of `slices` 16-k slices, dealt evenly: 4 rb
+// nb MFMAs of 64 cycles a slice on each SIMD (320 with the clock's drop under
+// FP64 load), what a slice costs besides, and the latency that a slice leaves
+// open when the CU's other workgroups are few. Within 15% of the measured
+// times from 320 x 160 x 23847 to 191711 x 1126 x 2560.
+double tile_cycles(const TileShape& t, int64_t wgs, int64_t slices) {
+  const int64_t rounds = (wgs + 255) / 256;
+  return double(slices) * (double(rounds) * (320.0 * t.rb * t.nb + 200.0) + 1000.0);
 }
 
-// Column tile width. 128-wide tiles read A half as often but were slower on
-// the Davidson shapes (fewer workgroups, longer B-tile loads): 64 is used.
-int col_tile(int64_t) { return 64; }
+int64_t tiles_of(const TileShape& t, int64_t M, int64_t N) {
+  return ((M + 64 * t.rb - 1) / (64 * t.rb)) * ((N + 16 * t.nb - 1) / (16 * t.nb));
+}
 
-int tn_splits(int64_t M, int64_t N, int64_t K) {
-  const int bn = col_tile(N);
-  const int64_t tiles = ((M + TM - 1) / TM) * ((N + bn - 1) / bn);
-  // ~512 workgroups (two per CU): more splits cost more in the partial sums
-  // than they gain in occupancy on the Davidson shapes.
-  int64_t want = std::max<int64_t>(1, 512 / std::max<int64_t>(tiles, 1));
-  int64_t maxs = std::max<int64_t>(1, K / 256);
-  return int(std::min<int64_t>({want, maxs, 256}));
+// Products with a short k range and a small C run on k_gemm_short: below this
+// the tiles fill too few CUs (NN 320 x 320 x 320: 5.6 us against 9.6 with the
+// best tile, 320 x 160 x 320: 4.1 against 9.5); 640 x 640 x 640 is level.
+bool short_product(int64_t M, int64_t N, int64_t K) {
+  return K <= 1024 && ((M + 15) / 16) * ((N + 15) / 16) <= 800;
+}
+
+template <bool TA>
+void launch_short(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
+                  const double* B, int64_t ldb, double beta, double* C, int64_t ldc) {
+  // 32-wide tiles where they still give most CUs a workgroup.
+  const int64_t rows = (M + 15) / 16;
+  if (rows * ((N + 31) / 32) >= 192)
+    hipLaunchKernelGGL((gemm64::k_gemm_short<TA, 2>), dim3(unsigned(rows), unsigned((N + 31) / 32)), dim3(256), 0, s,
+                       M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  else
+    hipLaunchKernelGGL((gemm64::k_gemm_short<TA, 1>), dim3(unsigned(rows), unsigned((N + 15) / 16)), dim3(256), 0, s,
+                       M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+}
+
+template <typename F>
+void with_tile(const TileShape& t, const F& f) {
+  switch (t.rb * 16 + t.nb) {
+    case 17: return f(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+    case 18: return f(std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+    case 19: return f(std::integral_constant<int, 1>(), std::integral_constant<int, 3>());
+    case 21: return f(std::integral_constant<int, 1>(), std::integral_constant<int, 5>());
+    case 22: return f(std::integral_constant<int, 1>(), std::integral_constant<int, 6>());
+    case 34: return f(std::integral_constant<int, 2>(), std::integral_constant<int, 2>());
+    case 35: return f(std::integral_constant<int, 2>(), std::integral_constant<int, 3>());
+    case 36: return f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+    case 38: return f(std::integral_constant<int, 2>(), std::integral_constant<int, 6>());
+    case 40: return f(std::integral_constant<int, 2>(), std::integral_constant<int, 8>());
+  }
+  fail(BD_ERR_APPLICATION, "gemm tile");
+}
+
+unsigned xcd_grid(int64_t total) {
+  if (total > (int64_t(1) << 30)) fail(BD_ERR_INVALID_PARAMETER, "gemm shape too large");
+  return unsigned((total + gemm64::kXcds - 1) / gemm64::kXcds * gemm64::kXcds);
+}
+
+// Most K chunks a split product may take: 64 k at least in each and partial
+// sums of at most 16 MB, or eight copies of C where that is more (four slices
+// of k in a short range: the factor's products count on K / 256 there).
+int64_t max_splits(int64_t M, int64_t N, int64_t K) {
+  const int64_t few = std::max<int64_t>(1, std::min<int64_t>(K / 256, 8));
+  if (K < 1024) return few;
+  return std::min<int64_t>(K / 64, std::max(few, (int64_t(1) << 21) / (M * N)));
+}
+
+struct TnPlan {
+  TileShape tile;
+  int64_t chunk;
+  int splits;
+};
+
+// The tile and split with the fewest cycles: the tiles' own, and the partial
+// sums written and read (in part in cache) at about 2,300 bytes a cycle.
+TnPlan tn_plan(int64_t M, int64_t N, int64_t K) {
+  TnPlan best{kTiles[0], K, 1};
+  double least = -1.0;
+  const int64_t most = max_splits(M, N, K);
+  for (const TileShape& t : kTiles) {
+    const int64_t tiles = tiles_of(t, M, N);
+    for (int64_t fill = 1; fill <= 8; ++fill) {
+      const int64_t want = std::max<int64_t>(1, std::min(most, fill * 256 / tiles));
+      int64_t chunk = (K + want - 1) / want;
+      chunk = (chunk + gemm64::TK - 1) / gemm64::TK * gemm64::TK;
+      const int64_t used = std::max<int64_t>(1, (K + chunk - 1) / std::max<int64_t>(chunk, 1));
+      const double cost = tile_cycles(t, tiles * used, chunk / gemm64::TK) + double(used * M * N) * (16.0 / 2300.0);
+      if (least < 0.0 || cost < least) {
+        least = cost;
+        best = {t, chunk, int(used)};
+      }
+    }
+  }
+  return best;
 }
 }  // namespace
 
 void gemm_nn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
              int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc) {
   if (M <= 0 || N <= 0) return;
-  const int bn = col_tile(N);
-  dim3 grid(unsigned((M + TM - 1) / TM), unsigned((N + bn - 1) / bn));
-  if (int64_t(grid.x) * grid.y < 128 && K >= TK) {  // under half the CUs busy: quarter-size tiles
-    dim3 g32(unsigned((M + TS - 1) / TS), unsigned((N + TS - 1) / TS));
-    hipLaunchKernelGGL(k_gemm_s32<false>, g32, dim3(256), 0, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-  } else if (bn == 128)
-    hipLaunchKernelGGL(k_gemm_nn<128>, grid, dim3(256), 0, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-  else
-    hipLaunchKernelGGL(k_gemm_nn<64>, grid, dim3(256), 0, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  if (short_product(M, N, K)) return launch_short<false>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  const int64_t slices = (K + gemm64::TK - 1) / gemm64::TK;
+  const TileShape* best = &kTiles[0];
+  for (const TileShape& t : kTiles)
+    if (tile_cycles(t, tiles_of(t, M, N), slices) < tile_cycles(*best, tiles_of(*best, M, N), slices)) best = &t;
+  with_tile(*best, [&](auto rb, auto nb) {
+    constexpr int RB = decltype(rb)::value, NB = decltype(nb)::value;
+    const int64_t tiles_n = (N + 16 * NB - 1) / (16 * NB), total = tiles_of({RB, NB}, M, N);
+    hipLaunchKernelGGL((gemm64::k_gemm_nn<RB, NB>), dim3(xcd_grid(total)), dim3(256), 0, s, M, N, K, int(tiles_n),
+                       int(total), alpha, A, lda, B, ldb, beta, C, ldc);
+  });
 }
 
-// Covers the partial sums of every product M' x N' with M' <= M, N' <= N at
-// this K, so one buffer serves every call up to its sizing shape:
-// tn_splits is not monotone (fewer tiles take more splits). A split count
-// above one is at most 512 / tiles with tiles >= M'N' / (TM * 64), and at
-// most min(K / 256, 256).
+// Monotone in M and N at a fixed K, and never below max_splits M N, so one
+// buffer serves every call up to its sizing shape.
 int64_t gemm_tn_work(int64_t M, int64_t N, int64_t K) {
-  const int64_t smax = std::min<int64_t>(std::max<int64_t>(1, K / 256), 256);
-  return std::max(M * N, std::min(int64_t(512) * TM * col_tile(N), smax * M * N));
+  const int64_t few = std::max<int64_t>(1, std::min<int64_t>(K / 256, 8));
+  if (K < 1024) return few * M * N;
+  return std::min(K / 64 * M * N, std::max(few * M * N, int64_t(1) << 21));
 }
 
 void gemm_tn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
              int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc,
              double* work) {
   if (M <= 0 || N <= 0) return;
-  const int splits = tn_splits(M, N, K);
-  int64_t chunk = (K + splits - 1) / splits;
-  chunk = ((chunk + TK - 1) / TK) * TK;
-  const int used = int((K + chunk - 1) / std::max<int64_t>(chunk, 1));
-  const int bn = col_tile(N);
-  const int tiles_m = int((M + TM - 1) / TM), tiles = tiles_m * int((N + bn - 1) / bn);
-  if (used <= 1 && tiles < 128 && K >= TK) {
-    // one K chunk and under half the CUs busy: quarter-size tiles, C written
-    // directly (no partial sums)
-    dim3 g32(unsigned((M + TS - 1) / TS), unsigned((N + TS - 1) / TS));
-    hipLaunchKernelGGL(k_gemm_s32<true>, g32, dim3(256), 0, s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-    return;
-  }
-  const int wgs = tiles * std::max(used, 1);
-  const dim3 grid(unsigned((wgs + kXcds - 1) / kXcds * kXcds));
-  if (bn == 128)
-    hipLaunchKernelGGL(k_gemm_tn_part<128>, grid, dim3(256), 0, s, M, N, K, chunk, tiles_m, tiles, wgs, A, lda, B,
-                       ldb, work);
-  else
-    hipLaunchKernelGGL(k_gemm_tn_part<64>, grid, dim3(256), 0, s, M, N, K, chunk, tiles_m, tiles, wgs, A, lda, B,
-                       ldb, work);
-  const int64_t total = M * N;
-  hipLaunchKernelGGL(k_gemm_tn_reduce, dim3(unsigned((total + 255) / 256)), dim3(256), 0, s, M, N,
-                     std::max(used, 1), alpha, work, beta, C, ldc);
+  if (short_product(M, N, K)) return launch_short<true>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  const TnPlan p = tn_plan(M, N, K);
+  with_tile(p.tile, [&](auto rb, auto nb) {
+    constexpr int RB = decltype(rb)::value, NB = decltype(nb)::value;
+    const int64_t tiles_m = (M + 64 * RB - 1) / (64 * RB), tiles = tiles_of({RB, NB}, M, N);
+    const int64_t total = tiles * p.splits;
+    hipLaunchKernelGGL((gemm64::k_gemm_tn<RB, NB>), dim3(xcd_grid(total)), dim3(256), 0, s, M, N, K, p.chunk,
+                       int(tiles_m), int(tiles), int(total), A, lda, B, ldb, work);
+  });
+  hipLaunchKernelGGL(gemm64::k_gemm_reduce, dim3(unsigned((M * N + 63) / 64)), dim3(256), 0, s, M, N, p.splits, alpha,
+                     work, beta, C, ldc);
 }
 
 }  // namespace bd
