@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libbaandi_amd.so")
 ARCH = "gfx950"
 
-SOURCES = ["errors.cpp", "setup.cpp", "gemm.hip", "gemm_bf16x3.hip", "op.hip", "plane.hip", "plane_apply_f64.hip",
+SOURCES = ["errors.cpp", "setup.cpp", "gemm.hip", "gemm_bf16x3.hip", "op.hip", "stick.hip", "plane.hip", "plane_apply_f64.hip",
            "plane_apply_f32.hip", "plane_density_f64.hip", "plane_density_f32.hip", "plane_kept_f64.hip",
            "plane_kept_f32.hip", "kbatch.hip", "eigen.hip", "subspace.hip",
            "mlp.hip", "davidson.hip", "kdavidson.hip", "field.hip", "setup_dev.hip"]

@@ -61,6 +61,7 @@ __device__ __forceinline__ void stage_roots(c2<T>* dst, const c2<double>* src, i
   for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = {T(src[i].x), T(src[i].y)};
 }
 
+// The x pass for lengths without a paired kernel (stick.hip).
 // Pack ORC column pair t into its sticks and inverse-transform along x. The
 // stick buffer and the transform use F (double, or float in the mixed tier);
 // the ORC columns are always double.
@@ -597,12 +598,18 @@ StickPlan build_stick_plan(const System& s) {
   p.T = 32;
   while (p.T > 1 && !fft_fits(p.T, p.rx)) p.T /= 2;
   if (!fft_fits(p.T, p.rx)) fail(BD_ERR_INVALID_PARAMETER, "x FFT does not fit a workgroup");
+  // The paired x pass where it is built for the length (it reads rows in twos).
+  if (s.nrep > 1) p.xshape = stick_shape(p.n0);
+  if (p.xshape.on) p.T = p.xshape.tile;
   p.chunk = 16;
   while (p.chunk > 1 && !fft_fits(p.chunk, p.rz)) p.chunk /= 2;
   p.chunk = std::min(p.chunk, p.n1);
   // Mirror units (stick + its inversion partner) packed whole into tiles, so
   // +G and -G of every representative share a tile.
+  // (the mirrors after the sticks they belong to, so that a wavefront's slots
+  // are neighbours in the stick buffer).
   std::vector<int> tile_of(p.S, -1), slot_of(p.S, -1);
+  std::vector<std::vector<std::pair<int, int>>> units(1);
   int tile = 0, used = 0;
   for (int i = 0; i < p.S; ++i) {
     if (tile_of[i] >= 0) continue;
@@ -616,13 +623,17 @@ StickPlan build_stick_plan(const System& s) {
     if (used + need > p.T) {
       ++tile;
       used = 0;
+      units.emplace_back();
     }
-    tile_of[i] = tile;
-    slot_of[i] = used++;
-    if (j != i) {
-      tile_of[j] = tile;
-      slot_of[j] = used++;
-    }
+    tile_of[i] = tile_of[j] = tile;
+    units[tile].push_back({i, j});
+    used += need;
+  }
+  for (const auto& in_tile : units) {
+    int slot = 0;
+    for (const auto& u : in_tile) slot_of[u.first] = slot++;
+    for (const auto& u : in_tile)
+      if (u.second != u.first) slot_of[u.second] = slot++;
   }
   p.ntiles = tile + 1;
   p.Spad = p.ntiles * p.T;
@@ -637,6 +648,14 @@ StickPlan build_stick_plan(const System& s) {
     if (d < 0) d = pads++;
   // Representative entries grouped by tile.
   std::vector<std::vector<int4>> per(p.ntiles);
+  const StickShape& sh = p.xshape;
+  const int row = sh.on ? sh.row : p.n0;
+  if (sh.on) p.rep_at.assign(size_t(p.Spad / sh.per) * sh.a * 64, 0);
+  auto place = [&](int stick, int xi, int value) {
+    if (!sh.on) return;
+    const int at = tile_of[stick] * p.T + slot_of[stick], wave = at / sh.per, line = at % sh.per;
+    p.rep_at[(size_t(wave) * sh.a + xi / sh.b) * 64 + line * sh.b + xi % sh.b] = value;
+  };
   for (int64_t r = 0; r < s.nrep; ++r) {
     int a0, b0, c0, a1, b1, c1;
     split(s.plus_flat[r], a0, b0, c0);
@@ -644,7 +663,9 @@ StickPlan build_stick_plan(const System& s) {
     int sp = index[{c0, b0}], sm = index[{c1, b1}];
     if (tile_of[sp] != tile_of[sm]) fail(BD_ERR_APPLICATION, "mirror pair split across tiles");
     per[tile_of[sp]].push_back(
-        make_int4(int(r), slot_of[sp] * p.n0 + a0, slot_of[sm] * p.n0 + a1, 0));
+        make_int4(int(r), slot_of[sp] * row + a0, slot_of[sm] * row + a1, 0));
+    if (r > 0) place(sm, a1, -int(r + 1));
+    place(sp, a0, int(r + 1));
   }
   p.tile_off.assign(1, 0);
   for (auto& v : per) {
@@ -858,6 +879,10 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   d_stick_yz.upload(plan.stick_yz.data(), plan.stick_yz.size(), stream);
   d_stick_dst.alloc(plan.stick_dst.size());
   d_stick_dst.upload(plan.stick_dst.data(), plan.stick_dst.size(), stream);
+  if (plan.xshape.on) {
+    d_rep_at.alloc(plan.rep_at.size());
+    d_rep_at.upload(plan.rep_at.data(), plan.rep_at.size(), stream);
+  }
   if (!plan.lines.empty()) pair = pair_shape(plan.n1, plan.n2, plan.Z, elem);
   if (pair.on) {
     d_lines.alloc(plan.lines.size());
@@ -986,6 +1011,67 @@ PairArgs<F> GammaOp::pair_args(int pairs) const {
 }
 
 template <typename F>
+StickArgs<F> GammaOp::stick_args(const double* x, int64_t ldx, int m, c2<F>* sticks) const {
+  StickArgs<F> a{};
+  a.x = x;
+  a.ldx = ldx;
+  a.m = m;
+  a.n0 = plan.n0;
+  a.Spad = plan.Spad;
+  a.tiles = plan.ntiles;
+  a.pairs = slots(m);
+  a.rep_at = d_rep_at.p;
+  a.tile_off = d_tile_off.p;
+  a.entries = d_entries.p;
+  a.dst = d_stick_dst.p;
+  a.roots = d_roots.p;
+  a.kinetic = d_kinetic.p;
+  a.inv_n = 1.0 / double(N);
+  a.sticks = sticks;
+  return a;
+}
+
+// X -> x-transformed sticks of every FFT slot.
+template <typename F>
+void GammaOp::columns_to_sticks(const double* x, int64_t ldx, int m) {
+  const StickPlan& p = plan;
+  const size_t e = sizeof(c2<F>);
+  const dim3 tiles(p.ntiles, slots(m));
+  c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
+  if (kb)
+    hipLaunchKernelGGL(k_kstick_inverse<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, p.n0, p.T, p.Spad,
+                       d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
+  else if (p.xshape.on)
+    stick_inverse<F>(stream, p.xshape, stick_args<F>(x, ldx, m, sticks));
+  else
+    hipLaunchKernelGGL(k_stick_inverse<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, m, p.n0, p.T,
+                       p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
+}
+
+// Sticks -> Y = local part + T_G X, or (accumulate) Y += local part.
+template <typename F>
+void GammaOp::sticks_to_columns(const double* x, int64_t ldx, double* y, int64_t ldy, int m, c2<F>* sticks,
+                                bool accumulate) {
+  const StickPlan& p = plan;
+  const size_t e = sizeof(c2<F>);
+  const dim3 tiles(p.ntiles, slots(m));
+  if (kb) {
+    hipLaunchKernelGGL(k_kstick_forward<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, y, ldy, p.n0, p.T,
+                       p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
+                       1.0 / double(N));
+  } else if (p.xshape.on) {
+    StickArgs<F> a = stick_args<F>(x, ldx, m, sticks);
+    a.y = y;
+    a.ldy = ldy;
+    stick_forward<F>(stream, p.xshape, a, accumulate);
+  } else {
+    hipLaunchKernelGGL(k_stick_forward<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, y, ldy, m, p.n0,
+                       p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
+                       1.0 / double(N), accumulate ? 1 : 0);
+  }
+}
+
+template <typename F>
 void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
   const StickPlan& p = plan;
   const int pairs = slots(m);
@@ -998,12 +1084,7 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
   // bits the stick/plane path gives.
   const bool paired = pair.on && !kb;
   if (profiling) BD_HIP(hipEventRecord(ev[0], stream));
-  if (kb)
-    hipLaunchKernelGGL(k_kstick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
-  else
-    hipLaunchKernelGGL(k_stick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
+  columns_to_sticks<F>(x, ldx, m);
   if (profiling) BD_HIP(hipEventRecord(ev[1], stream));
   if (paired) {
     const PairArgs<F> a = pair_args<F>(pairs);
@@ -1022,14 +1103,7 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
                        nullptr, 0.0, nullptr, nullptr);
   }
   if (profiling) BD_HIP(hipEventRecord(ev[2], stream));
-  if (kb)
-    hipLaunchKernelGGL(k_kstick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, y, ldy, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks,
-                       d_kinetic.p, 1.0 / double(N));
-  else
-    hipLaunchKernelGGL(k_stick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, y, ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx,
-                       sticks, d_kinetic.p, 1.0 / double(N), 0);
+  sticks_to_columns<F>(x, ldx, y, ldy, m, sticks, false);
   if (profiling) BD_HIP(hipEventRecord(ev[3], stream));
 }
 
@@ -1039,12 +1113,7 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
   const int pairs = slots(m);
   const size_t e = sizeof(c2<F>);
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
-  if (kb)
-    hipLaunchKernelGGL(k_kstick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
-  else
-    hipLaunchKernelGGL(k_stick_inverse<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x,
-                       ldx, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
+  columns_to_sticks<F>(x, ldx, m);
   const int groups = std::min(pairs, kDensityGroups);
   // Warm start: keep the pairs' real-space fields (Gamma, fused plane pass).
   c2<F>* keep = kept_on ? reinterpret_cast<c2<F>*>(d_kept.p) : nullptr;
@@ -1112,9 +1181,7 @@ void GammaOp::kept_apply(const double* x, int64_t ldx, int m, const double* dv, 
   else
     hipLaunchKernelGGL((k_plane_kept<F, 256>), dim3(pairs, p.n0), dim3(256), plane_lds(p, e), stream, sticks, p.n0,
                        p.n1, p.n2, p.Spad, p.Z, p.chunk, d_stick_yz.p, d_zc.p, d_roots.p, p.ry, p.rz, dvf, kept);
-  hipLaunchKernelGGL(k_stick_forward<F>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x, ldx, y,
-                     ldy, m, p.n0, p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
-                     1.0 / double(N), 1);
+  sticks_to_columns<F>(x, ldx, y, ldy, m, sticks, true);
   if constexpr (std::is_same_v<F, float>) refresh_potential32();  // the float copy is V(r) again
 }
 

@@ -9,6 +9,7 @@
 #include "fft_device.hpp"
 #include "gemm.hpp"
 #include "plane.hpp"
+#include "stick.hpp"
 #include "system.hpp"
 
 namespace bd {
@@ -49,10 +50,12 @@ struct StickPlan {
   int zb = 0;   // split plane pass: z lines per y-transform batch (0: fused k_plane)
   RadixPlan rx, ry, rz;
   std::vector<int> tile_off;       // ntiles+1 offsets into entries
-  std::vector<int4> entries;       // Gamma: (rep, plus slot*n0+x, minus slot*n0+x, 0)
+  std::vector<int4> entries;       // Gamma: (rep, plus slot*row+x, minus slot*row+x, 0), row = xshape.row or n0
                                    // k: (basis index, slot*n0+x, -1, 0)
   std::vector<int2> stick_yz;      // per stick buffer position: (i1, zc), (-1,-1) pad
   std::vector<int> stick_dst;      // tile * T + slot -> stick buffer position
+  StickShape xshape;               // Gamma: the paired x pass, where it applies
+  std::vector<int> rep_at;         // with it: StickArgs::rep_at
   // The z lines of the sticks in cyclic order from z = zs, the buffer holding
   // them one after the other; empty when a line (or the set of lines) is not
   // one cyclic run, which the paired plane pass needs.
@@ -118,7 +121,7 @@ struct GammaOp {
   DevBuf<int> d_tile_off, d_zc;
   DevBuf<int4> d_entries;
   DevBuf<int2> d_stick_yz;
-  DevBuf<int> d_stick_dst;
+  DevBuf<int> d_stick_dst, d_rep_at;
   DevBuf<PlaneLine> d_lines;
   PairShape pair;  // the paired plane pass (plane.hpp), where it applies
   DevBuf<c2<double>> d_sticks2;  // its output sticks where planes go by row parity
@@ -154,6 +157,12 @@ struct GammaOp {
   void apply_kept(const double* x, int64_t ldx, int m, const double* dv, double* y, int64_t ldy);
   template <typename F>
   PairArgs<F> pair_args(int pairs) const;
+  template <typename F>
+  void columns_to_sticks(const double* x, int64_t ldx, int m);
+  template <typename F>
+  void sticks_to_columns(const double* x, int64_t ldx, double* y, int64_t ldy, int m, c2<F>* sticks, bool accumulate);
+  template <typename F>
+  StickArgs<F> stick_args(const double* x, int64_t ldx, int m, c2<F>* sticks) const;
   template <typename F>
   void kept_apply(const double* x, int64_t ldx, int m, const double* dv, double* y, int64_t ldy);
   DevBuf<int> d_fpos;
