@@ -62,10 +62,23 @@ struct Group {
   float o;       // network output of the lane's row (same in all four quads)
 };
 
+// W2 (and W2^T) rows in LDS, 4 bf16 of padding each: the 16 rows an A-operand
+// read touches then start in different banks (64-element rows all start in
+// two).
+constexpr int kRowW2 = kHidden + 4;
+constexpr int kLdsW2 = 512, kLdsW2T = kLdsW2 + kHidden * kRowW2 / 2, kLdsFloats = kLdsW2T + kHidden * kRowW2 / 2;
+
+// LDS traffic between the lanes of one wave: its LDS instructions complete in
+// order, so only the compiler has to be held back.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Network output for the lane's row from features u (sb: the blob in LDS).
 __device__ __forceinline__ void forward_group(const float* sb, float u0, float u1, float u2, float u3, Group& G) {
   const int lane = threadIdx.x & 63, q = lane >> 4, e = lane & 15;
-  const unsigned short* W2 = reinterpret_cast<const unsigned short*>(sb + kBlobW2);
+  const unsigned short* W2 = reinterpret_cast<const unsigned short*>(sb + kLdsW2);
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -84,7 +97,7 @@ __device__ __forceinline__ void forward_group(const float* sb, float u0, float u
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const bf16x4 a = *reinterpret_cast<const bf16x4*>(&W2[(16 * rb + e) * 64 + 16 * kb + 4 * q]);
+      const bf16x4 a = *reinterpret_cast<const bf16x4*>(&W2[(16 * rb + e) * kRowW2 + 16 * kb + 4 * q]);
       acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, G.hb[kb], acc, 0, 0, 0);
     }
 #pragma unroll
@@ -100,11 +113,19 @@ __device__ __forceinline__ void forward_group(const float* sb, float u0, float u
   G.o = part + sb[hb3];
 }
 
-// The first `count` floats of the blob into LDS: inference reads W1, the
-// biases, w3 and W2 (kBlobW2T floats); training also reads W2^T.
-template <int count = kBlobFloats>
+// The blob into LDS: inference reads W1, the biases, w3 and W2 (the first
+// kLdsW2T floats); training also reads W2^T.
+template <bool train>
 __device__ __forceinline__ void load_blob(float* sb, const float* blob) {
-  for (int i = threadIdx.x; i < count; i += blockDim.x) sb[i] = blob[i];
+  constexpr int half = kHidden / 2, count = train ? kBlobFloats : kBlobW2T;
+  for (int i = threadIdx.x; i < count; i += blockDim.x) {
+    int at = i;
+    if (i >= kBlobW2) {
+      const int r = (i - kBlobW2) / half;  // (W2^T's rows follow W2's)
+      at = kLdsW2 + r * (kRowW2 / 2) + (i - kBlobW2) % half;
+    }
+    sb[at] = blob[i];
+  }
   __syncthreads();
 }
 
@@ -187,9 +208,9 @@ __global__ __launch_bounds__(256) void k_correct(int64_t n, const double* __rest
                                                  const double* __restrict__ diag, double vbar,
                                                  const float* __restrict__ blob, double* __restrict__ E,
                                                  double* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) float sb[kBlobW2T];
+  __shared__ __attribute__((aligned(16))) float sb[kLdsW2T];
   __shared__ double red[2][4];
-  load_blob<kBlobW2T>(sb, blob);
+  load_blob<false>(sb, blob);
   const int j = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, e = lane & 15;
   const double th = theta_ritz[j];
   const float T = float(Tb[j]);
@@ -253,8 +274,8 @@ __global__ void k_reduce_norms(int k, int nblk, const double* __restrict__ part,
 
 __global__ __launch_bounds__(256) void k_forward_k(int64_t n, const float* __restrict__ g, float T, float ritz,
                                                    float vbar, const float* __restrict__ blob, float* __restrict__ K) {
-  __shared__ __attribute__((aligned(16))) float sb[kBlobW2T];
-  load_blob<kBlobW2T>(sb, blob);
+  __shared__ __attribute__((aligned(16))) float sb[kLdsW2T];
+  load_blob<false>(sb, blob);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, e = lane & 15;
   const float u1 = band_u1(T), u2 = (ritz - vbar) / T, u3 = vbar;
   for (int64_t base = int64_t(blockIdx.x) * 64; base < n; base += int64_t(gridDim.x) * 64) {
@@ -284,9 +305,9 @@ __device__ __forceinline__ BandIn band_in(const float* scal, int b) {
 // Per band of the batch and block: sum a t, sum a a, sum t t (a = K r).
 __global__ __launch_bounds__(256) void k_train_fwd(TrainSet ts, const int* __restrict__ batch,
                                                    const float* __restrict__ blob, double* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) float sb[kBlobFloats];
+  __shared__ __attribute__((aligned(16))) float sb[kLdsW2T];
   __shared__ double red[3][4];
-  load_blob(sb, blob);
+  load_blob<false>(sb, blob);
   const int bi = blockIdx.y, b = batch[bi];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, e = lane & 15;
   const BandIn B = band_in(ts.scal, b);
@@ -321,71 +342,132 @@ __global__ __launch_bounds__(256) void k_train_fwd(TrainSet ts, const int* __res
   }
 }
 
-// Loss and dL/da = alpha t + beta a per batch band (mean over the batch).
-__global__ void k_band_coef(int batch, int nblk, const double* __restrict__ part, double* __restrict__ coef,
-                            double* __restrict__ loss) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Loss and dL/da = alpha t + beta a per batch band (mean over the batch): a
+// wave per band, then the bands in order. (One thread over all of it spent 115
+// us on 16 bands of 64 blocks, a load's latency each.)
+__global__ __launch_bounds__(256) void k_band_coef(int batch, int nblk, const double* __restrict__ part,
+                                                   double* __restrict__ coef, double* __restrict__ loss) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ double band_loss[4];
   double total = 0.0;
-  for (int bi = 0; bi < batch; ++bi) {
-    double c = 0.0, A = 0.0, B = 0.0;
-    for (int p = 0; p < nblk; ++p) {
-      c += part[(int64_t(bi) * nblk + p) * 3];
-      A += part[(int64_t(bi) * nblk + p) * 3 + 1];
-      B += part[(int64_t(bi) * nblk + p) * 3 + 2];
+  for (int b0 = 0; b0 < batch; b0 += 4) {
+    const int bi = b0 + wave;
+    if (bi < batch) {
+      double c = 0.0, A = 0.0, B = 0.0;
+      for (int p = lane; p < nblk; p += 64) {
+        c += part[(int64_t(bi) * nblk + p) * 3];
+        A += part[(int64_t(bi) * nblk + p) * 3 + 1];
+        B += part[(int64_t(bi) * nblk + p) * 3 + 2];
+      }
+      c = wave_sum_d(c);
+      A = wave_sum_d(A);
+      B = wave_sum_d(B);
+      if (lane == 0) {
+        double L = 1.0, alpha = 0.0, beta = 0.0;
+        if (A > 0.0 && B > 0.0) {
+          L = 1.0 - c * c / (A * B);
+          alpha = -2.0 * c / (A * B) / batch;
+          beta = 2.0 * c * c / (A * A * B) / batch;
+        }
+        coef[2 * bi] = alpha;
+        coef[2 * bi + 1] = beta;
+        band_loss[wave] = L;
+      }
     }
-    double L = 1.0, alpha = 0.0, beta = 0.0;
-    if (A > 0.0 && B > 0.0) {
-      L = 1.0 - c * c / (A * B);
-      alpha = -2.0 * c / (A * B) / batch;
-      beta = 2.0 * c * c / (A * A * B) / batch;
-    }
-    coef[2 * bi] = alpha;
-    coef[2 * bi + 1] = beta;
-    total += L;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 0; w < 4 && b0 + w < batch; ++w) total += band_loss[w];
+    __syncthreads();
   }
-  loss[0] = total / batch;
+  if (threadIdx.x == 0) loss[0] = total / batch;
 }
 
-// Backward over all rows of the batch; per-wave gradient partials (kCount floats each).
-__global__ __launch_bounds__(256) void k_train_bwd(TrainSet ts, const int* __restrict__ batch, int nbatch,
+// Backward over all rows of the batch; per-workgroup gradient partials (kCount
+// floats each, the four waves added in order). A wave's groups follow one
+// another and its LDS transposes are its own: no barrier in the loop.
+// Bound by the transcendentals of the tanh (two a unit and row) and by the
+// VALU, so the chip needs every SIMD: about 512 workgroups (two waves a SIMD,
+// what the registers allow). 16 bands of 23,847 rows: 317 -> 94 us (128
+// workgroups before, with the weight rows in two banks and a barrier twice a
+// group).
+__global__ __launch_bounds__(256, 2) void k_train_bwd(TrainSet ts, const int* __restrict__ batch, int nbatch,
                                                    const float* __restrict__ blob, const double* __restrict__ coef,
                                                    float* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) float sb[kBlobFloats];
+  __shared__ __attribute__((aligned(16))) float sb[kLdsFloats];
   __shared__ __attribute__((aligned(16))) unsigned short d2T[4][64 * 16];  // per wave: delta2[unit][row]
   __shared__ __attribute__((aligned(16))) unsigned short h1T[4][64 * 16];  // per wave: bf16(h1)[unit][row]
-  load_blob(sb, blob);
+  load_blob<true>(sb, blob);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, e = lane & 15;
-  const unsigned short* W2T = reinterpret_cast<const unsigned short*>(sb + kBlobW2T);
+  const unsigned short* W2T = reinterpret_cast<const unsigned short*>(sb + kLdsW2T);
   const int64_t gpb = (ts.n + 15) / 16;  // row groups per band
-  const int64_t total = gpb * nbatch;
-  const int64_t per_iter = int64_t(gridDim.x) * 4;
-  const int64_t iters = (total + per_iter - 1) / per_iter;
+  const int64_t total = gpb * nbatch, waves = int64_t(gridDim.x) * 4;
+  const int64_t per = (total + waves - 1) / waves;  // groups of a wave, one after the other
+  const int64_t first = (int64_t(blockIdx.x) * 4 + wave) * per, last = min(first + per, total);
   f32x4 dW2[4][4];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int c = 0; c < 4; ++c) dW2[a][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float dW1[16][4], db1[16], db2[16], dw3[16], db3 = 0.0f;
+  float dW1[16], db1[16], db2[16], dw3[16], db3 = 0.0f;
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    dW1[k][0] = dW1[k][1] = dW1[k][2] = dW1[k][3] = 0.0f;
-    db1[k] = db2[k] = dw3[k] = 0.0f;
-  }
-  for (int64_t it = 0; it < iters; ++it) {
-    const int64_t gidx = (it * gridDim.x + blockIdx.x) * 4 + wave;
-    const bool valid = gidx < total;
-    const int bi = valid ? int(gidx / gpb) : 0;
-    const int64_t row = (valid ? gidx % gpb : 0) * 16 + e;
-    const bool ok = valid && row < ts.n;
-    const int b = batch[bi];
-    const BandIn B = band_in(ts.scal, b);
-    const float u0 = log1pf((ok ? ts.g[row] : 0.0f) / B.T);
+  for (int k = 0; k < 16; ++k) dW1[k] = db1[k] = db2[k] = dw3[k] = 0.0f;
+  // Features 1 to 3 are the band's, the same in all its rows: a band's sum of
+  // delta1 gives their gradients, folded in when the wave leaves the band.
+  __shared__ float folded[4][kHidden][4];  // per wave and unit: db1, dW1[1 .. 3]
+#pragma unroll
+  for (int i = 0; i < 4; ++i) folded[wave][lane][i] = 0.0f;
+  wave_sync();
+  auto sum_rows = [](float v) {  // over the 16 rows held by lanes of the same quad
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+    return v;
+  };
+  auto fold = [&](const BandIn& B) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const float v = sum_rows(db1[k]);
+      db1[k] = 0.0f;
+      if (e == 0) {
+        float* f = folded[wave][16 * (k >> 2) + 4 * q + (k & 3)];
+        f[0] += v;
+        f[1] = fmaf(v, B.u1, f[1]);
+        f[2] = fmaf(v, B.u2, f[2]);
+        f[3] = fmaf(v, B.u3, f[3]);
+      }
+    }
+  };
+  int bi = int(min(first, total - 1) / gpb);
+  int64_t group = first - bi * gpb;  // within band bi
+  int b = batch[bi];
+  BandIn B = band_in(ts.scal, b);
+  // The next group's row is loaded while this one runs through the network.
+  float g_next = 0.0f, r_next = 0.0f, t_next = 0.0f;
+  auto fetch = [&](int64_t row, int band) {
+    const int64_t at = min(row, ts.n - 1);
+    g_next = ts.g[at];
+    r_next = ts.R[int64_t(band) * ts.n + at];
+    t_next = ts.Tg[int64_t(band) * ts.n + at];
+  };
+  if (first < last) fetch(group * 16 + e, b);
+  for (int64_t done = first; done < last; ++done, ++group) {
+    if (group >= gpb) {
+      fold(B);
+      group = 0;
+      b = batch[++bi];
+      B = band_in(ts.scal, b);
+    }
+    const bool ok = group * 16 + e < ts.n;
+    const float g = g_next, r = r_next, t = t_next;
+    if (done + 1 < last) {
+      if (group + 1 < gpb) fetch((group + 1) * 16 + e, b);
+      else fetch(e, batch[bi + 1]);
+    }
+    const float u0 = log1pf((ok ? g : 0.0f) / B.T);
     Group G;
     forward_group(sb, u0, B.u1, B.u2, B.u3, G);
     float dLdo = 0.0f;
     if (ok) {
       const float K = expf(G.o);
-      const float r = ts.R[int64_t(b) * ts.n + row], t = ts.Tg[int64_t(b) * ts.n + row];
       const double a = double(K) * double(r);
       dLdo = float((coef[2 * bi] * t + coef[2 * bi + 1] * a) * double(r) * double(K));
     }
@@ -410,7 +492,7 @@ __global__ __launch_bounds__(256) void k_train_bwd(TrainSet ts, const int* __res
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
-        const bf16x4 a = *reinterpret_cast<const bf16x4*>(&W2T[(16 * rb + e) * 64 + 16 * kb + 4 * q]);
+        const bf16x4 a = *reinterpret_cast<const bf16x4*>(&W2T[(16 * rb + e) * kRowW2 + 16 * kb + 4 * q]);
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, d2b[kb], acc, 0, 0, 0);
       }
 #pragma unroll
@@ -419,14 +501,11 @@ __global__ __launch_bounds__(256) void k_train_bwd(TrainSet ts, const int* __res
         const float h1 = G.h1[k];
         const float d1 = acc[i] * (1.0f - h1 * h1);
         db1[k] += d1;
-        dW1[k][0] = fmaf(d1, u0, dW1[k][0]);
-        dW1[k][1] = fmaf(d1, B.u1, dW1[k][1]);
-        dW1[k][2] = fmaf(d1, B.u2, dW1[k][2]);
-        dW1[k][3] = fmaf(d1, B.u3, dW1[k][3]);
+        dW1[k] = fmaf(d1, u0, dW1[k]);
         h1T[wave][(16 * rb + 4 * q + i) * 16 + e] = static_cast<unsigned short>(G.hb[rb][i]);
       }
     }
-    __syncthreads();
+    wave_sync();
     // dW2[out][in] += sum_rows delta2[out][row] h1[in][row].
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
@@ -437,54 +516,80 @@ __global__ __launch_bounds__(256) void k_train_bwd(TrainSet ts, const int* __res
         dW2[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, dW2[rb][cb], 0, 0, 0);
       }
     }
-    __syncthreads();
+    wave_sync();
   }
-  float* P = part + (int64_t(blockIdx.x) * 4 + wave) * kCount;
-#pragma unroll
-  for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) P[oW2 + (16 * rb + 4 * q + i) * kHidden + 16 * cb + e] = dW2[rb][cb][i];
-  // The other gradients: sum over the 16 rows held by lanes of the same quad.
+  fold(B);
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-      dW1[k][0] += __shfl_xor(dW1[k][0], off, 64);
-      dW1[k][1] += __shfl_xor(dW1[k][1], off, 64);
-      dW1[k][2] += __shfl_xor(dW1[k][2], off, 64);
-      dW1[k][3] += __shfl_xor(dW1[k][3], off, 64);
-      db1[k] += __shfl_xor(db1[k], off, 64);
-      db2[k] += __shfl_xor(db2[k], off, 64);
-      dw3[k] += __shfl_xor(dw3[k], off, 64);
-    }
+    dW1[k] = sum_rows(dW1[k]);
+    db2[k] = sum_rows(db2[k]);
+    dw3[k] = sum_rows(dw3[k]);
   }
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) db3 += __shfl_xor(db3, off, 64);
-  if (e == 0) {
+  // The waves add their gradients one after the other, over the blob.
+  static_assert(kCount <= kLdsFloats, "gradient over the blob");
+  float* P = sb;
+  for (int w = 0; w < 4; ++w) {
+    __syncthreads();
+    if (wave != w) continue;
+    auto put = [&](int at, float v) { P[at] = w == 0 ? v : P[at] + v; };
 #pragma unroll
-    for (int b4 = 0; b4 < 4; ++b4)
+    for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = b4 * 4 + i, n = 16 * b4 + 4 * q + i;
-        P[oW1 + 4 * n] = dW1[k][0];
-        P[oW1 + 4 * n + 1] = dW1[k][1];
-        P[oW1 + 4 * n + 2] = dW1[k][2];
-        P[oW1 + 4 * n + 3] = dW1[k][3];
-        P[ob1 + n] = db1[k];
-        P[ob2 + n] = db2[k];
-        P[ow3 + n] = dw3[k];
-      }
+      for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(oW2 + (16 * rb + 4 * q + i) * kHidden + 16 * cb + e, dW2[rb][cb][i]);
+    if (e == 0) {
+#pragma unroll
+      for (int b4 = 0; b4 < 4; ++b4)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int k = b4 * 4 + i, n = 16 * b4 + 4 * q + i;
+          const float* f = folded[wave][n];
+          put(oW1 + 4 * n, dW1[k]);
+          put(oW1 + 4 * n + 1, f[1]);
+          put(oW1 + 4 * n + 2, f[2]);
+          put(oW1 + 4 * n + 3, f[3]);
+          put(ob1 + n, f[0]);
+          put(ob2 + n, db2[k]);
+          put(ow3 + n, dw3[k]);
+        }
+    }
+    if (lane == 0) put(ob3, db3);
   }
-  if (lane == 0) P[ob3] = db3;
+  __syncthreads();
+  for (int i = threadIdx.x; i < kCount; i += 256) part[int64_t(blockIdx.x) * kCount + i] = P[i];
 }
 
-__global__ void k_grad_reduce(int waves, const float* __restrict__ part, float* __restrict__ grad) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= kCount) return;
+// Sum of the workgroups' partials in a fixed order: 16 segments of them side
+// by side (a load's latency a partial bound the one-thread sums: 127 us for
+// 512 partials), then the segments in order.
+constexpr int kReduceSeg = 16;
+__global__ __launch_bounds__(64 * kReduceSeg) void k_grad_reduce(int parts, const float* __restrict__ part,
+                                                                 float* __restrict__ grad) {
+  __shared__ double sum[kReduceSeg][64];
+  const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;
+  const int per = (parts + kReduceSeg - 1) / kReduceSeg, end = min(parts, (seg + 1) * per);
   double s = 0.0;
-  for (int w = 0; w < waves; ++w) s += part[int64_t(w) * kCount + p];
+  if (p < kCount) {
+    int w = seg * per;
+    for (; w + 8 <= end; w += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part[int64_t(w + u) * kCount + p];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; w < end; ++w) s += part[int64_t(w) * kCount + p];
+  }
+  sum[seg][lane] = s;
+  __syncthreads();
+  if (seg != 0 || p >= kCount) return;
+  s = 0.0;
+#pragma unroll
+  for (int g = 0; g < kReduceSeg; ++g) s += sum[g][lane];
   grad[p] = float(s);
 }
 
@@ -502,7 +607,13 @@ __global__ void k_adam(float* __restrict__ th, const float* __restrict__ g, floa
 
 constexpr int kCorrectBlocks = 128;
 constexpr int kTrainFwdBlocks = 64;
-constexpr int kTrainBwdBlocks = 128;
+constexpr int kTrainBwdBlocks = 512;
+
+// Workgroups of the backward kernel: at least four groups a wave, so that a
+// small batch does not spend its time on partial gradients.
+int bwd_blocks(int64_t n, int batch) {
+  return int(std::max<int64_t>(1, std::min<int64_t>(kTrainBwdBlocks, (n + 15) / 16 * batch / 16)));
+}
 }  // namespace
 
 void quantize(hipStream_t s, const float* theta, float* blob) {
@@ -531,10 +642,9 @@ void correct(hipStream_t s, int64_t n, int k, const double* X, const double* HX,
 }
 
 int64_t train_work(int64_t n, int batch) {
-  (void)n;
   // fwd partials, coefficients, loss, then float gradient partials (as doubles).
   const int64_t fwd = 3 * int64_t(batch) * kTrainFwdBlocks;
-  const int64_t bwd = (int64_t(kTrainBwdBlocks) * 4 * kCount + 1) / 2;
+  const int64_t bwd = (int64_t(bwd_blocks(n, batch)) * kCount + 1) / 2;
   return fwd + 2 * int64_t(batch) + 2 + bwd + 1;  // + the loss word
 }
 
@@ -545,9 +655,10 @@ void loss_grad(hipStream_t s, const TrainSet& ts, const int* batch_dev, int batc
   double* coef = fwd + 3 * int64_t(batch) * kTrainFwdBlocks;
   float* gpart = reinterpret_cast<float*>(coef + 2 * int64_t(batch) + 2);
   hipLaunchKernelGGL(k_train_fwd, dim3(kTrainFwdBlocks, batch), dim3(256), 0, s, ts, batch_dev, blob, fwd);
-  hipLaunchKernelGGL(k_band_coef, dim3(1), dim3(64), 0, s, batch, kTrainFwdBlocks, fwd, coef, loss);
-  hipLaunchKernelGGL(k_train_bwd, dim3(kTrainBwdBlocks), dim3(256), 0, s, ts, batch_dev, batch, blob, coef, gpart);
-  hipLaunchKernelGGL(k_grad_reduce, dim3((kCount + 255) / 256), dim3(256), 0, s, kTrainBwdBlocks * 4, gpart, grad);
+  hipLaunchKernelGGL(k_band_coef, dim3(1), dim3(256), 0, s, batch, kTrainFwdBlocks, fwd, coef, loss);
+  const int blocks = bwd_blocks(ts.n, batch);
+  hipLaunchKernelGGL(k_train_bwd, dim3(blocks), dim3(256), 0, s, ts, batch_dev, batch, blob, coef, gpart);
+  hipLaunchKernelGGL(k_grad_reduce, dim3((kCount + 63) / 64), dim3(64 * kReduceSeg), 0, s, blocks, gpart, grad);
 }
 
 void adam(hipStream_t s, float* theta, const float* grad, float* m, float* v, int step, float lr) {
