@@ -20,7 +20,7 @@ ARCH = "gfx950"
 
 SOURCES = ["errors.cpp", "setup.cpp", "gemm.hip", "gemm_bf16x3.hip", "op.hip", "stick.hip", "plane.hip", "plane_apply_f64.hip",
            "plane_apply_f32.hip", "plane_density_f64.hip", "plane_density_f32.hip", "plane_kept_f64.hip",
-           "plane_kept_f32.hip", "kbatch.hip", "eigen.hip", "subspace.hip",
+           "plane_kept_f32.hip", "kbatch.hip", "kpair.hip", "eigen.hip", "subspace.hip",
            "mlp.hip", "davidson.hip", "kdavidson.hip", "field.hip", "setup_dev.hip"]
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-result",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -1469,6 +1469,8 @@ struct KBlocks {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 
+  KPairShape pair;
+
   KBlocks(const std::vector<GammaOp*>& o, int nb_, int mode) : ops(o), nb(nb_) {
     const GammaOp& o0 = *ops[0];
     f = o0.fshape;
@@ -1483,6 +1485,7 @@ struct KBlocks {
       blocks.emplace_back(new BlockGraph(*op, nb, mode));
     }
     const int count = int(ops.size());
+    pair = kpair_common(std::vector<const GammaOp*>(ops.begin(), ops.end()).data(), count);
     std::vector<KWork> ws(count), wt(count);
     for (int k = 0; k < count; ++k) {
       BlockGraph& b = *blocks[k];
@@ -1531,7 +1534,9 @@ struct KBlocks {
 
   void batched_apply(const DevBuf<KWork>& w) {
     const KWork none{};
-    fused_launch(*ops[0], f, lds, w.p, none, int(ops.size()), int(ops.size()) * nb, main);
+    const int count = int(ops.size());
+    if (pair.on) kpair_launch(*ops[0], pair, w.p, none, count, count * nb, main);
+    else fused_launch(*ops[0], f, lds, w.p, none, count, count * nb, main);
   }
 
   void enqueue() {

@@ -19,16 +19,34 @@ struct c2 {
   T x, y;
 };
 
+// The transforms' arithmetic is written out with its fused multiply-adds, and
+// the compiler adds none of its own (fp contract(off)): the same line has the
+// same bits in every kernel that transforms it.
 template <typename T>
-__host__ __device__ __forceinline__ c2<T> cadd(c2<T> a, c2<T> b) { return {a.x + b.x, a.y + b.y}; }
-template <typename T>
-__host__ __device__ __forceinline__ c2<T> csub(c2<T> a, c2<T> b) { return {a.x - b.x, a.y - b.y}; }
-template <typename T>
-__host__ __device__ __forceinline__ c2<T> cmul(c2<T> a, c2<T> b) {
-  return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+__host__ __device__ __forceinline__ T fma_of(T a, T b, T c) {
+  if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
+  else return __builtin_fmaf(a, b, c);
 }
 template <typename T>
-__host__ __device__ __forceinline__ c2<T> cscale(c2<T> a, T s) { return {a.x * s, a.y * s}; }
+__host__ __device__ __forceinline__ c2<T> cadd(c2<T> a, c2<T> b) {
+#pragma clang fp contract(off)
+  return {a.x + b.x, a.y + b.y};
+}
+template <typename T>
+__host__ __device__ __forceinline__ c2<T> csub(c2<T> a, c2<T> b) {
+#pragma clang fp contract(off)
+  return {a.x - b.x, a.y - b.y};
+}
+template <typename T>
+__host__ __device__ __forceinline__ c2<T> cmul(c2<T> a, c2<T> b) {
+#pragma clang fp contract(off)
+  return {fma_of(a.x, b.x, -(a.y * b.y)), fma_of(a.x, b.y, a.y * b.x)};
+}
+template <typename T>
+__host__ __device__ __forceinline__ c2<T> cscale(c2<T> a, T s) {
+#pragma clang fp contract(off)
+  return {a.x * s, a.y * s};
+}
 // Multiply by -i (forward) or +i (inverse).
 template <bool INV, typename T>
 __host__ __device__ __forceinline__ c2<T> rot_i(c2<T> a) {
@@ -91,6 +109,7 @@ __host__ __device__ __forceinline__ void dft_coprime(c2<T>* v) {
 // In-register DFT of length R with root e^{-2 pi i/R} (e^{+} for INV).
 template <int R, bool INV, typename T>
 __host__ __device__ __forceinline__ void dft(c2<T>* v) {
+#pragma clang fp contract(off)
   if constexpr (R == 6) {
     dft_coprime<2, 3, INV>(v);
   } else if constexpr (R == 10) {
@@ -137,11 +156,11 @@ __host__ __device__ __forceinline__ void dft(c2<T>* v) {
   } else if constexpr (R == 3) {
     const T h = T(0.86602540378443864676372317075294);  // sin(2 pi/3)
     c2<T> s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
-    c2<T> t = {v[0].x - T(0.5) * s.x, v[0].y - T(0.5) * s.y};
-    c2<T> u = rot_i<INV>(cscale(d, h));
+    c2<T> t = {fma_of(T(-0.5), s.x, v[0].x), fma_of(T(-0.5), s.y, v[0].y)};
+    const T g = INV ? -h : h;  // t +- (-+i) h d
     v[0] = cadd(v[0], s);
-    v[1] = cadd(t, u);
-    v[2] = csub(t, u);
+    v[1] = {fma_of(g, d.y, t.x), fma_of(-g, d.x, t.y)};
+    v[2] = {fma_of(-g, d.y, t.x), fma_of(g, d.x, t.y)};
   } else if constexpr (R == 4) {
     c2<T> s02 = cadd(v[0], v[2]), d02 = csub(v[0], v[2]);
     c2<T> s13 = cadd(v[1], v[3]), d13 = rot_i<INV>(csub(v[1], v[3]));
@@ -156,10 +175,10 @@ __host__ __device__ __forceinline__ void dft(c2<T>* v) {
     const T s2 = T(0.58778525229247312916870595463907);   // sin(4 pi/5)
     c2<T> s14 = cadd(v[1], v[4]), d14 = csub(v[1], v[4]);
     c2<T> s23 = cadd(v[2], v[3]), d23 = csub(v[2], v[3]);
-    c2<T> a1 = {v[0].x + c1 * s14.x + c2_ * s23.x, v[0].y + c1 * s14.y + c2_ * s23.y};
-    c2<T> a2 = {v[0].x + c2_ * s14.x + c1 * s23.x, v[0].y + c2_ * s14.y + c1 * s23.y};
-    c2<T> b1 = rot_i<INV>(c2<T>{s1 * d14.x + s2 * d23.x, s1 * d14.y + s2 * d23.y});
-    c2<T> b2 = rot_i<INV>(c2<T>{s2 * d14.x - s1 * d23.x, s2 * d14.y - s1 * d23.y});
+    c2<T> a1 = {fma_of(c2_, s23.x, fma_of(c1, s14.x, v[0].x)), fma_of(c2_, s23.y, fma_of(c1, s14.y, v[0].y))};
+    c2<T> a2 = {fma_of(c1, s23.x, fma_of(c2_, s14.x, v[0].x)), fma_of(c1, s23.y, fma_of(c2_, s14.y, v[0].y))};
+    c2<T> b1 = rot_i<INV>(c2<T>{fma_of(s1, d14.x, s2 * d23.x), fma_of(s1, d14.y, s2 * d23.y)});
+    c2<T> b2 = rot_i<INV>(c2<T>{fma_of(s2, d14.x, -(s1 * d23.x)), fma_of(s2, d14.y, -(s1 * d23.y))});
     v[0] = cadd(v[0], cadd(s14, s23));
     v[1] = cadd(a1, b1);
     v[4] = csub(a1, b1);

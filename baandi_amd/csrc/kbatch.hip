@@ -1,4 +1,5 @@
-// k-point H·X with one workgroup per column: the whole 3D FFT of the column
+// k-point H·X with one workgroup per column, for grids without a paired kernel
+// (kpair.hip): the whole 3D FFT of the column
 // stays in LDS (its sticks, then one y-z plane at a time), so a column costs
 // one read of X, one read of V (L2-resident, shared by every column) and one
 // write of Y. One launch covers every column of every k point of a batch
@@ -241,6 +242,10 @@ KWork GammaOp::kwork(const double* x, int64_t ldx, int m, double* y, int64_t ldy
   w.blockd = d_blockd.p;
   w.np2 = int(nproj);
   w.nc = nc;
+  w.fpos_row = d_fpos_row.p;
+  w.lines = d_lines.p;
+  w.rep_at = d_rep_at.p;
+  w.zs = plan.zs;
   return w;
 }
 
@@ -260,7 +265,8 @@ void fused_launch(const GammaOp& op, const FusedShape& f, size_t lds, const KWor
 // One k point: the work entry travels as a kernel argument.
 void GammaOp::fused_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
   const KWork w = kwork(x, ldx, m, y, ldy, 0);
-  fused_launch(*this, fshape, fused_lds(fshape), nullptr, w, 1, m, stream);
+  if (kpair.on) kpair_launch(*this, kpair, nullptr, w, 1, m, stream);
+  else fused_launch(*this, fshape, fused_lds(fshape), nullptr, w, 1, m, stream);
 }
 
 }  // namespace bd
@@ -272,6 +278,7 @@ struct bd_k_batch {
   std::vector<bd_gamma_op*> ops;
   bd::DevBuf<bd::KWork> works;
   std::vector<bd::KWork> host;
+  bd::KPairShape pair;
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
   ~bd_k_batch() {
@@ -293,6 +300,9 @@ extern "C" bd_status bd_k_batch_create(bd_gamma_op* const* ops, int32_t count, b
         bd::fail(BD_ERR_INVALID_PARAMETER, "k batch ops must share the system and precision");
       b->ops.push_back(ops[i]);
     }
+    std::vector<const bd::GammaOp*> list;
+    for (bd_gamma_op* op : b->ops) list.push_back(&op->op);
+    b->pair = bd::kpair_common(list.data(), count);
     b->works.alloc(size_t(count));
     b->host.resize(size_t(count));
     BD_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
@@ -334,7 +344,8 @@ extern "C" bd_status bd_k_batch_apply_dev(bd_k_batch* b, const double* const* x,
     }
     BD_HIP(hipMemcpyAsync(b->works.p, b->host.data(), sizeof(bd::KWork) * count, hipMemcpyHostToDevice, b->stream));
     const bd::KWork none{};
-    bd::fused_launch(b->ops[0]->op, f, lds, b->works.p, none, count, total, b->stream);
+    if (b->pair.on) bd::kpair_launch(b->ops[0]->op, b->pair, b->works.p, none, count, total, b->stream);
+    else bd::fused_launch(b->ops[0]->op, f, lds, b->works.p, none, count, total, b->stream);
     // The host copy of the work table must outlive the transfer.
     BD_HIP(hipStreamSynchronize(b->stream));
   });
@@ -422,20 +433,21 @@ extern "C" bd_status bd_gamma_op_autotune(bd_gamma_op* h, int32_t m, int32_t rep
             if (o.fused_valid(f) && cands.size() < 96) cands.push_back(f);
           }
     }
+    // The paired kernel does not use the shape: only its time is taken.
+    if (o.kpair.on) cands.assign(1, o.fshape);
     if (cands.empty()) bd::fail(BD_ERR_APPLICATION, "no valid fused shape");
     // Inputs: the op's staging buffers (contents do not affect the timing).
     BD_HIP(hipMemsetAsync(o.d_x.p, 0, size_t(o.n) * m * 8, o.stream));
-    const bd::KWork w = o.kwork(o.d_x.p, o.n, m, o.d_y.p, o.n, 0);
     hipEvent_t a, z;
     BD_HIP(hipEventCreate(&a));
     BD_HIP(hipEventCreate(&z));
     double best = 1e300;
     bd::FusedShape pick = o.fshape;
     for (const auto& f : cands) {
-      const size_t lds = o.fused_lds(f);
-      bd::fused_launch(o, f, lds, nullptr, w, 1, m, o.stream);  // warm-up
+      o.fshape = f;
+      o.fused_apply(o.d_x.p, o.n, m, o.d_y.p, o.n);  // warm-up
       BD_HIP(hipEventRecord(a, o.stream));
-      for (int r = 0; r < reps; ++r) bd::fused_launch(o, f, lds, nullptr, w, 1, m, o.stream);
+      for (int r = 0; r < reps; ++r) o.fused_apply(o.d_x.p, o.n, m, o.d_y.p, o.n);
       BD_HIP(hipEventRecord(z, o.stream));
       BD_HIP(hipEventSynchronize(z));
       float ms = 0.f;

@@ -935,6 +935,7 @@ struct KDavidson {
   std::vector<KPoint> kp;
   FusedShape fshape;
   size_t flds = 0;
+  KPairShape pair;
 
   KDavidson(const std::vector<bd_gamma_op*>& ops_, int nb_, int cap_)
       : ops(ops_), count(int(ops_.size())), nb(nb_), cap(cap_) {
@@ -953,6 +954,9 @@ struct KDavidson {
       nmax = std::max(nmax, o.n);
       per += size_t(o.n) * (4 * cap + nb) + size_t(2) * (3 * cap * cap + cap * nb);
     }
+    std::vector<const GammaOp*> list;
+    for (auto* h : ops) list.push_back(&h->op);
+    pair = kpair_common(list.data(), count);
     arena.alloc(per);
     norms.alloc(size_t(count) * kKB);
     BD_HIP(hipMalloc(&stat, sizeof(KStat) * count));
@@ -1036,7 +1040,8 @@ struct KDavidson {
     if (total == 0) return;
     upload(works.p, hworks.data(), sizeof(KWork) * count);
     const KWork none{};
-    fused_launch(ops[0]->op, fshape, flds, works.p, none, count, total, main);
+    if (pair.on) kpair_launch(ops[0]->op, pair, works.p, none, count, total, main);
+    else fused_launch(ops[0]->op, fshape, flds, works.p, none, count, total, main);
   }
 
   void border(int which, int mode) {

@@ -677,7 +677,10 @@ StickPlan build_stick_plan(const System& s) {
 
 // The k sphere has no inversion partner to keep in a tile: occupied sticks
 // (keyed (z, y) as at Gamma) fill tiles of T in key order.
-StickPlan build_k_stick_plan(const System& s, const KBasis& kb) {
+// The paired passes apply where both are built for the grid, but not to a
+// column that only the radix-pass fused kernel holds in one workgroup: its
+// staged passes keep that kernel's arithmetic.
+StickPlan build_k_stick_plan(const System& s, const KBasis& kb, int nproj, size_t elem) {
   StickPlan p{};
   p.n0 = s.dims[0];
   p.n1 = s.dims[1];
@@ -717,6 +720,12 @@ StickPlan build_k_stick_plan(const System& s, const KBasis& kb) {
   p.chunk = 16;
   while (p.chunk > 1 && !fft_fits(p.chunk, p.rz)) p.chunk /= 2;
   p.chunk = std::min(p.chunk, p.n1);
+  if (!p.lines.empty() && pair_shape(p.n1, p.n2, p.Z, elem).on &&
+      (kpair_shape(p, nproj, elem).on || size_t(p.S) * p.n0 * elem > 160 * 1024))
+    p.xshape = stick_shape(p.n0);
+  const StickShape& sh = p.xshape;
+  if (sh.on) p.T = sh.tile;
+  const int row = sh.on ? sh.row : p.n0;
   p.ntiles = (p.S + p.T - 1) / p.T;
   p.Spad = p.ntiles * p.T;
   p.stick_yz.assign(p.Spad, make_int2(-1, -1));
@@ -724,11 +733,13 @@ StickPlan build_k_stick_plan(const System& s, const KBasis& kb) {
   p.stick_dst.resize(p.Spad);
   std::iota(p.stick_dst.begin(), p.stick_dst.end(), 0);
   std::vector<std::vector<int4>> per(p.ntiles);
+  if (sh.on) p.rep_at.assign(size_t(p.Spad / sh.per) * sh.a * 64, 0);
   for (int64_t g = 0; g < kb.nk; ++g) {
     int a, b, c;
     split(kb.flat[g], a, b, c);
     const int st = index[{c, b}];
-    per[st / p.T].push_back(make_int4(int(g), (st % p.T) * p.n0 + a, -1, 0));
+    per[st / p.T].push_back(make_int4(int(g), (st % p.T) * row + a, -1, 0));
+    if (sh.on) p.rep_at[(size_t(st / sh.per) * sh.a + a / sh.b) * 64 + (st % sh.per) * sh.b + a % sh.b] = int(g) + 1;
     p.fpos.push_back(st * p.n0 + a);
   }
   p.tile_off.assign(1, 0);
@@ -781,8 +792,8 @@ void GammaOp::enable_split(int zb) {
   const int pairs = slots(capacity);
   int batch = int(std::max<size_t>(1, (size_t(2) << 30) / plane));
   batch = std::min(pairs, std::max(batch, kDensityGroups));
-  // (Gamma ops on the paired pass move no plane through HBM.)
-  if ((kb || !pair.on) && d_planes.n < (size_t(batch) * plane + 15) / 16) {
+  // (Ops on the paired pass move no plane through HBM.)
+  if (!paired() && d_planes.n < (size_t(batch) * plane + 15) / 16) {
     DevBuf<c2<double>> fresh;
     fresh.alloc((size_t(batch) * plane + 15) / 16);
     std::swap(d_planes.p, fresh.p);
@@ -855,9 +866,9 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   precision = prec;
   gemm.bf16x3 = prec == BD_MIXED;
   nproj = kb ? 2 * s.nproj : s.nproj;
-  plan = kb ? build_k_stick_plan(s, *kb) : build_stick_plan(s);
-  size_t lds_max = size_t(prop.sharedMemPerBlock);
   const size_t elem = fft32() ? sizeof(c2<float>) : sizeof(c2<double>);
+  plan = kb ? build_k_stick_plan(s, *kb, int(nproj), elem) : build_stick_plan(s);
+  size_t lds_max = size_t(prop.sharedMemPerBlock);
   if (stick_lds(plan, elem) > lds_max) fail(BD_ERR_INVALID_PARAMETER, "x FFT tile exceeds the device LDS");
   if (fft32()) allow_lds<float>(plan);
   else allow_lds<double>(plan);
@@ -909,7 +920,7 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   }
   const int pairs = slots(cap);
   d_sticks.alloc(size_t(pairs) * plan.n0 * plan.Spad);
-  if (pair.on && pair.split > 1 && !kb) d_sticks2.alloc(size_t(pairs) * plan.n0 * plan.Spad);
+  if (paired() && pair.split > 1) d_sticks2.alloc(size_t(pairs) * plan.n0 * plan.Spad);
   // Planes that do not fit one workgroup go through the split pass.
   if (!fft_fits(plan.Z, plan.ry) || plane_lds(plan, elem) > lds_max) enable_split(0);
   // Host-pointer entry points stage through these (no allocation after create).
@@ -935,6 +946,14 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
     if (!fused_valid(f)) f.xplanes = 1;
     fused = fused_valid(f) && fused_lds(f) <= lds_max;
     if (fused) fshape = f;
+    if (plan.xshape.on) kpair = kpair_shape(plan, int(nproj), elem);
+    if (kpair.on) {
+      std::vector<int> rows(plan.fpos);
+      for (int& v : rows) v = v / plan.n0 * plan.xshape.row + v % plan.n0;
+      d_fpos_row.alloc(rows.size());
+      d_fpos_row.upload(rows.data(), rows.size(), stream);
+      BD_HIP(hipStreamSynchronize(stream));  // (rows ends here)
+    }
   }
   for (auto& e : ev) BD_HIP(hipEventCreate(&e));
   BD_HIP(hipStreamSynchronize(stream));
@@ -1038,11 +1057,11 @@ void GammaOp::columns_to_sticks(const double* x, int64_t ldx, int m) {
   const size_t e = sizeof(c2<F>);
   const dim3 tiles(p.ntiles, slots(m));
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
-  if (kb)
+  if (kb && !p.xshape.on)
     hipLaunchKernelGGL(k_kstick_inverse<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, p.n0, p.T, p.Spad,
                        d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
   else if (p.xshape.on)
-    stick_inverse<F>(stream, p.xshape, stick_args<F>(x, ldx, m, sticks));
+    stick_inverse<F>(stream, p.xshape, stick_args<F>(x, ldx, m, sticks), kb != nullptr);
   else
     hipLaunchKernelGGL(k_stick_inverse<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, m, p.n0, p.T,
                        p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks);
@@ -1055,7 +1074,7 @@ void GammaOp::sticks_to_columns(const double* x, int64_t ldx, double* y, int64_t
   const StickPlan& p = plan;
   const size_t e = sizeof(c2<F>);
   const dim3 tiles(p.ntiles, slots(m));
-  if (kb) {
+  if (kb && !p.xshape.on) {
     hipLaunchKernelGGL(k_kstick_forward<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, y, ldy, p.n0, p.T,
                        p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
                        1.0 / double(N));
@@ -1063,7 +1082,7 @@ void GammaOp::sticks_to_columns(const double* x, int64_t ldx, double* y, int64_t
     StickArgs<F> a = stick_args<F>(x, ldx, m, sticks);
     a.y = y;
     a.ldy = ldy;
-    stick_forward<F>(stream, p.xshape, a, accumulate);
+    stick_forward<F>(stream, p.xshape, a, kb ? StickOut::k : accumulate ? StickOut::add : StickOut::h);
   } else {
     hipLaunchKernelGGL(k_stick_forward<F>, tiles, dim3(kThreads), stick_lds(p, e), stream, x, ldx, y, ldy, m, p.n0,
                        p.T, p.Spad, d_tile_off.p, d_entries.p, d_stick_dst.p, d_roots.p, p.rx, sticks, d_kinetic.p,
@@ -1080,13 +1099,10 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
   const F* pot;
   if constexpr (std::is_same_v<F, float>) pot = d_potential32.p;
   else pot = d_potential.p;
-  // k-point ops keep the radix passes of the fused one-workgroup kernel, whose
-  // bits the stick/plane path gives.
-  const bool paired = pair.on && !kb;
   if (profiling) BD_HIP(hipEventRecord(ev[0], stream));
   columns_to_sticks<F>(x, ldx, m);
   if (profiling) BD_HIP(hipEventRecord(ev[1], stream));
-  if (paired) {
+  if (paired()) {
     const PairArgs<F> a = pair_args<F>(pairs);
     pair_launch<F>(stream, pair, 0, a, 1);
     sticks = a.out;

@@ -80,6 +80,12 @@ struct KWork {
   const double* proj2;    // 2nk x np2, column-major (ld 2nk)
   const double* blockd;   // nc x nc
   int np2, nc;
+  // The paired kernel (kpair.hip): LDS slots at its stick stride, the lines of
+  // the plane (cyclically from z = zs), the lanes' coefficients.
+  const int* fpos_row;
+  const PlaneLine* lines;
+  const int* rep_at;
+  int zs;
 };
 
 // Launch shape of the fused kernel: threads per workgroup, sticks per x-FFT
@@ -90,6 +96,13 @@ struct FusedShape {
   int xlines = 0;
   int zrows = 0;
   int xplanes = 1;  // y-z planes transformed together
+};
+
+// The paired one-workgroup-per-column k kernel on one plan (kpair.hip).
+struct KPairShape {
+  bool on = false;
+  int waves = 0;
+  size_t lds = 0;
 };
 
 struct DavidsonWork;
@@ -136,6 +149,8 @@ struct GammaOp {
   // when its LDS fits; the three-stage stick/plane path otherwise.
   bool fused = false;
   FusedShape fshape;
+  KPairShape kpair;  // runs instead of the fused kernel where it is built
+  bool paired() const { return pair.on && (!kb || plan.xshape.on); }
   int plane_threads = 256;  // k_plane workgroup size (256 or 512; tuned with plan.chunk)
   // Split plane pass (plan.zb > 0): plane buffer [pair][x][Z][n1] for
   // plane_batch FFT slots at a time.
@@ -165,7 +180,7 @@ struct GammaOp {
   StickArgs<F> stick_args(const double* x, int64_t ldx, int m, c2<F>* sticks) const;
   template <typename F>
   void kept_apply(const double* x, int64_t ldx, int m, const double* dv, double* y, int64_t ldy);
-  DevBuf<int> d_fpos;
+  DevBuf<int> d_fpos, d_fpos_row;
   KWork kwork(const double* x, int64_t ldx, int m, double* y, int64_t ldy, int first) const;
   size_t fused_lds(const FusedShape& f) const;
   bool fused_valid(const FusedShape& f) const;
@@ -195,6 +210,13 @@ struct GammaOp {
   void density(const double* x, int64_t ldx, int m, const double* w, double* rho, bool accumulate = false);
 };
 
+// The paired kernel for one op's columns, for several ops together (off where
+// one of them has none), and its launch (arguments as fused_launch).
+KPairShape kpair_shape(const StickPlan& p, int nproj, size_t elem);
+KPairShape kpair_common(const GammaOp* const* ops, int count);
+void kpair_launch(const GammaOp& op, const KPairShape& f, const KWork* works_dev, const KWork& one, int count,
+                  int total, hipStream_t s);
+
 // Launch the fused H·X for `total` work items over `count` k points (works on
 // the device); all share the grid, radix plans, roots and precision of `op`.
 // works_dev == nullptr: the single entry `one` is used (passed by value).
@@ -203,7 +225,7 @@ void fused_launch(const GammaOp& op, const FusedShape& f, size_t lds, const KWor
 bool fft_fits_threads(int nlines, const RadixPlan& rp, int threads);
 
 StickPlan build_stick_plan(const System& s);
-StickPlan build_k_stick_plan(const System& s, const KBasis& kb);
+StickPlan build_k_stick_plan(const System& s, const KBasis& kb, int nproj, size_t elem);
 RadixPlan radix_plan(int n, bool big);
 
 }  // namespace bd

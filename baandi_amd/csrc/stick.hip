@@ -1,4 +1,4 @@
-// The x pass at Gamma. A wavefront owns whole sticks: `per` lines of n0 = A B
+// The x pass. A wavefront owns whole sticks: `per` lines of n0 = A B
 // points, pass one as A-point transforms (B of them a line, one per lane),
 // pass two as B-point transforms, the values changing lanes in the line's own
 // LDS row, which only this wavefront touches. The inverse reads the ORC
@@ -70,7 +70,7 @@ __device__ __forceinline__ bool place(const StickArgs<F>& a, int& tile, int& pai
   return pair < a.pairs;
 }
 
-template <typename F, int A, int B>
+template <typename F, int A, int B, bool K>
 __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_inverse(StickArgs<F> a) {
   using S = Line<A, B>;
   __shared__ c2<F> image[S::tile * S::row];
@@ -78,8 +78,8 @@ __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_inver
   int tile, t;
   if (!place(a, tile, t)) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const bool hb = 2 * t + 1 < a.m;
-  const double* xa = a.x + int64_t(2 * t) * a.ldx;
+  const bool hb = !K && 2 * t + 1 < a.m;
+  const double* xa = a.x + int64_t(K ? t : 2 * t) * a.ldx;
   const double* xb = hb ? xa + a.ldx : xa;
   const int* ids = a.rep_at + ((int64_t(tile) * kWaves + wave) * A) * 64 + lane;
   int id[A];
@@ -88,22 +88,34 @@ __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_inver
   for (int i = threadIdx.x; i < S::n; i += 64 * kWaves) rt[i] = {F(a.roots[i].x), F(a.roots[i].y)};
   const int l1 = lane / B, j1 = lane - l1 * B;
   const int l2 = lane / A, j2 = lane - l2 * A;
-  Rows2 pa[A], pb[A];
-#pragma unroll
-  for (int r = 0; r < A; ++r) {
-    const int i = abs(id[r]) - 1;  // (none: -1)
-    const int64_t at = i > 0 ? 2 * int64_t(i) - 1 : 0;
-    pa[r] = *reinterpret_cast<const Rows2*>(xa + at);
-    pb[r] = *reinterpret_cast<const Rows2*>(xb + at);
-  }
-  // +G: a + i b; -G: conj(a) + i conj(b). Selects by factors, so that the
-  // loads above stay together.
   c2<F> v[A];
+  if (K) {
+    double2 c[A];
 #pragma unroll
-  for (int r = 0; r < A; ++r) {
-    const double one = id[r] == 1 ? 1.0 : 0.0;  // G = 0: row 0 alone, unscaled
-    const double s = abs(id[r]) > 1 ? kInvSqrt2 : 0.0, sign = id[r] > 0 ? s : -s, both = hb ? 1.0 : 0.0;
-    v[r] = {F((s + one) * pa[r].re - both * sign * pb[r].im), F(both * (s + one) * pb[r].re + sign * pa[r].im)};
+    for (int r = 0; r < A; ++r)
+      c[r] = *reinterpret_cast<const double2*>(xa + 2 * int64_t(id[r] > 0 ? id[r] - 1 : 0));
+#pragma unroll
+    for (int r = 0; r < A; ++r) {
+      const double s = id[r] > 0 ? 1.0 : 0.0;
+      v[r] = {F(s * c[r].x), F(s * c[r].y)};
+    }
+  } else {
+    Rows2 pa[A], pb[A];
+#pragma unroll
+    for (int r = 0; r < A; ++r) {
+      const int i = abs(id[r]) - 1;  // (none: -1)
+      const int64_t at = i > 0 ? 2 * int64_t(i) - 1 : 0;
+      pa[r] = *reinterpret_cast<const Rows2*>(xa + at);
+      pb[r] = *reinterpret_cast<const Rows2*>(xb + at);
+    }
+    // +G: a + i b; -G: conj(a) + i conj(b). Selects by factors, so that the
+    // loads above stay together.
+#pragma unroll
+    for (int r = 0; r < A; ++r) {
+      const double one = id[r] == 1 ? 1.0 : 0.0;  // G = 0: row 0 alone, unscaled
+      const double s = abs(id[r]) > 1 ? kInvSqrt2 : 0.0, sign = id[r] > 0 ? s : -s, both = hb ? 1.0 : 0.0;
+      v[r] = {F((s + one) * pa[r].re - both * sign * pb[r].im), F(both * (s + one) * pb[r].re + sign * pa[r].im)};
+    }
   }
   __syncthreads();  // the roots
   if (l1 < S::per) {
@@ -131,7 +143,7 @@ __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_inver
   }
 }
 
-template <typename F, int A, int B, bool ACC>
+template <typename F, int A, int B, StickOut OUT>
 __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_forward(StickArgs<F> a) {
   using S = Line<A, B>;
   __shared__ c2<F> image[S::tile * S::row];
@@ -175,6 +187,22 @@ __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_forwa
 #pragma unroll
       for (int r = 0; r < A; ++r) line[j1 + B * r] = v[r];
     }
+  }
+  constexpr bool ACC = OUT == StickOut::add;
+  if (OUT == StickOut::k) {
+    const double* x = a.x + int64_t(t) * a.ldx;
+    double* y = a.y + int64_t(t) * a.ldy;
+    __syncthreads();
+    for (; e < e1; e += 64 * kWaves) {
+      en = a.entries[e];
+      const int64_t at = 2 * int64_t(en.x);
+      const c2<F> h = image[en.y];
+      const double2 v = *reinterpret_cast<const double2*>(x + at);
+      const double k = a.kinetic[at];
+      *reinterpret_cast<double2*>(y + at) =
+          make_double2(double(h.x) * a.inv_n + k * v.x, double(h.y) * a.inv_n + k * v.y);
+    }
+    return;
   }
   const bool hb = 2 * t + 1 < a.m;
   const double* xa = a.x + int64_t(2 * t) * a.ldx;
@@ -228,22 +256,30 @@ __global__ __launch_bounds__(64 * kWaves) BD_WAVES(2, 4) void k_stick_pair_forwa
   X(15, 9) X(12, 12) X(15, 10) X(16, 10)
 
 template <typename F>
-struct StickKernels {
-  void (*inverse)(StickArgs<F>) = nullptr;
-  void (*forward)(StickArgs<F>) = nullptr;
-  void (*accumulate)(StickArgs<F>) = nullptr;
-};
+using StickKernel = void (*)(StickArgs<F>);
 
 template <typename F>
-StickKernels<F> kernels(int n0) {
+StickKernel<F> inverse_kernel(int n0, bool k) {
   switch (n0) {
 #define BD_CASE(A, B) \
   case A * B:         \
-    return {&k_stick_pair_inverse<F, A, B>, &k_stick_pair_forward<F, A, B, false>, &k_stick_pair_forward<F, A, B, true>};
+    return k ? &k_stick_pair_inverse<F, A, B, true> : &k_stick_pair_inverse<F, A, B, false>;
     BD_LINES(BD_CASE)
 #undef BD_CASE
   }
-  return {};
+  return nullptr;
+}
+
+template <typename F, StickOut OUT>
+StickKernel<F> forward_kernel(int n0) {
+  switch (n0) {
+#define BD_CASE(A, B) \
+  case A * B:         \
+    return &k_stick_pair_forward<F, A, B, OUT>;
+    BD_LINES(BD_CASE)
+#undef BD_CASE
+  }
+  return nullptr;
 }
 
 // Whole pairs to the XCDs where that leaves none of them more than a quarter
@@ -268,24 +304,27 @@ StickShape stick_shape(int n0) {
 }
 
 template <typename F>
-void stick_inverse(hipStream_t s, const StickShape& shape, StickArgs<F> a) {
-  const StickKernels<F> k = kernels<F>(shape.a * shape.b);
-  if (!k.inverse) fail(BD_ERR_APPLICATION, "no x-pass kernel");
+void stick_inverse(hipStream_t s, const StickShape& shape, StickArgs<F> a, bool k) {
+  const StickKernel<F> f = inverse_kernel<F>(shape.a * shape.b, k);
+  if (!f) fail(BD_ERR_APPLICATION, "no x-pass kernel");
   const unsigned blocks = grid(a);
-  hipLaunchKernelGGL(k.inverse, dim3(blocks), dim3(64 * kWaves), 0, s, a);
+  hipLaunchKernelGGL(f, dim3(blocks), dim3(64 * kWaves), 0, s, a);
 }
 
 template <typename F>
-void stick_forward(hipStream_t s, const StickShape& shape, StickArgs<F> a, bool accumulate) {
-  const StickKernels<F> k = kernels<F>(shape.a * shape.b);
-  if (!k.forward) fail(BD_ERR_APPLICATION, "no x-pass kernel");
+void stick_forward(hipStream_t s, const StickShape& shape, StickArgs<F> a, StickOut out) {
+  const int n0 = shape.a * shape.b;
+  const StickKernel<F> f = out == StickOut::h     ? forward_kernel<F, StickOut::h>(n0)
+                           : out == StickOut::add ? forward_kernel<F, StickOut::add>(n0)
+                                                  : forward_kernel<F, StickOut::k>(n0);
+  if (!f) fail(BD_ERR_APPLICATION, "no x-pass kernel");
   const unsigned blocks = grid(a);
-  hipLaunchKernelGGL(accumulate ? k.accumulate : k.forward, dim3(blocks), dim3(64 * kWaves), 0, s, a);
+  hipLaunchKernelGGL(f, dim3(blocks), dim3(64 * kWaves), 0, s, a);
 }
 
-template void stick_inverse<double>(hipStream_t, const StickShape&, StickArgs<double>);
-template void stick_inverse<float>(hipStream_t, const StickShape&, StickArgs<float>);
-template void stick_forward<double>(hipStream_t, const StickShape&, StickArgs<double>, bool);
-template void stick_forward<float>(hipStream_t, const StickShape&, StickArgs<float>, bool);
+template void stick_inverse<double>(hipStream_t, const StickShape&, StickArgs<double>, bool);
+template void stick_inverse<float>(hipStream_t, const StickShape&, StickArgs<float>, bool);
+template void stick_forward<double>(hipStream_t, const StickShape&, StickArgs<double>, StickOut);
+template void stick_forward<float>(hipStream_t, const StickShape&, StickArgs<float>, StickOut);
 
 }  // namespace bd

@@ -1,5 +1,6 @@
-// The x pass at Gamma: ORC columns <-> x-transformed sticks, each stick as two
-// in-register radix passes of one wavefront (stick.hip).
+// The x pass: columns (ORC rows at Gamma, interleaved Re and Im at k) <->
+// x-transformed sticks, each stick as two in-register radix passes of one
+// wavefront (stick.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -29,19 +30,22 @@ struct StickArgs {
   int m;              // columns
   int n0, Spad, tiles, pairs;
   int by_xcd;         // deal whole pairs to the XCDs
-  const int* rep_at;  // inverse: [tile][wave][r][lane], 0 or +-(representative + 1)
+  const int* rep_at;  // inverse: [tile][wave][r][lane], 0 or +-(representative + 1), at k coefficient + 1
   const int* tile_off;
-  const int4* entries;  // forward: (representative, +G, -G positions in the LDS image, 0)
+  const int4* entries;  // forward: (representative, +G, -G positions in the LDS image, 0); at k (coefficient, position, -1, 0)
   const int* dst;       // stick buffer position of each slot
   const c2<double>* roots;
   const double* kinetic;
   double inv_n;
   c2<F>* sticks;  // [pair][x][Spad]
 };
+// k: one complex column per FFT slot instead of a pair of real ones.
 template <typename F>
-void stick_inverse(hipStream_t s, const StickShape& shape, StickArgs<F> a);
-// accumulate: y += the local part alone; otherwise y = local part + T_G x.
+void stick_inverse(hipStream_t s, const StickShape& shape, StickArgs<F> a, bool k);
+// h: y = local part + T_G x; add: y += the local part alone; k: as h, on
+// complex columns.
+enum class StickOut { h, add, k };
 template <typename F>
-void stick_forward(hipStream_t s, const StickShape& shape, StickArgs<F> a, bool accumulate);
+void stick_forward(hipStream_t s, const StickShape& shape, StickArgs<F> a, StickOut out);
 
 }  // namespace bd
