@@ -38,7 +38,7 @@ namespace {
 constexpr int kKB = 24;    // bands per k point
 constexpr int kKCap = 48;  // complex basis columns per k point
 constexpr int kKT = 256;
-constexpr int kEigT = 256;  // k_kd_eigen workgroup (64 measured twice as slow: the rounds are work-bound)
+constexpr int kEigT = 512;  // k_kd_eigen workgroup
 constexpr double kEps = std::numeric_limits<double>::epsilon();
 constexpr double kPivotMin = kEps / 1e-12;  // PIVOT_RATIO_MIN, lean_davidson.rs:64
 constexpr double kOrthoLimit = 1e-12;       // ORTHOGONALITY_LIMIT, ref_davidson/ideal_reset.rs:7
@@ -135,6 +135,13 @@ __device__ __forceinline__ double2 zadd(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 zsub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 zscale(double s, double2 a) { return make_double2(s * a.x, s * a.y); }
 __device__ __forceinline__ double zabs2(double2 a) { return a.x * a.x + a.y * a.y; }
+
+// LDS traffic between the lanes of one wave: its LDS instructions complete in
+// order, so only the compiler has to be held back.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 // Deterministic workgroup sum (fixed tree), valid on every thread.
 __device__ double kd_sum(double v, double* red) {
@@ -332,14 +339,22 @@ __global__ __launch_bounds__(kKT) void k_kd_normalize(const KDesc* __restrict__ 
 // B[:, from:to] with B = V (which 0: S) or HV (which 1: H), written to both
 // triangles of M (exactly Hermitian, real diagonal), over the range of
 // kd_range(mode). which 2: the rank repair's projection G = V[:, :m]^H
-// V[:, m:m + kept] into E (ld m, k points in repair). A 16 x 16 tile of G per
-// workgroup, 64 rows at a time through LDS; for which 1 a non-finite H·V
-// entry sets stat.nonfinite_h.
+// V[:, m:m + kept] into E (ld m, k points in repair). For which 1 a non-finite
+// H·V entry sets stat.nonfinite_h.
+//
+// A 16 x 16 tile of G per workgroup on the matrix cores (FP64 16x16x4): lane l
+// holds row l / 16 of four complex rows of column l % 16, 16 bytes, the (re,
+// im) pair of V and of B; re = vr br + vi bi and im = vr bi - vi br are two
+// MFMAs each. The rows are split over the 4 waves, whose loads run kAhead
+// steps ahead, and their sums are added in wave order. Bound by the loads
+// (up to 50 MB of V a launch) and their latency. Al 6x6x6 map, mean of a
+// launch over 108 k points: 23 us, 49 with products a thread an entry out of
+// LDS.
 __global__ __launch_bounds__(kKT) void k_kd_border(const KDesc* __restrict__ D, KStat* __restrict__ St, int which,
                                                    int mode, int nb, int cap) {
-  constexpr int R = 64;
-  __shared__ double2 vs[16][R + 1];
-  __shared__ double2 bs[16][R + 1];
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  constexpr int kAhead = 6, kWaves = kKT / 64;
+  __shared__ double2 part[kWaves][256];
   const KDesc& d = D[blockIdx.z];
   KStat& st = St[blockIdx.z];
   int from, to, rows;
@@ -354,27 +369,44 @@ __global__ __launch_bounds__(kKT) void k_kd_border(const KDesc* __restrict__ D, 
   }
   const int i0 = blockIdx.x * 16, j0 = blockIdx.y * 16;
   if (i0 >= rows || j0 >= to - from) return;
-  const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
   const int64_t nc = d.n / 2;
-  const double2* V = reinterpret_cast<const double2*>(d.V);
-  const double2* B = reinterpret_cast<const double2*>(which == 1 ? d.HV : d.V);
-  double2 acc = make_double2(0.0, 0.0);
+  // Columns past the range repeat its last one (their sums are not stored).
+  const double2* V = reinterpret_cast<const double2*>(d.V) + min(i0 + li, rows - 1) * nc;
+  const double2* B = reinterpret_cast<const double2*>(which == 1 ? d.HV : d.V) + min(from + j0 + li, to - 1) * nc;
+  const int64_t steps = (nc + 3) / 4, span = (steps + kWaves - 1) / kWaves;
+  const int64_t s0 = min(wave * span, steps), s1 = min(s0 + span, steps);
+  f64x4 re = {0.0, 0.0, 0.0, 0.0}, im = re;
   int bad = 0;
-  for (int64_t r0 = 0; r0 < nc; r0 += R) {
-    for (int t = threadIdx.x; t < 16 * R; t += blockDim.x) {
-      const int c = t / R, rr = t % R;
-      const int64_t r = r0 + rr;
-      const int iv = i0 + c, jb = from + j0 + c;
-      vs[c][rr] = (iv < rows && r < nc) ? V[r + iv * nc] : make_double2(0.0, 0.0);
-      double2 b = (jb < to && r < nc) ? B[r + jb * nc] : make_double2(0.0, 0.0);
-      bad |= !(isfinite(b.x) && isfinite(b.y));
-      bs[c][rr] = b;
+  double2 v[kAhead], b[kAhead];
+  auto fetch = [&](double2& fv, double2& fb, int64_t s) {
+    const int64_t r = 4 * s + lg;
+    const bool in = r < nc;
+    fv = V[in ? r : nc - 1];
+    fb = B[in ? r : nc - 1];
+    if (!in) fv = fb = make_double2(0.0, 0.0);
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+    if (s0 + u < s1) fetch(v[u], b[u], s0 + u);
+  for (int64_t s = s0; s < s1; s += kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (s + u >= s1) break;
+      bad |= !(isfinite(b[u].x) && isfinite(b[u].y));
+      re = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u].x, b[u].x, re, 0, 0, 0);
+      im = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u].x, b[u].y, im, 0, 0, 0);
+      re = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u].y, b[u].y, re, 0, 0, 0);
+      im = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[u].y, b[u].x, im, 0, 0, 0);
+      if (s + u + kAhead < s1) fetch(v[u], b[u], s + u + kAhead);
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int rr = 0; rr < R; ++rr) acc = zadd(acc, zcmul(vs[ti][rr], bs[tj][rr]));
-    __syncthreads();
   }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) part[wave][(lg + 4 * u) * 16 + li] = make_double2(re[u], im[u]);
+  __syncthreads();
+  const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
+  const double2 acc = zadd(zadd(part[0][threadIdx.x], part[1][threadIdx.x]),
+                           zadd(part[2][threadIdx.x], part[3][threadIdx.x]));
   if (which == 1 && bad) st.nonfinite_h = 1;
   const int i = i0 + ti, jc = from + j0 + tj;
   if (i >= rows || jc >= to) return;
@@ -479,13 +511,24 @@ __global__ __launch_bounds__(kKT) void k_kd_factor(const KDesc* __restrict__ D, 
 // (a fixed, deterministic order; the rotations keep the eigenvectors
 // orthonormal, equal eigenvalues included), the lowest nb values ascending
 // into stat.values and C = L^-H Y. Skipped when the factor was rejected.
-__global__ __launch_bounds__(kKT) void k_kd_eigen(const KDesc* __restrict__ D, KStat* __restrict__ St, int mode,
-                                                  int nb, int cap) {
+//
+// Bound by the chain of rounds: a round is the pairs' rotations (two
+// reciprocal square roots each: with h = hypot((aqq - app) / 2, |apq|), c^2 =
+// 1/2 + |aqq - app| / 4h and s e = apq / 2hc), a barrier, and one pass that
+// takes every 2 x 2 block of pairs through both sides of the rotation in
+// registers (half the waves; the lower blocks are mirrored, so A stays exactly
+// Hermitian) and turns Q's columns (the other half). The substitutions run
+// eight lanes a column. Al 6x6x6 map, mean of a launch over 108 k points: 268
+// us; 529 with a thread a column in the substitutions, separate passes over
+// A's columns and rows, and a whole sweep to find that nothing is left.
+__global__ __launch_bounds__(kEigT) void k_kd_eigen(const KDesc* __restrict__ D, KStat* __restrict__ St, int mode,
+                                                    int nb, int cap) {
   extern __shared__ double2 esh[];
-  __shared__ double red[kKT / 64];
-  __shared__ double rot[kKCap / 2][4];
-  __shared__ int rp[kKCap / 2][2];
-  __shared__ int nrot, perm[kKCap];
+  constexpr int kPairs = kKCap / 2;
+  __shared__ double red[kEigT / 64];
+  __shared__ double rot[kPairs][3];  // c, s e (s signed)
+  __shared__ int rp[kPairs][2];
+  __shared__ int left, perm[kKCap];
   const KDesc& d = D[blockIdx.x];
   KStat& st = St[blockIdx.x];
   int m;
@@ -497,134 +540,180 @@ __global__ __launch_bounds__(kKT) void k_kd_eigen(const KDesc* __restrict__ D, K
     m = nb;
   }
   if (st.factor_bad || st.nonfinite_h || st.repair_bad) return;
+  const int tid = threadIdx.x;
   // Leading dimension m + 1 (odd): a row of a matrix (stride la) spreads over
   // the LDS banks.
   const int la = m + 1;
   double2* Ls = esh;          // m x m
   double2* A = Ls + m * la;   // m x m
   double2* W = A + m * la;    // m x m: L^-1 H, then the eigenvectors Q
-  for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
+  for (int t = tid; t < m * m; t += kEigT) {
     const int i = t % m, j = t / m;
     Ls[i + j * la] = d.L[i + int64_t(j) * cap];
     W[i + j * la] = d.H[i + int64_t(j) * cap];
   }
   __syncthreads();
-  // W = L^-1 H (forward substitution per column), then A = L^-1 W^H.
-  for (int j = threadIdx.x; j < m; j += blockDim.x)
-    for (int i = 0; i < m; ++i) {
-      double2 z = W[i + j * la];
-      for (int p = 0; p < i; ++p) z = zsub(z, zmul(Ls[i + p * la], W[p + j * la]));
-      W[i + j * la] = zscale(1.0 / Ls[i + i * la].x, z);
+  // X <- L^-1 X, eight lanes a column (a column belongs to one wave).
+  const int sub = tid & 7, col0 = tid >> 3;
+  auto forward = [&](double2* X) {
+    for (int j = col0; j < m; j += kEigT / 8) {
+      double2* x = X + j * la;
+      for (int i = 0; i < m; ++i) {
+        double2 z = make_double2(0.0, 0.0);
+        for (int p = sub; p < i; p += 8) z = zadd(z, zmul(Ls[i + p * la], x[p]));
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) {
+          z.x += __shfl_xor(z.x, off);
+          z.y += __shfl_xor(z.y, off);
+        }
+        if (sub == 0) x[i] = zscale(1.0 / Ls[i + i * la].x, zsub(x[i], z));
+        wave_order();
+      }
     }
+  };
+  // W = L^-1 H, then A = L^-1 W^H.
+  forward(W);
   __syncthreads();
-  for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
+  for (int t = tid; t < m * m; t += kEigT) {
     const int i = t % m, j = t / m;
     A[i + j * la] = zconj(W[j + i * la]);
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < m; j += blockDim.x)
-    for (int i = 0; i < m; ++i) {
-      double2 z = A[i + j * la];
-      for (int p = 0; p < i; ++p) z = zsub(z, zmul(Ls[i + p * la], A[p + j * la]));
-      A[i + j * la] = zscale(1.0 / Ls[i + i * la].x, z);
-    }
+  forward(A);
   __syncthreads();
   // Hermitise (in W), then back into A; Q = I in W.
-  for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
+  for (int t = tid; t < m * m; t += kEigT) {
     const int i = t % m, j = t / m;
     const double2 a = A[i + j * la], b = zconj(A[j + i * la]);
     W[i + j * la] = i == j ? make_double2(0.5 * (a.x + b.x), 0.0) : zscale(0.5, zadd(a, b));
   }
   __syncthreads();
   double fro = 0.0;
-  for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
+  for (int t = tid; t < m * m; t += kEigT) {
     const int i = t % m, j = t / m;
     A[i + j * la] = W[i + j * la];
     W[i + j * la] = i == j ? make_double2(1.0, 0.0) : make_double2(0.0, 0.0);
     fro += zabs2(A[i + j * la]);
   }
-  const double thr = kEps * sqrt(kd_sum(fro, red));
+  const double thr = kEps * sqrt(kd_sum(fro, red)), thr2 = thr * thr;
   const int mp = m + (m & 1);  // players; an odd m has one idle player per round
-  const int pairs = mp / 2;
+  const int pairs = mp / 2, blocks = pairs * (pairs + 1) / 2;
+  // This thread's blocks (u, v), u <= v, row by row of the triangle; at most
+  // two of the 300.
+  int bu[2], bv[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int w = tid + k * (kEigT / 2);
+    int v = 0;
+    while ((v + 1) * (v + 2) / 2 <= w) ++v;
+    bu[k] = w - v * (v + 1) / 2;
+    bv[k] = v;
+  }
+  static_assert(kPairs * (kPairs + 1) / 2 <= kEigT, "two blocks a thread");
   for (int sweep = 0; sweep < 60; ++sweep) {
-    if (threadIdx.x == 0) nrot = 0;
+    // Done when no entry is above the threshold.
+    if (tid == 0) left = 0;
     __syncthreads();
+    int any = 0;
+    for (int t = tid; t < m * m; t += kEigT) {
+      const int i = t % m, j = t / m;
+      any |= i < j && zabs2(A[i + j * la]) > thr2;
+    }
+    if (any) left = 1;
+    __syncthreads();
+    if (!left) break;
     for (int round = 0; round < mp - 1; ++round) {
-      if (threadIdx.x < pairs) {
-        const int t = threadIdx.x;
+      if (tid < pairs) {
+        const int t = tid;
         const int a = t == 0 ? mp - 1 : (t - 1 + round) % (mp - 1);
         const int b = (mp - 2 - t + round) % (mp - 1);
-        int p = min(a, b), q = max(a, b);
-        double c = 1.0, s = 0.0, er = 1.0, ei = 0.0;
+        const int p = min(a, b), q = max(a, b);
+        double c = 1.0, sx = 0.0, sy = 0.0;
         if (q < m) {
           const double2 apq = A[p + q * la];
-          const double r = sqrt(zabs2(apq));
-          if (r > thr) {
-            const double app = A[p + p * la].x, aqq = A[q + q * la].x;
-            const double ir = 1.0 / r;
-            const double th = 0.5 * (aqq - app) * ir;
-            const double tt = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-            c = 1.0 / sqrt(tt * tt + 1.0);
-            s = tt * c;
-            er = apq.x * ir;
-            ei = apq.y * ir;
-            atomicAdd(&nrot, 1);
-          } else {
-            q = -1;
+          const double r2 = zabs2(apq);
+          if (r2 > thr2) {
+            const double dd = 0.5 * (A[q + q * la].x - A[p + p * la].x);
+            const double ih = rsqrt(dd * dd + r2);
+            const double c2 = 0.5 + 0.5 * fabs(dd) * ih;
+            const double rc = rsqrt(c2);
+            c = c2 * rc;
+            const double g = (dd >= 0.0 ? 0.5 : -0.5) * ih * rc;
+            sx = g * apq.x;
+            sy = g * apq.y;
           }
-        } else {
-          q = -1;
         }
         rot[t][0] = c;
-        rot[t][1] = s;
-        rot[t][2] = er;
-        rot[t][3] = ei;
+        rot[t][1] = sx;
+        rot[t][2] = sy;
         rp[t][0] = p;
-        rp[t][1] = q;
+        rp[t][1] = q < m ? q : -1;  // (the idle player: no partner)
       }
       __syncthreads();
-      // Columns: A <- A U, Q <- Q U with U = [[c, s e], [-s conj(e), c]].
-      for (int w = threadIdx.x; w < pairs * m; w += blockDim.x) {
-        const int t = w / m, i = w % m;
-        const int p = rp[t][0], q = rp[t][1];
-        if (q < 0) continue;
-        const double c = rot[t][0], s = rot[t][1];
-        const double2 e = make_double2(rot[t][2], rot[t][3]);
-        const double2 aip = A[i + p * la], aiq = A[i + q * la];
-        A[i + p * la] = zsub(zscale(c, aip), zscale(s, zmul(zconj(e), aiq)));
-        A[i + q * la] = zadd(zscale(s, zmul(e, aip)), zscale(c, aiq));
-        const double2 qip = W[i + p * la], qiq = W[i + q * la];
-        W[i + p * la] = zsub(zscale(c, qip), zscale(s, zmul(zconj(e), qiq)));
-        W[i + q * la] = zadd(zscale(s, zmul(e, qip)), zscale(c, qiq));
-      }
-      __syncthreads();
-      // Rows: A <- U^H A; the pivot entries are set to their exact values.
-      for (int w = threadIdx.x; w < pairs * m; w += blockDim.x) {
-        const int t = w / m, j = w % m;
-        const int p = rp[t][0], q = rp[t][1];
-        if (q < 0) continue;
-        const double c = rot[t][0], s = rot[t][1];
-        const double2 e = make_double2(rot[t][2], rot[t][3]);
-        const double2 apj = A[p + j * la], aqj = A[q + j * la];
-        double2 np = zsub(zscale(c, apj), zscale(s, zmul(e, aqj)));
-        double2 nq = zadd(zscale(s, zmul(zconj(e), apj)), zscale(c, aqj));
-        if (j == p) {
-          np.y = 0.0;
-          nq = make_double2(0.0, 0.0);
-        } else if (j == q) {
-          np = make_double2(0.0, 0.0);
-          nq.y = 0.0;
+      // U = [[c, s e], [-s conj(e), c]] on each pair: A <- U^H A U, Q <- Q U.
+      if (tid < kEigT / 2) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          if (tid + k * (kEigT / 2) >= blocks) continue;
+          const int u = bu[k], v = bv[k];
+          const int p1 = rp[u][0], q1 = rp[u][1], p2 = rp[v][0], q2 = rp[v][1];
+          const double c1 = rot[u][0], c2 = rot[v][0];
+          const double2 e1 = make_double2(rot[u][1], rot[u][2]), e2 = make_double2(rot[v][1], rot[v][2]);
+          const bool id1 = e1.x == 0.0 && e1.y == 0.0, id2 = e2.x == 0.0 && e2.y == 0.0;
+          if (id1 && id2) continue;
+          const double2 zero = make_double2(0.0, 0.0);
+          const double2 pp = A[p1 + p2 * la];
+          const double2 pq = q2 >= 0 ? A[p1 + q2 * la] : zero;
+          const double2 qp = q1 >= 0 ? A[q1 + p2 * la] : zero;
+          const double2 qq = q1 >= 0 && q2 >= 0 ? A[q1 + q2 * la] : zero;
+          // Columns: (x, y) <- (c x - conj(se) y, se x + c y).
+          const double2 pp1 = zsub(zscale(c2, pp), zcmul(e2, pq)), pq1 = zadd(zmul(e2, pp), zscale(c2, pq));
+          const double2 qp1 = zsub(zscale(c2, qp), zcmul(e2, qq)), qq1 = zadd(zmul(e2, qp), zscale(c2, qq));
+          // Rows: (x, y) <- (c x - se y, conj(se) x + c y).
+          double2 npp = zsub(zscale(c1, pp1), zmul(e1, qp1)), nqp = zadd(zcmul(e1, pp1), zscale(c1, qp1));
+          double2 npq = zsub(zscale(c1, pq1), zmul(e1, qq1)), nqq = zadd(zcmul(e1, pq1), zscale(c1, qq1));
+          if (u == v) {  // the pivots' exact values
+            npp.y = nqq.y = 0.0;
+            npq = nqp = zero;
+          }
+          auto put = [&](int i, int j, double2 z) {
+            A[i + j * la] = z;
+            if (u != v) A[j + i * la] = zconj(z);
+          };
+          put(p1, p2, npp);
+          if (q2 >= 0) put(p1, q2, npq);
+          if (q1 >= 0) put(q1, p2, nqp);
+          if (q1 >= 0 && q2 >= 0) put(q1, q2, nqq);
         }
-        A[p + j * la] = np;
-        A[q + j * la] = nq;
+      } else {
+        const int w0 = tid - kEigT / 2;
+        int t = w0 / m, i = w0 - t * m;
+        const int dt = (kEigT / 2) / m, di = kEigT / 2 - dt * m;
+        for (int w = w0; w < pairs * m; w += kEigT / 2) {
+          const int p = rp[t][0], q = rp[t][1];
+          const double c = rot[t][0];
+          const double2 e = make_double2(rot[t][1], rot[t][2]);
+          if (q >= 0 && !(e.x == 0.0 && e.y == 0.0)) {
+            const double2 x = W[i + p * la], y = W[i + q * la];
+            W[i + p * la] = zsub(zscale(c, x), zcmul(e, y));
+            W[i + q * la] = zadd(zmul(e, x), zscale(c, y));
+          }
+          t += dt;
+          i += di;
+          if (i >= m) {
+            i -= m;
+            ++t;
+          }
+        }
       }
       __syncthreads();
     }
-    if (nrot == 0) break;
-    __syncthreads();
   }
-  // Ascending order (ties by index), the lowest nb.
-  for (int i = threadIdx.x; i < m; i += blockDim.x) {
+  // Ascending order (ties by index), the lowest nb. (Not a number compares
+  // with nothing: the index itself then stands.)
+  if (tid < m) perm[tid] = tid;
+  __syncthreads();
+  for (int i = tid; i < m; i += kEigT) {
     const double di = A[i + i * la].x;
     int rank = 0;
     for (int j = 0; j < m; ++j) {
@@ -635,20 +724,29 @@ __global__ __launch_bounds__(kKT) void k_kd_eigen(const KDesc* __restrict__ D, K
   }
   __syncthreads();
   int nf = 0;
-  for (int r = threadIdx.x; r < nb; r += blockDim.x) {
+  for (int r = tid; r < nb; r += kEigT) {
     const double v = A[perm[r] + perm[r] * la].x;
     nf |= !isfinite(v);
     st.values[r] = v;
   }
-  // C = L^-H Y (back substitution per wanted column).
-  for (int r = threadIdx.x; r < nb; r += blockDim.x) {
-    const int src = perm[r];
-    double2* c = d.C + int64_t(r) * cap;
+  // C = L^-H Y: back substitution per wanted column in place in Q.
+  for (int r = col0; r < nb; r += kEigT / 8) {
+    double2* x = W + perm[r] * la;
     for (int i = m - 1; i >= 0; --i) {
-      double2 z = W[i + src * la];
-      for (int p = i + 1; p < m; ++p) z = zsub(z, zcmul(Ls[p + i * la], c[p]));
-      c[i] = zscale(1.0 / Ls[i + i * la].x, z);
-      nf |= !(isfinite(c[i].x) && isfinite(c[i].y));
+      double2 z = make_double2(0.0, 0.0);
+      for (int p = i + 1 + sub; p < m; p += 8) z = zadd(z, zcmul(Ls[p + i * la], x[p]));
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) {
+        z.x += __shfl_xor(z.x, off);
+        z.y += __shfl_xor(z.y, off);
+      }
+      if (sub == 0) {
+        const double2 y = zscale(1.0 / Ls[i + i * la].x, zsub(x[i], z));
+        x[i] = y;
+        d.C[i + int64_t(r) * cap] = y;
+        nf |= !(isfinite(y.x) && isfinite(y.y));
+      }
+      wave_order();
     }
   }
   if (nf) st.eig_bad = 1;
