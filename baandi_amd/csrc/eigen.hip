@@ -1053,6 +1053,297 @@ __global__ __launch_bounds__(kCT) void k_td_coop(int m, int nw, double* __restri
   }
 }
 
+// The same exchange with everything else of a step in registers, for m <= 64 R
+// and at most C columns of a worker in each of its 4 waves: lane l of a wave
+// owns rows l + 64 t of its columns, of the reflector v, of w and of the
+// copies of columns k + 1 and k + 2. Every wave of every worker forms w, the
+// copies and the next reflector by itself from the exchanged words (the same
+// code on the same data, the same bits everywhere), so a step meets the
+// workgroup once, where each wave has polled its share of the words and all of
+// them read them from LDS. A worker's columns take the update of step k in the
+// pass that multiplies them by v_{k+1}.
+//
+// Bound by the exchange (a store and a load through memory) and the chain of
+// wave sums around it (y.v, |x|^2, the products): 2.7 us a step at m = 320,
+// 3.1 us with the columns, reflector and sums in LDS (k_td_coop, eight
+// barriers a step).
+__device__ __forceinline__ double pick(const double* x, int t, int count) {
+  double v = x[0];
+#pragma unroll
+  for (int i = 1; i < 12; ++i)
+    if (i < count) v = i == t ? x[i] : v;
+  return v;
+}
+
+// Lane l's value of v (l uniform across the wave).
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+
+size_t coop_reg_lds(int m, int nw) { return size_t((int64_t((m + nw - 1) / nw) + 8) * m + 2) * 8; }
+
+template <int R, int C>
+__global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, double* __restrict__ A, int64_t lda,
+                                                     double* __restrict__ d, double* __restrict__ e,
+                                                     double* __restrict__ tau, uint64_t* __restrict__ words,
+                                                     int* __restrict__ info, long long spins) {
+  static_assert(kCT == 256 && R <= 12, "rows of a lane, four waves");
+  constexpr int NWV = kCT / 64, kRd = (64 * R + kCT - 1) / kCT;
+  extern __shared__ __align__(16) double sh[];
+  const int me = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ncl = (m - me + nw - 1) / nw;  // columns me, me + nw, ...
+  double* Al = sh;                         // the reflectors of this worker's columns, m rows each
+  double* ys = Al + int64_t((m + nw - 1) / nw) * m;  // two slots of y
+  double* cs = ys + 2 * m;                           // two slots of column k + 2
+  double* vs = cs + 2 * m + int64_t(wave) * m;       // this wave's copy of v
+  // One flag a parity: a wave that fails at step k + 1 must not stop another
+  // that has yet to look at step k's.
+  int* go = reinterpret_cast<int*>(cs + 2 * m + NWV * int64_t(m));
+  uint64_t* yslot[2] = {words, words + 2 * int64_t(m)};
+  uint64_t* cslot[2] = {words + 4 * int64_t(m), words + 6 * int64_t(m)};
+  if (tid < 2) go[tid] = 1;
+  __syncthreads();
+  // Own column ci of this wave: global column me + (wave + 4 ci) nw.
+  double a[C][R], v[R], c1[R], c2[R];
+  auto entry = [&](int r, int c) { return r >= m || c >= m ? 0.0 : r >= c ? A[r + int64_t(c) * lda] : A[c + int64_t(r) * lda]; };
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int r = lane + 64 * t;
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) a[ci][t] = entry(r, me + (wave + NWV * ci) * nw);
+    c2[t] = entry(r, 0);
+    c1[t] = entry(r, 1);
+  }
+  double tk = 0.0;
+  // Reflector k from `col` (column k as of step k - 1): v (zero up to row k),
+  // tau; d, e and tau by one wave, the owner keeps v for the end.
+  auto reflector = [&](int k, const double* col) {
+    double ss = 0.0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) ss = lane + 64 * t > k ? fma(col[t], col[t], ss) : ss;
+    ss = wave_sum(ss);
+    const double x0 = lane_value(pick(col, (k + 1) >> 6, R), (k + 1) & 63);
+    const double sigma = sqrt(ss);
+    double alpha = 0.0;
+    tk = 0.0;
+    if (sigma > 0.0) {
+      alpha = x0 >= 0.0 ? -sigma : sigma;
+      tk = 1.0 / (sigma * (sigma + fabs(x0)));
+    }
+    const double first = sigma > 0.0 ? x0 - alpha : x0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = lane + 64 * t;
+      v[t] = r == k + 1 ? first : r > k + 1 ? col[t] : 0.0;
+      if (r < m) vs[r] = v[t];
+    }
+    if (me == 0 && wave == 0) {
+      const double dk = lane_value(pick(col, k >> 6, R), k & 63);
+      if (lane == 0) {
+        d[k] = dk;
+        e[k] = alpha;
+        tau[k] = tk;
+      }
+    }
+    if (k % nw == me && wave == NWV - 1) {
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        if (lane + 64 * t < m) Al[int64_t(k / nw) * m + lane + 64 * t] = v[t];
+    }
+  };
+  // y_j = A[:, j].v of the own columns j > k, published by one lane each.
+  auto products = [&](int k, uint64_t* yb) {
+    double s[C];
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      s[ci] = 0.0;
+#pragma unroll
+      for (int t = 0; t < R; ++t) s[ci] = fma(a[ci][t], v[t], s[ci]);
+    }
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) s[ci] = wave_sum(s[ci]);
+    double mine = s[0];
+#pragma unroll
+    for (int ci = 1; ci < C; ++ci) mine = lane == ci ? s[ci] : mine;
+    const int j = me + (wave + NWV * lane) * nw;
+    if (lane < C && j > k && j < m) ll_put(yb + 2 * j, mine, uint32_t(k + 1));
+  };
+  reflector(0, c2);
+  int k = 0;
+  bool failed = false;
+  for (; k + 2 < m; ++k) {
+    const uint32_t tag = uint32_t(k + 1);
+    uint64_t* yb = yslot[k & 1];
+    uint64_t* cb = cslot[k & 1];
+    // A. Column k + 2 from its owner (as of step k - 1), this wave's products.
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci)
+      if (me + (wave + NWV * ci) * nw == k + 2) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+          const int r = lane + 64 * t;
+          if (r > k && r < m) ll_put(cb + 2 * r, a[ci][t], tag);
+        }
+      }
+    products(k, yb);
+    // B. This wave's share of y and of column k + 2 into LDS.
+    double* yl = ys + (k & 1) * m;
+    double* cl = cs + (k & 1) * m;
+    bool ok = spins >= 0;
+    {
+      bool late[kRd];
+#pragma unroll
+      for (int j = 0; j < kRd; ++j) {
+        const int r = tid + j * kCT;
+        late[j] = r > k && r < m;
+        if (r < m && r <= k) yl[r] = cl[r] = 0.0;
+      }
+      // The words are on their way for about this long, and polling them
+      // meanwhile holds the writers up (m = 160, 240, 320: 690, 1054, 1511 us
+      // a whole solve; 811, 1244, 1603 polling at once).
+      __builtin_amdgcn_s_sleep(14);
+      for (long long tries = 0; ok; ++tries) {
+        uint64_t w4[kRd][4];
+#pragma unroll
+        for (int j = 0; j < kRd; ++j)
+          if (late[j]) {
+            const uint64_t* py = yb + 2 * (tid + j * kCT);
+            const uint64_t* pc = cb + 2 * (tid + j * kCT);
+            w4[j][0] = __hip_atomic_load(py, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            w4[j][1] = __hip_atomic_load(py + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            w4[j][2] = __hip_atomic_load(pc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            w4[j][3] = __hip_atomic_load(pc + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < kRd; ++j)
+          if (late[j]) {
+            const int r = tid + j * kCT;
+            if (uint32_t(w4[j][0] >> 32) == tag && uint32_t(w4[j][1] >> 32) == tag &&
+                uint32_t(w4[j][2] >> 32) == tag && uint32_t(w4[j][3] >> 32) == tag) {
+              yl[r] = __longlong_as_double((long long)((w4[j][1] << 32) | (w4[j][0] & 0xffffffffull)));
+              cl[r] = __longlong_as_double((long long)((w4[j][3] << 32) | (w4[j][2] & 0xffffffffull)));
+              late[j] = false;
+            } else {
+              any = true;
+            }
+          }
+        if (!any) break;
+        if (tries > spins) ok = false;
+        if ((tries & 63) == 63 && __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) ok = false;
+      }
+    }
+    if (!ok) go[k & 1] = 0;
+    __syncthreads();
+    if (!go[k & 1]) {
+      failed = true;
+      break;
+    }
+    // w = tau y - (tau^2/2 y.v) v in every wave; a column j takes the update
+    // c - (v w_j + w v_j), each product rounded on its own.
+    double w[R], s = 0.0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = lane + 64 * t;
+      w[t] = r < m ? yl[r] : 0.0;
+      c2[t] = r < m ? cl[r] : 0.0;
+      s = fma(w[t], v[t], s);
+    }
+    const double y1 = yl[k + 1], y2 = yl[k + 2], v1 = vs[k + 1], v2 = vs[k + 2];
+    double yj[C], vj[C];
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      const int j = min(me + (wave + NWV * ci) * nw, m - 1);
+      yj[ci] = yl[j];
+      vj[ci] = vs[j];
+    }
+    s = wave_sum(s);
+    const double K = 0.5 * tk * tk * s;
+    auto w_of = [&](double y, double x) { return fma(-K, x, __dmul_rn(tk, y)); };
+    auto updated = [&](double c, double x, double wr, double xj, double wj) {
+      return c - __dadd_rn(__dmul_rn(x, wj), __dmul_rn(wr, xj));
+    };
+    const double w1 = w_of(y1, v1), w2 = w_of(y2, v2);
+    double wj[C], vold[R];
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) wj[ci] = w_of(yj[ci], vj[ci]);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      w[t] = w_of(w[t], v[t]);
+      c1[t] = updated(c1[t], v[t], w[t], v1, w1);
+      c2[t] = updated(c2[t], v[t], w[t], v2, w2);
+      vold[t] = v[t];
+    }
+    // C. Reflector k + 1 (or, after the last step, the trailing 2 x 2).
+    if (k + 3 < m) {
+      reflector(k + 1, c1);
+    } else if (me == 0 && wave == 0) {
+      const double da = lane_value(pick(c1, (m - 2) >> 6, R), (m - 2) & 63);
+      const double eb = lane_value(pick(c1, (m - 1) >> 6, R), (m - 1) & 63);
+      const double db = lane_value(pick(c2, (m - 1) >> 6, R), (m - 1) & 63);
+      if (lane == 0) {
+        d[m - 2] = da;
+        e[m - 2] = eb;
+        tau[m - 2] = 0.0;
+        d[m - 1] = db;
+        tau[m - 1] = 0.0;
+      }
+    }
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+#pragma unroll
+      for (int t = 0; t < R; ++t) a[ci][t] = updated(a[ci][t], vold[t], w[t], vj[ci], wj[ci]);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) c1[t] = c2[t];
+  }
+  if (failed) {
+    // Abandoned: the failure is in *info; a zero tridiagonal keeps the
+    // later stages' inputs finite.
+    if (tid == 0) __hip_atomic_store(info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = tid; i < m; i += kCT) {
+      d[i] = 0.0;
+      e[i] = 0.0;
+      tau[i] = 0.0;
+    }
+    return;
+  }
+  __syncthreads();  // the reflectors, kept by one wave
+  for (int lc = 0; lc < ncl; ++lc) {
+    const int c = me + lc * nw;
+    if (c >= m - 2) continue;
+    const double* col = Al + int64_t(lc) * m;
+    for (int r = c + 1 + tid; r < m; r += kCT) A[r + int64_t(c) * lda] = col[r];
+  }
+}
+
+typedef void (*CoopReg)(int, int, double*, int64_t, double*, double*, double*, uint64_t*, int*, long long);
+
+// The register kernel for m rows on nw workers; nullptr where a lane's share
+// does not fit (few workers, or past 640 rows, where the reflectors and slots
+// no longer fit the LDS either).
+CoopReg coop_reg_kernel(int m, int nw) {
+  const int R = (m + 63) / 64, C = ((m + nw - 1) / nw + 3) / 4;
+  if (coop_reg_lds(m, nw) > 160 * 1024) return nullptr;
+  if (R <= 6 && C <= 3) {
+    switch (R) {
+      case 1:
+      case 2: return &k_td_coop_reg<2, 3>;
+      case 3: return &k_td_coop_reg<3, 3>;
+      case 4: return &k_td_coop_reg<4, 3>;
+      case 5: return &k_td_coop_reg<5, 3>;
+      case 6: return &k_td_coop_reg<6, 3>;
+    }
+  }
+  if (R <= 8 && C <= 4) return &k_td_coop_reg<8, 4>;
+  if (R <= 10 && C <= 5) return &k_td_coop_reg<10, 5>;
+  return nullptr;
+}
+
 // ---------------------------------------------------------------------------
 // 1e. Complex Hermitian tridiagonalisation (the k-point Davidson's reduced
 // problem): Householder reflectors H_k = I - tau_k v_k v_k^H with v_k[0] = 1
@@ -1903,10 +2194,16 @@ void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, do
   if (m >= 3 && m >= multi_from.load()) {
     tridiag_multi(s, m, A, lda, L, L.td);
   } else if (nw > 0) {
-    allow_full_lds(reinterpret_cast<const void*>(&k_td_coop), "k_td_coop");
     zero_doubles(s, reinterpret_cast<double*>(L.words), coop_words(m));
-    hipLaunchKernelGGL(k_td_coop, dim3(nw), dim3(kCT), coop_lds(m, nw), s, m, nw, A, lda, L.d, L.e, L.tau,
-                       L.words, info, (long long)coop_spins.load());
+    if (const CoopReg reg = coop_reg_kernel(m, nw)) {
+      if (coop_reg_lds(m, nw) > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(reg), "k_td_coop_reg");
+      hipLaunchKernelGGL(reg, dim3(nw), dim3(kCT), coop_reg_lds(m, nw), s, m, nw, A, lda, L.d, L.e, L.tau, L.words,
+                         info, (long long)coop_spins.load());
+    } else {
+      allow_full_lds(reinterpret_cast<const void*>(&k_td_coop), "k_td_coop");
+      hipLaunchKernelGGL(k_td_coop, dim3(nw), dim3(kCT), coop_lds(m, nw), s, m, nw, A, lda, L.d, L.e, L.tau,
+                         L.words, info, (long long)coop_spins.load());
+    }
   } else if (blocked && m >= 3 && panel_lds <= 160 * 1024) {
     if (panel_lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_tridiag_panel), "k_tridiag_panel");
     hipLaunchKernelGGL(k_lower_to_upper, dim3((m + 255) / 256, m), dim3(256), 0, s, m, A, lda);
