@@ -25,7 +25,7 @@ namespace bd {
 
 namespace {
 constexpr int kCT = 1024;
-constexpr int kInvRows = 2;  // k_chol_inv_lds: rows per lane of the substitution (k <= 128)
+constexpr int kInvRows = 2;  // k_chol_inv_lds: rows a lane (k <= 128)
 constexpr double kPivotRatioMin = DBL_EPSILON / 1e-12;  // lean_davidson.rs:62-64
 
 // Lane l's value of v (l uniform across the wave).
@@ -48,88 +48,153 @@ __global__ void k_copy_block(int k, const double* __restrict__ S, int64_t lds, d
 }
 
 // Cholesky of the k x k block G (k <= 64 * kInvRows) with the pivot-ratio
-// test, then T22 = L^{-1} into T (ld ldt), zero above the diagonal. The block
-// sits in LDS as a packed lower triangle (column-major): an LDL^T elimination
-// with one barrier per column (column j is only read while the columns right
-// of it are updated), then L = column j over sqrt(d_j), then L^{-1} by
-// forward substitution, a wave per column with the right-hand side in
-// registers. A flag already set by an earlier block of the same border
-// leaves the block untouched; min_ratio keeps the minimum over the blocks.
+// test, then T22 = L^{-1} into T (ld ldt), zero above the diagonal. A flag
+// already set by an earlier block of the same border leaves the block
+// untouched; min_ratio keeps the minimum over the blocks.
+//
+// G = M D M^T with M unit lower: column l sits in the registers of wave
+// l mod 16 (lane i owns row i, and i + 64 past 64 rows), and a step passes one column
+// through LDS: one barrier, one division. The pivots are tested together at
+// the end (a failed one only spoils later columns, which nobody then reads).
+// M^{-1} by forward substitution, a wave's columns side by side so that their
+// chains (a lane read and the update) overlap; L^{-1} = D^{-1/2} M^{-1}.
+// Bound by the chain of steps. k = 80: 51 us, k = 20: 7; 98 and 16 with the
+// block as a packed triangle in LDS, two divisions a step and one column at a
+// time in the substitution.
+template <int NC>
 __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __restrict__ G,
                                                       const double* __restrict__ sdiag, int64_t sstride,
                                                       double* __restrict__ T22, int64_t ldt, int* __restrict__ flag,
                                                       double* __restrict__ min_ratio) {
   extern __shared__ double sh[];
   if (flag[0]) return;  // an earlier block of this border failed: uniform exit
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  constexpr int nw = kCT / 64;
-  double* P = sh;
-  double* rhsall = sh + int64_t(k) * (k + 1) / 2;
-  auto pk = [k](int i, int l) { return l * k - (l * (l - 1)) / 2 + (i - l); };
-  for (int l = wave; l < k; l += nw)
-    for (int i = l + lane; i < k; i += 64) P[pk(i, l)] = G[i + int64_t(l) * k];
+  // NC columns a wave; rows a lane.
+  constexpr int nw = kCT / 64, R = NC * nw <= 64 ? 1 : 2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ldm = k + 1;
+  double* M = sh;                        // k columns of ldm
+  double* pass = M + int64_t(k) * ldm;   // two slots of k: the column of a step
+  double* dv = pass + 2 * k;             // k: the pivots
+  double a[NC][R];
+  int row[R];  // this lane's rows, the last one's for those past it
+#pragma unroll
+  for (int t = 0; t < R; ++t) row[t] = min(lane + 64 * t, k - 1);
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int l = wave + nw * c, i = lane + 64 * t;
+      a[c][t] = l < k && i < k && i >= l ? G[i + int64_t(l) * k] : 0.0;
+    }
+#pragma unroll
+  for (int jc = 0; jc < NC; ++jc)
+    for (int jw = 0; jw < nw; ++jw) {
+      const int j = jc * nw + jw;
+      if (j >= k) break;
+      double* col = pass + (j & 1) * k;
+      if (wave == jw) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+          const int i = lane + 64 * t;
+          if (i < k) col[i] = a[jc][t];
+          if (i == j) dv[j] = a[jc][t];
+        }
+      }
+      __syncthreads();
+      // (Columns up to j take the update too; nothing reads them again.)
+      const double dj = col[j];
+      double mine[R], alj[NC];
+#pragma unroll
+      for (int t = 0; t < R; ++t) mine[t] = col[row[t]];
+#pragma unroll
+      for (int c = jc; c < NC; ++c) alj[c] = col[min(wave + nw * c, k - 1)];
+      const double inv_d = 1.0 / dj;
+#pragma unroll
+      for (int t = 0; t < R; ++t) mine[t] *= inv_d;
+#pragma unroll
+      for (int c = jc; c < NC; ++c)
+#pragma unroll
+        for (int t = 0; t < R; ++t) a[c][t] = fma(-alj[c], mine[t], a[c][t]);
+      if (wave == jw) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+          const int i = lane + 64 * t;
+          if (i < k) M[i + int64_t(j) * ldm] = i > j ? mine[t] : 0.0;
+        }
+      }
+    }
   __syncthreads();
+  // The pivots' ratios, up to the first that fails.
   double mr = INFINITY;
-  for (int j = 0; j < k; ++j) {
-    const double dj = P[pk(j, j)];
-    const double ratio = dj / sdiag[int64_t(j) * sstride];
-    if (isnan(ratio) || ratio < kPivotRatioMin) {
-      if (tid == 0) {
-        flag[0] = 1;
-        min_ratio[0] = isnan(ratio) ? 0.0 : fmin(min_ratio[0], fmin(mr, ratio));
+  bool failed = false, nan = false;
+  for (int j0 = 0; j0 < k && !failed; j0 += 64) {
+    const int j = j0 + lane;
+    const double ratio = j < k ? dv[j] / sdiag[int64_t(j) * sstride] : INFINITY;
+    const unsigned long long bad = __ballot(isnan(ratio) || ratio < kPivotRatioMin);
+    const int first = bad ? __ffsll(static_cast<long long>(bad)) - 1 : 63;
+    double r = lane <= first ? ratio : INFINITY;
+    nan = bad && isnan(__shfl(ratio, first, 64));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_xor(r, off, 64));
+    mr = fmin(mr, r);
+    failed = bad != 0;
+  }
+  if (tid == 0) {
+    min_ratio[0] = nan ? 0.0 : fmin(min_ratio[0], mr);
+    if (failed) flag[0] = 1;
+  }
+  if (failed) return;  // every wave found the same: uniform exit
+  double x[NC][R], ml[R];  // (M is zero up to the diagonal)
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    ml[t] = M[row[t]];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) x[c][t] = lane + 64 * t == wave + nw * c ? 1.0 : 0.0;
+  }
+#pragma unroll
+  for (int tl = 0; tl < R; ++tl) {
+    const int end = min(k, 64 * (tl + 1));
+    for (int l = 64 * tl; l < end; ++l) {
+      double next[R];
+#pragma unroll
+      for (int t = 0; t < R; ++t) next[t] = M[row[t] + int64_t(min(l + 1, k - 1)) * ldm];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const double xl = read_lane(x[c][tl], l - 64 * tl);
+#pragma unroll
+        for (int t = 0; t < R; ++t) x[c][t] = fma(-ml[t], xl, x[c][t]);
       }
-      return;  // every thread read the same pivot: uniform exit
-    }
-    mr = fmin(mr, ratio);
-    const double inv_d = 1.0 / dj;
-    for (int l = j + 1 + wave; l < k; l += nw) {
-      const double alj = P[pk(l, j)] * inv_d;
-      const int base_j = pk(0, j), base_l = pk(0, l);  // column starts (row index offsets follow)
-      for (int i = l + lane; i < k; i += 64) P[base_l + i] -= P[base_j + i] * alj;
-    }
-    __syncthreads();
-  }
-  for (int l = wave; l < k; l += nw) {
-    const double sd = sqrt(P[pk(l, l)]);
-    for (int i = l + 1 + lane; i < k; i += 64) P[pk(i, l)] /= sd;
-  }
-  __syncthreads();
-  for (int l = tid; l < k; l += kCT) {
-    const double sd = sqrt(P[pk(l, l)]);
-    P[pk(l, l)] = sd;
-    rhsall[l] = 1.0 / sd;  // reciprocal diagonal for the substitution
-  }
-  __syncthreads();
-  if (tid == 0) min_ratio[0] = fmin(min_ratio[0], mr);
-  // Column c of L^{-1}: forward substitution L x = e_c, one wave per column,
-  // the right-hand side in registers (lane owns rows lane + 64 t, t <
-  // kInvRows), x_l broadcast from its owner lane: the serial chain per row is
-  // a lane read, a multiply and the update, with no LDS round trip.
-  const double* rd = rhsall;
-  for (int c = __builtin_amdgcn_readfirstlane(wave); c < k; c += nw) {
-    double r[kInvRows];
 #pragma unroll
-    for (int t = 0; t < kInvRows; ++t) r[t] = lane + 64 * t == c ? 1.0 : 0.0;
-    for (int l = c; l < k; ++l) {
-      const int tl = l >> 6, ll = l & 63;
-      double own = r[0];
-#pragma unroll
-      for (int t = 1; t < kInvRows; ++t) own = tl == t ? r[t] : own;
-      const double x = read_lane(own, ll) * rd[l];
-      const int base_l = pk(0, l);  // P[base_l + i] is in bounds for every i < k
-#pragma unroll
-      for (int t = 0; t < kInvRows; ++t) {
-        const int i = lane + 64 * t;
-        const double upd = r[t] - P[base_l + min(i, k - 1)] * x;
-        r[t] = i == l ? x : ((i > l && i < k) ? upd : r[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < kInvRows; ++t) {
-      const int i = lane + 64 * t;
-      if (i < k) T22[i + int64_t(c) * ldt] = i >= c ? r[t] : 0.0;
+      for (int t = 0; t < R; ++t) ml[t] = next[t];
     }
   }
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int i = lane + 64 * t;
+    if (i >= k) continue;
+    const double rs = 1.0 / sqrt(dv[i]);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int l = wave + nw * c;
+      if (l < k) T22[i + int64_t(l) * ldt] = i >= l ? x[c][t] * rs : 0.0;
+    }
+  }
+}
+
+typedef void (*CholInv)(int, const double*, const double*, int64_t, double*, int64_t, int*, double*);
+CholInv chol_inv_kernel(int k) {
+  switch ((k * 64 + kCT - 1) / kCT) {  // columns a wave
+    case 1: return &k_chol_inv_lds<1>;
+    case 2: return &k_chol_inv_lds<2>;
+    case 3: return &k_chol_inv_lds<3>;
+    case 4: return &k_chol_inv_lds<4>;
+    case 5: return &k_chol_inv_lds<5>;
+    case 6: return &k_chol_inv_lds<6>;
+    case 7: return &k_chol_inv_lds<7>;
+    case 8: return &k_chol_inv_lds<8>;
+  }
+  return nullptr;
 }
 
 // One wave per new row i of T: finiteness and the growth guard.
@@ -197,7 +262,7 @@ int64_t factor_gwork(int cap) { return int64_t(cap < 256 ? 1 : cap / 256) * cap 
 
 namespace {
 // Widest border block k_chol_inv_lds holds: its rows live in the kInvRows
-// registers of a lane, and k(k+1)/2 + k doubles fit the 160 KB of LDS.
+// registers of a lane, and k(k + 1) + 3k doubles fit the 160 KB of LDS.
 constexpr int kFactorBlock = 64 * kInvRows;
 // Widest block a border is split into: the elimination costs ~k^3 / 3 in
 // barriered column steps, so narrower blocks plus the extension GEMMs cost less.
@@ -212,10 +277,11 @@ void extend_block(hipStream_t s, const double* S, double* T, int cap, int from, 
                      S + from + int64_t(from) * cap, int64_t(cap), fw.G);
   if (from > 0) gemm_tn(s, k, k, from, -1.0, fw.W, from, fw.W, from, 1.0, fw.G, k, fw.gwork);
   double* T22 = T + from + int64_t(from) * cap;
-  const size_t lds = (size_t(k) * (k + 1) / 2 + size_t(k)) * 8;
+  const size_t lds = (size_t(k) * (k + 1) + 3 * size_t(k)) * 8;
   if (k > kFactorBlock || lds > 160 * 1024) fail(BD_ERR_INVALID_PARAMETER, "inverse Cholesky block too large");
-  if (lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_chol_inv_lds), "k_chol_inv_lds");
-  hipLaunchKernelGGL(k_chol_inv_lds, dim3(1), dim3(kCT), lds, s, k, fw.G, S + from + int64_t(from) * cap,
+  const CholInv chol = chol_inv_kernel(k);
+  if (lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(chol), "k_chol_inv_lds");
+  hipLaunchKernelGGL(chol, dim3(1), dim3(kCT), lds, s, k, fw.G, S + from + int64_t(from) * cap,
                      int64_t(cap) + 1, T22, int64_t(cap), fw.flag, fw.min_ratio);
   if (from > 0) {
     gemm_tn(s, k, from, from, 1.0, fw.W, from, T, cap, 0.0, fw.U, k, fw.gwork);         // U = W^T T11
