@@ -1053,7 +1053,9 @@ __global__ __launch_bounds__(kCT) void k_td_coop(int m, int nw, double* __restri
   }
 }
 
-// The same exchange with everything else of a step in registers, for m <= 64 R
+// The first `steps` reflectors by the same exchange with everything else of a
+// step in registers (steps < m - 2: the trailing matrix goes back into A's
+// lower triangle), for m <= 64 R
 // and at most C columns of a worker in each of its 4 waves: lane l of a wave
 // owns rows l + 64 t of its columns, of the reflector v, of w and of the
 // copies of columns k + 1 and k + 2. Every wave of every worker forms w, the
@@ -1085,7 +1087,7 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 size_t coop_reg_lds(int m, int nw) { return size_t((int64_t((m + nw - 1) / nw) + 8) * m + 2) * 8; }
 
 template <int R, int C>
-__global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, double* __restrict__ A, int64_t lda,
+__global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, int steps, double* __restrict__ A, int64_t lda,
                                                      double* __restrict__ d, double* __restrict__ e,
                                                      double* __restrict__ tau, uint64_t* __restrict__ words,
                                                      int* __restrict__ info, long long spins) {
@@ -1175,7 +1177,7 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, double* __re
   reflector(0, c2);
   int k = 0;
   bool failed = false;
-  for (; k + 2 < m; ++k) {
+  for (; k < steps; ++k) {
     const uint32_t tag = uint32_t(k + 1);
     uint64_t* yb = yslot[k & 1];
     uint64_t* cb = cslot[k & 1];
@@ -1278,10 +1280,10 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, double* __re
       c2[t] = updated(c2[t], v[t], w[t], v2, w2);
       vold[t] = v[t];
     }
-    // C. Reflector k + 1 (or, after the last step, the trailing 2 x 2).
-    if (k + 3 < m) {
+    // C. Reflector k + 1 (or, after the last step of all, the trailing 2 x 2).
+    if (k + 1 < steps) {
       reflector(k + 1, c1);
-    } else if (me == 0 && wave == 0) {
+    } else if (steps == m - 2 && me == 0 && wave == 0) {
       const double da = lane_value(pick(c1, (m - 2) >> 6, R), (m - 2) & 63);
       const double eb = lane_value(pick(c1, (m - 1) >> 6, R), (m - 1) & 63);
       const double db = lane_value(pick(c2, (m - 1) >> 6, R), (m - 1) & 63);
@@ -1313,15 +1315,234 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, double* __re
     return;
   }
   __syncthreads();  // the reflectors, kept by one wave
+  // What is left to reduce (lower triangle), for the kernel that goes on.
+  if (steps < m - 2) {
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      const int c = me + (wave + NWV * ci) * nw;
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        if (c >= steps && c < m && lane + 64 * t >= c && lane + 64 * t < m)
+          A[lane + 64 * t + int64_t(c) * lda] = a[ci][t];
+    }
+  }
   for (int lc = 0; lc < ncl; ++lc) {
     const int c = me + lc * nw;
-    if (c >= m - 2) continue;
+    if (c >= steps) continue;
     const double* col = Al + int64_t(lc) * m;
     for (int r = c + 1 + tid; r < m; r += kCT) A[r + int64_t(c) * lda] = col[r];
   }
 }
 
-typedef void (*CoopReg)(int, int, double*, int64_t, double*, double*, double*, uint64_t*, int*, long long);
+// A small matrix (m <= 64 R), or the end of a large one, in one workgroup of
+// eight waves as in k_td_coop_reg: columns in registers (wave w owns columns
+// w + 8 ci), every wave forms w, the column copies and the next reflector by
+// itself; y and column k + 2 pass through LDS, one barrier a step. The C sums
+// of a wave's products are reduced together: lane halves and then 16-lane rows
+// are swapped between pairs of sums, so that each add halves the sums left,
+// and only the last four levels run within a row.
+//
+// Bound by the chain of a step (three wave sums, a square root, a division, the
+// barrier): 1.3 us a step up to 64 rows, 2.3 us up to 128. m = 40: 107 -> 43
+// us (k_tridiag_panel); m = 320 with its last 128 rows here: 860 -> 725 us.
+constexpr int kOneT = 512;
+
+// s[0 .. C-1] summed over the wave's lanes: afterwards lane 15 of row r (of 16
+// lanes) holds, in out[q], the sum 4 q + {0, 2, 1, 3}[r].
+template <int C>
+__device__ __forceinline__ void wave_sums(const double (&s)[C], double (&out)[C / 4]) {
+  auto swap_add = [](double x, double y, auto swap) {
+    const auto lo = swap(unsigned(__double2loint(x)), unsigned(__double2loint(y)));
+    const auto hi = swap(unsigned(__double2hiint(x)), unsigned(__double2hiint(y)));
+    return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
+  };
+  auto swap32 = [](unsigned x, unsigned y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+  auto swap16 = [](unsigned x, unsigned y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+#pragma unroll
+  for (int q = 0; q < C / 4; ++q) {
+    double v = swap_add(swap_add(s[4 * q], s[4 * q + 1], swap32), swap_add(s[4 * q + 2], s[4 * q + 3], swap32), swap16);
+    v += dpp::move<0x111, 0xF, 0xF>(v);  // row_shr:1, 2, 4, 8
+    v += dpp::move<0x112, 0xF, 0xF>(v);
+    v += dpp::move<0x114, 0xF, 0xF>(v);
+    v += dpp::move<0x118, 0xF, 0xF>(v);
+    out[q] = v;
+  }
+}
+
+template <int R, int C>
+__global__ __launch_bounds__(kOneT) void k_td_one(int m, int steps, double* __restrict__ A, int64_t lda,
+                                                  double* __restrict__ d, double* __restrict__ e,
+                                                  double* __restrict__ tau) {
+  constexpr int NWV = kOneT / 64, N = 64 * R;
+  static_assert(C % 4 == 0 && NWV * C == N, "columns of a wave");
+  __shared__ double ys[2][N], cs[2][N];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  double a[C][R], v[R], c1[R], c2[R];
+  auto entry = [&](int r, int c) { return r >= m || c >= m ? 0.0 : r >= c ? A[r + int64_t(c) * lda] : A[c + int64_t(r) * lda]; };
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int r = lane + 64 * t;
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) a[ci][t] = entry(r, wave + NWV * ci);
+    c2[t] = entry(r, 0);
+    c1[t] = entry(r, 1);
+  }
+  for (int i = threadIdx.x; i < 2 * N; i += kOneT) ys[i / N][i % N] = cs[i / N][i % N] = 0.0;
+  __syncthreads();  // A is read: reflectors may go into it
+  double tk = 0.0;
+  auto reflector = [&](int k, const double* col) {
+    double ss = 0.0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) ss = lane + 64 * t > k ? fma(col[t], col[t], ss) : ss;
+    ss = wave_sum(ss);
+    const double x0 = lane_value(pick(col, (k + 1) >> 6, R), (k + 1) & 63);
+    const double sigma = sqrt(ss);
+    double alpha = 0.0;
+    tk = 0.0;
+    if (sigma > 0.0) {
+      alpha = x0 >= 0.0 ? -sigma : sigma;
+      tk = 1.0 / (sigma * (sigma + fabs(x0)));
+    }
+    const double first = sigma > 0.0 ? x0 - alpha : x0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const int r = lane + 64 * t;
+      v[t] = r == k + 1 ? first : r > k + 1 ? col[t] : 0.0;
+    }
+    if (wave == k % NWV) {
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        const int r = lane + 64 * t;
+        if (r > k && r < m) A[r + int64_t(k) * lda] = v[t];
+      }
+      const double dk = lane_value(pick(col, k >> 6, R), k & 63);
+      if (lane == 0) {
+        d[k] = dk;
+        e[k] = alpha;
+        tau[k] = tk;
+      }
+    }
+  };
+  reflector(0, c2);
+  for (int k = 0; k < steps; ++k) {
+    double* yl = ys[k & 1];
+    double* cl = cs[k & 1];
+    // A. Column k + 2 (as of step k - 1) and this wave's products.
+    if ((k + 2) % NWV == wave) {
+#pragma unroll
+      for (int t = 0; t < R; ++t) {
+        double c = a[0][t];
+#pragma unroll
+        for (int ci = 1; ci < C; ++ci) c = ci == (k + 2) / NWV ? a[ci][t] : c;
+        cl[lane + 64 * t] = c;
+      }
+    }
+    double s[C], sums[C / 4];
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      s[ci] = a[ci][0] * v[0];
+#pragma unroll
+      for (int t = 1; t < R; ++t) s[ci] = fma(a[ci][t], v[t], s[ci]);
+    }
+    wave_sums(s, sums);
+    if ((lane & 15) == 15) {
+      const int row = lane >> 4, at = row == 1 ? 2 : row == 2 ? 1 : row;
+#pragma unroll
+      for (int q = 0; q < C / 4; ++q) {
+        const int j = wave + NWV * (4 * q + at);
+        yl[j] = j > k ? sums[q] : 0.0;
+      }
+    }
+    __syncthreads();
+    // B. w = tau y - (tau^2/2 y.v) v in every wave; a column j takes the update
+    // c - (v w_j + w v_j), each product rounded on its own.
+    double w[R], vold[R], yv = 0.0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      w[t] = yl[lane + 64 * t];
+      c2[t] = cl[lane + 64 * t];
+      yv = fma(w[t], v[t], yv);
+    }
+    yv = wave_sum(yv);
+    const double K = 0.5 * tk * tk * yv;
+    auto updated = [&](double c, double x, double wr, double xj, double wj) {
+      return c - __dadd_rn(__dmul_rn(x, wj), __dmul_rn(wr, xj));
+    };
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      w[t] = fma(-K, v[t], __dmul_rn(tk, w[t]));
+      vold[t] = v[t];
+    }
+    const double v1 = lane_value(pick(v, (k + 1) >> 6, R), (k + 1) & 63);
+    const double v2 = lane_value(pick(v, (k + 2) >> 6, R), (k + 2) & 63);
+    const double w1 = lane_value(pick(w, (k + 1) >> 6, R), (k + 1) & 63);
+    const double w2 = lane_value(pick(w, (k + 2) >> 6, R), (k + 2) & 63);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      c1[t] = updated(c1[t], v[t], w[t], v1, w1);
+      c2[t] = updated(c2[t], v[t], w[t], v2, w2);
+    }
+    // C. Reflector k + 1 (or, after the last step of all, the trailing 2 x 2).
+    if (k + 1 < steps) {
+      reflector(k + 1, c1);
+    } else if (steps == m - 2 && wave == 0) {
+      const double da = lane_value(pick(c1, (m - 2) >> 6, R), (m - 2) & 63);
+      const double eb = lane_value(pick(c1, (m - 1) >> 6, R), (m - 1) & 63);
+      const double db = lane_value(pick(c2, (m - 1) >> 6, R), (m - 1) & 63);
+      if (lane == 0) {
+        d[m - 2] = da;
+        e[m - 2] = eb;
+        tau[m - 2] = 0.0;
+        d[m - 1] = db;
+        tau[m - 1] = 0.0;
+      }
+    }
+    // Row j of column j = wave + NWV ci: lane j % 64, t = j / 64. (Taken a
+    // few columns at a time: all at once they would not fit the scalar
+    // registers.)
+    constexpr int P = 64 / NWV;
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      if (ci % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+      const double wj = lane_value(w[ci / P], wave + NWV * (ci % P));
+      const double vj = lane_value(vold[ci / P], wave + NWV * (ci % P));
+#pragma unroll
+      for (int t = 0; t < R; ++t) a[ci][t] = updated(a[ci][t], vold[t], w[t], vj, wj);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) c1[t] = c2[t];
+  }
+  if (steps < m - 2) {
+#pragma unroll
+    for (int ci = 0; ci < C; ++ci) {
+      const int c = wave + NWV * ci;
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        if (c >= steps && c < m && lane + 64 * t >= c && lane + 64 * t < m)
+          A[lane + 64 * t + int64_t(c) * lda] = a[ci][t];
+    }
+  }
+}
+
+// Matrices of 3 <= m <= kOneMax, 64 rows a register: the kernel for two
+// registers takes the size down to 64, where the one for one register goes on.
+constexpr int kOneMax = 128;
+
+void tridiag_one(hipStream_t s, int m, double* A, int64_t lda, double* d, double* e, double* tau) {
+  if (m > 64) {
+    const int steps = m - 64;
+    hipLaunchKernelGGL((k_td_one<2, 16>), dim3(1), dim3(kOneT), 0, s, m, steps, A, lda, d, e, tau);
+    A += steps * (lda + 1);
+    d += steps;
+    e += steps;
+    tau += steps;
+    m = 64;
+  }
+  hipLaunchKernelGGL((k_td_one<1, 8>), dim3(1), dim3(kOneT), 0, s, m, m - 2, A, lda, d, e, tau);
+}
+
+typedef void (*CoopReg)(int, int, int, double*, int64_t, double*, double*, double*, uint64_t*, int*, long long);
 
 // The register kernel for m rows on nw workers; nullptr where a lane's share
 // does not fit (few workers, or past 640 rows, where the reflectors and slots
@@ -2212,20 +2433,28 @@ void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, do
   const EigenLayout L = eigen_layout(m, want, work);
   hipLaunchKernelGGL(k_zero_i, dim3(1), dim3(64), 0, s, info, 1);
   const size_t panel_lds = tridiag_panel_lds(m);
-  const int nw = blocked ? coop_worker_count(m) : 0;
+  const bool automatic = blocked && coop_workers.load() < 0;
+  const int nw = blocked && !(automatic && m <= kOneMax) ? coop_worker_count(m) : 0;
   if (m >= 3 && m >= multi_from.load()) {
     tridiag_multi(s, m, A, lda, L, L.td);
   } else if (nw > 0) {
     zero_doubles(s, reinterpret_cast<double*>(L.words), coop_words(m));
     if (const CoopReg reg = coop_reg_kernel(m, nw)) {
+      // The last kOneMax rows in one workgroup, where a step costs less than
+      // the exchange between several (2.7 us).
+      const int steps = automatic ? m - kOneMax : m - 2;
       if (coop_reg_lds(m, nw) > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(reg), "k_td_coop_reg");
-      hipLaunchKernelGGL(reg, dim3(nw), dim3(kCT), coop_reg_lds(m, nw), s, m, nw, A, lda, L.d, L.e, L.tau, L.words,
-                         info, (long long)coop_spins.load());
+      hipLaunchKernelGGL(reg, dim3(nw), dim3(kCT), coop_reg_lds(m, nw), s, m, nw, steps, A, lda, L.d, L.e, L.tau,
+                         L.words, info, (long long)coop_spins.load());
+      if (automatic)
+        tridiag_one(s, kOneMax, A + steps * (lda + 1), lda, L.d + steps, L.e + steps, L.tau + steps);
     } else {
       allow_full_lds(reinterpret_cast<const void*>(&k_td_coop), "k_td_coop");
       hipLaunchKernelGGL(k_td_coop, dim3(nw), dim3(kCT), coop_lds(m, nw), s, m, nw, A, lda, L.d, L.e, L.tau,
                          L.words, info, (long long)coop_spins.load());
     }
+  } else if (automatic && m >= 3 && m <= kOneMax) {
+    tridiag_one(s, m, A, lda, L.d, L.e, L.tau);
   } else if (blocked && m >= 3 && panel_lds <= 160 * 1024) {
     if (panel_lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_tridiag_panel), "k_tridiag_panel");
     hipLaunchKernelGGL(k_lower_to_upper, dim3((m + 255) / 256, m), dim3(256), 0, s, m, A, lda);
