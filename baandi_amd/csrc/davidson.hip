@@ -214,7 +214,14 @@ struct DavidsonWork {
   int* flag = nullptr;
   int* info = nullptr;  // [0] eigensolver, [1] factor verdict
   FactorWork fw;
+  // Pinned staging: kSlots uploads of up to nb values between two
+  // synchronisations, then the readbacks (nb values, nb values, two flags).
+  static constexpr int kSlots = 8;
+  char* pinned = nullptr;
+  size_t slot_bytes = 0;
   DavidsonWork(int64_t n_, int nb_, int cap_) : n(n_), nb(nb_), cap(cap_) {
+    slot_bytes = (size_t(nb) * 8 + 255) / 256 * 256;
+    BD_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), slot_bytes * (kSlots + 2) + 256, hipHostMallocDefault));
     const size_t c2 = size_t(cap) * cap;
     S.alloc(c2);
     H.alloc(c2);
@@ -256,6 +263,7 @@ struct DavidsonWork {
     BD_HIP(hipMalloc(&flag, sizeof(int)));
   }
   ~DavidsonWork() {
+    if (pinned) (void)hipHostFree(pinned);
     if (idx) (void)hipFree(idx);
     if (flag) (void)hipFree(flag);
     if (info) (void)hipFree(info);
@@ -289,7 +297,8 @@ struct Solver {
   // whether a guard trip has switched the ideal reset off for its rest.
   int contractions = 0;
   bool reset_disabled = false;
-  hipEvent_t ev0, ev1;
+  hipEvent_t ev0, ev1, ev2, ev3;
+  int slots_used = 0;
 
   Solver(GammaOp& op_, DavidsonWork& w_, const bd_davidson_options& o_, const double* diag_)
       : op(op_), w(w_), s(op_.stream), n(w_.n), nb(w_.nb), cap(w_.cap), o(o_), diag(diag_) {
@@ -303,10 +312,12 @@ struct Solver {
     old.assign(nb, 0.0);
     BD_HIP(hipEventCreate(&ev0));
     BD_HIP(hipEventCreate(&ev1));
+    BD_HIP(hipEventCreate(&ev2));
+    BD_HIP(hipEventCreate(&ev3));
   }
   ~Solver() {
-    (void)hipEventDestroy(ev0);
-    (void)hipEventDestroy(ev1);
+    (void)hipStreamSynchronize(s);  // (an error may leave copies from the staging queued)
+    for (hipEvent_t e : {ev0, ev1, ev2, ev3}) (void)hipEventDestroy(e);
   }
 
   double band_threshold(int i) const {
@@ -314,35 +325,60 @@ struct Solver {
     return std::max(5.0 * o.threshold, 5e-6);
   }
 
-  void sync() { BD_HIP(hipStreamSynchronize(s)); }
-  // Host sources are often temporaries: every upload completes before return.
+  void sync() {
+    BD_HIP(hipStreamSynchronize(s));
+    slots_used = 0;
+  }
+  // Uploads go through a pinned slot, which is filled again only after the
+  // stream has been synchronised: no upload waits. Readbacks land in pinned
+  // memory too; an iteration waits for its norms, for the factor's verdict
+  // together with H·X's finiteness, and for the Ritz values.
   void up_bytes(void* d, const void* h, size_t bytes) {
-    BD_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
-    sync();
+    if (slots_used == DavidsonWork::kSlots) sync();
+    char* slot = w.pinned + w.slot_bytes * slots_used++;
+    std::memcpy(slot, h, bytes);
+    BD_HIP(hipMemcpyAsync(d, slot, bytes, hipMemcpyHostToDevice, s));
   }
   void up(double* d, const double* h, size_t count) { up_bytes(d, h, count * 8); }
+  double* read_area(int which) {
+    return reinterpret_cast<double*>(w.pinned + w.slot_bytes * (DavidsonWork::kSlots + which));
+  }
+  int* read_flags() { return reinterpret_cast<int*>(w.pinned + w.slot_bytes * (DavidsonWork::kSlots + 2)); }
+  void read(int which, const double* d, size_t count) {
+    BD_HIP(hipMemcpyAsync(read_area(which), d, count * 8, hipMemcpyDeviceToHost, s));
+  }
+  void read_flag(int which, const int* d) {
+    BD_HIP(hipMemcpyAsync(read_flags() + which, d, sizeof(int), hipMemcpyDeviceToHost, s));
+  }
   void down(double* h, const double* d, size_t count) {
-    BD_HIP(hipMemcpyAsync(h, d, count * 8, hipMemcpyDeviceToHost, s));
+    read(0, d, count);
     sync();
+    std::memcpy(h, read_area(0), count * 8);
   }
 
   // H applied to k columns at src into dst, with the finiteness agreement of
-  // ref_davidson/workspace.rs:1013-1036.
-  void apply(const double* src, int k, double* dst) {
+  // ref_davidson/workspace.rs:1013-1036: queued, then looked at after a
+  // synchronisation.
+  void queue_apply(const double* src, int k, double* dst) {
     BD_HIP(hipEventRecord(ev0, s));
     op.apply(src, n, k, dst, n);
     BD_HIP(hipEventRecord(ev1, s));
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, w.flag);
     hipLaunchKernelGGL(k_finite, dim3(256), dim3(256), 0, s, dst, n * k, w.flag);
-    int bad = 0;
-    BD_HIP(hipMemcpyAsync(&bad, w.flag, sizeof(int), hipMemcpyDeviceToHost, s));
-    sync();
+    read_flag(0, w.flag);
+  }
+  void finish_apply(int k) {
     float ms = 0.f;
     BD_HIP(hipEventElapsedTime(&ms, ev0, ev1));
     t_apply += ms * 1e-3;
     rec.h_calls += 1;
     rec.h_columns += k;
-    if (bad) fail(BD_ERR_APPLICATION, "reference H application failed (non-finite output)");
+    if (read_flags()[0]) fail(BD_ERR_APPLICATION, "reference H application failed (non-finite output)");
+  }
+  void apply(const double* src, int k, double* dst) {
+    queue_apply(src, k, dst);
+    sync();
+    finish_apply(k);
   }
 
   // Border columns [from, to) of S (is_h false) or H_r, mirrored
@@ -356,14 +392,22 @@ struct Solver {
     mirror_border(s, M, cap, from, to);
   }
 
-  bool factor(int from, int to) {
-    auto t0 = std::chrono::steady_clock::now();
+  void queue_factor(int from, int to) {
+    BD_HIP(hipEventRecord(ev2, s));
     extend_inverse_cholesky_dev(s, w.S.p, w.T.p, cap, from, to, w.fw);
-    int verdict = 0;
-    BD_HIP(hipMemcpyAsync(&verdict, w.fw.flag, sizeof(int), hipMemcpyDeviceToHost, s));
+    BD_HIP(hipEventRecord(ev3, s));
+    read_flag(1, w.fw.flag);
+  }
+  bool finish_factor() {
+    float ms = 0.f;
+    BD_HIP(hipEventElapsedTime(&ms, ev2, ev3));
+    t_dense += ms * 1e-3;
+    return read_flags()[1] == 0;
+  }
+  bool factor(int from, int to) {
+    queue_factor(from, to);
     sync();
-    t_dense += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-    return verdict == 0;
+    return finish_factor();
   }
 
   // A = T H_r T^T, lowest nb eigenpairs, C = T^T Y (workspace.rs:435-499).
@@ -381,9 +425,11 @@ struct Solver {
       symmetrize(s, m, w.A.p, m);
       sym_eigen_lowest(s, m, nb, w.A.p, m, w.vals.p, w.Y.p, m, w.eigw.p, w.info, attempt == 0);
       gemm_nn(s, m, nb, m, 1.0, w.Tt.p, m, w.Y.p, m, 0.0, w.C.p, m);  // C
-      BD_HIP(hipMemcpyAsync(values.data(), w.vals.p, size_t(nb) * 8, hipMemcpyDeviceToHost, s));
-      BD_HIP(hipMemcpyAsync(&bad, w.info, sizeof(int), hipMemcpyDeviceToHost, s));
+      read(0, w.vals.p, size_t(nb));
+      read_flag(0, w.info);
       sync();
+      std::copy(read_area(0), read_area(0) + nb, values.begin());
+      bad = read_flags()[0];
       if (!bad) break;
       rec.eigen_retries += 1;
     }
@@ -475,8 +521,9 @@ struct Solver {
       mlp::correct(s, n, k, X, HX, w.theta.p, op.d_kinetic.p, diag, o.mlp_vbar, o.mlp_blob, w.E.p, w.norm2.p,
                    w.rnorm2.p, w.mlpw.p);
       std::vector<double> rn(k);
-      BD_HIP(hipMemcpyAsync(rn.data(), w.rnorm2.p, size_t(k) * 8, hipMemcpyDeviceToHost, s));
+      read(1, w.rnorm2.p, size_t(k));
       down(nrm.data(), w.norm2.p, k);
+      std::copy(read_area(1), read_area(1) + k, rn.begin());
       bool finite = true;
       for (double v : nrm) finite = finite && std::isfinite(v);
       if (!finite || mlp_regressed(active, rn)) {
@@ -615,18 +662,28 @@ struct Solver {
         staged = m + kk <= cap && kk > 0;
         k = normalize(nrm, staged ? V + int64_t(m) * n : w.E2.p);
       }
+      bool applied = false;
       if (!staged || k == 0) {
         k = k > 0 ? repair(m, k) : 0;
       } else {
+        // H·X of the new columns is queued behind the factor, whose verdict is
+        // looked at with it (a rejected border, which is rare, drops the
+        // product).
         border(m, m + k, false);
-        if (!factor(m, m + k)) {
+        queue_factor(m, m + k);
+        queue_apply(V + int64_t(m) * n, k, HV + int64_t(m) * n);
+        sync();
+        applied = finish_factor();
+        if (applied) {
+          finish_apply(k);
+        } else {
           BD_HIP(hipMemcpyAsync(w.E2.p, V + int64_t(m) * n, size_t(n) * k * 8, hipMemcpyDeviceToDevice, s));
           k = repair(m, k);
         }
       }
       std::copy(values.begin(), values.begin() + nb, old.begin());
       if (k > 0) {
-        apply(V + int64_t(m) * n, k, HV + int64_t(m) * n);
+        if (!applied) apply(V + int64_t(m) * n, k, HV + int64_t(m) * n);
         border(m, m + k, true);
         eigen(m + k);
         m += k;
