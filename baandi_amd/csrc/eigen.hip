@@ -1925,11 +1925,9 @@ __device__ double lu_solve_prefetch(int m, int want, int j, const LU& f, double*
   return nn;
 }
 
-// The per-vector work of inverse iteration: LU of (T - lambda' I) into g
-// (entries at i * stride + lane), a hashed start, two solves, unit norm.
-// Column j of the caller's output numbering seeds the start vector.
-__device__ void invit_vector(int m, int stride, int lane, int j, const double* ds, const double* es, double lam,
-                             double tiny, const LU& g, double* z) {
+// LU of (T - lambda' I) into g (entries at i * stride + lane).
+__device__ void invit_factor(int m, int stride, int lane, const double* ds, const double* es, double lam, double tiny,
+                             const LU& g) {
   auto at = [&](int i) { return int64_t(i) * stride + lane; };
   double a = ds[0] - lam, b = es[0];
   for (int i = 0; i + 1 < m; ++i) {
@@ -1968,9 +1966,17 @@ __device__ void invit_vector(int m, int stride, int lane, int j, const double* d
   g.U2[at(m - 1)] = 0.0;
   g.Lm[at(m - 1)] = 0.0;
   g.piv[at(m - 1)] = 0;
+}
+
+// The per-vector work of inverse iteration: the factors, a hashed start, two
+// solves (the second from the unscaled first: growth per solve is at most
+// ~1/(eps ||T||), far from overflow), then unit norm. Column j of the caller's
+// output numbering seeds the start vector.
+__device__ void invit_vector(int m, int stride, int lane, int j, const double* ds, const double* es, double lam,
+                             double tiny, const LU& g, double* z) {
+  auto at = [&](int i) { return int64_t(i) * stride + lane; };
+  invit_factor(m, stride, lane, ds, es, lam, tiny, g);
   for (int i = 0; i < m; ++i) z[at(i)] = hash_unit(i, j, 0);
-  // Two solves (the second from the unscaled first: growth per solve is at
-  // most ~1/(eps ||T||), far from overflow), then unit norm.
   lu_solve_prefetch(m, stride, lane, g, z);
   const double nn = lu_solve_prefetch(m, stride, lane, g, z);
   const double sc = nn > 0.0 ? 1.0 / sqrt(nn) : 0.0;
@@ -2010,16 +2016,17 @@ __global__ __launch_bounds__(64) void k_invit(int m, int want, const double* __r
 // LDS (a dependent chain of LDS accesses instead of L2 round trips), copied
 // to the global layout at the end (the cluster re-iteration reads them there).
 // 8 vectors per workgroup up to m = 476, 4 from there to m = 910.
+// A lane per vector runs the serial chains; the other lanes of the wave share
+// the loads, the start vectors, the scaling and the copies: 139 us at m = 320,
+// 160 vectors, 171 with a vector's lane doing all of its own.
 template <int kInvLds>
-__global__ __launch_bounds__(kInvLds) void k_invit_lds(int m, int want, const double* __restrict__ d,
-                                                       const double* __restrict__ e,
-                                                       const double* __restrict__ values,
-                                                       const double* __restrict__ tnorm_in, LU f,
-                                                       double* __restrict__ Z) {
+__global__ __launch_bounds__(64) void k_invit_lds(int m, int want, const double* __restrict__ d,
+                                                  const double* __restrict__ e, const double* __restrict__ values,
+                                                  const double* __restrict__ tnorm_in, LU f, double* __restrict__ Z) {
   extern __shared__ double sh[];
   double* ds = sh;
   double* es = sh + m;
-  const int64_t mv = int64_t(m) * kInvLds;
+  const int mv = m * kInvLds;
   LU g;
   g.U0i = sh + 2 * m;
   g.U1 = g.U0i + mv;
@@ -2027,24 +2034,35 @@ __global__ __launch_bounds__(kInvLds) void k_invit_lds(int m, int want, const do
   g.Lm = g.U2 + mv;
   double* z = g.Lm + mv;
   g.piv = reinterpret_cast<unsigned char*>(z + mv);
-  for (int i = threadIdx.x; i < m; i += blockDim.x) {
+  const int lane = threadIdx.x, j0 = blockIdx.x * kInvLds, j = j0 + lane;
+  const bool mine = lane < kInvLds && j < want;
+  for (int i = lane; i < m; i += 64) {
     ds[i] = d[i];
     es[i] = i + 1 < m ? e[i] : 0.0;
   }
+  for (int i = lane; i < min(want, j0 + kInvLds); i += 64) z[i] = values[i];  // (want <= m)
   __syncthreads();
-  const int lane = threadIdx.x;
-  const int j = blockIdx.x * kInvLds + lane;
-  if (j >= want) return;
   const double tiny = DBL_EPSILON * fmax(tnorm_in[0], DBL_MIN);
-  invit_vector(m, kInvLds, lane, j, ds, es, invit_shift(values, j, tnorm_in[0]), tiny, g, z);
-  for (int i = 0; i < m; ++i) {
-    const int64_t src = int64_t(i) * kInvLds + lane, dst = int64_t(i) * want + j;
-    Z[dst] = z[src];
-    f.U0i[dst] = g.U0i[src];
-    f.U1[dst] = g.U1[src];
-    f.U2[dst] = g.U2[src];
-    f.Lm[dst] = g.Lm[src];
-    f.piv[dst] = g.piv[src];
+  if (mine) invit_factor(m, kInvLds, lane, ds, es, invit_shift(z, j, tnorm_in[0]), tiny, g);
+  __syncthreads();
+  for (int t = lane; t < mv; t += 64) z[t] = hash_unit(t / kInvLds, j0 + t % kInvLds, 0);
+  __syncthreads();
+  if (mine) {
+    lu_solve_prefetch(m, kInvLds, lane, g, z);
+    const double nn = lu_solve_prefetch(m, kInvLds, lane, g, z);
+    ds[lane] = nn > 0.0 ? 1.0 / sqrt(nn) : 0.0;  // (d is done with)
+  }
+  __syncthreads();
+  for (int t = lane; t < mv; t += 64) {
+    const int l = t % kInvLds;
+    if (j0 + l >= want) continue;
+    const int64_t dst = int64_t(t / kInvLds) * want + j0 + l;
+    Z[dst] = z[t] * ds[l];
+    f.U0i[dst] = g.U0i[t];
+    f.U1[dst] = g.U1[t];
+    f.U2[dst] = g.U2[t];
+    f.Lm[dst] = g.Lm[t];
+    f.piv[dst] = g.piv[t];
   }
 }
 
@@ -2494,11 +2512,11 @@ void tridiag_vectors(hipStream_t s, int m, int want, const EigenLayout& L, doubl
   auto invit_lds = [m](int v) { return size_t(2 * m + 5 * int64_t(m) * v) * 8 + size_t(m) * v; };
   if (invit_lds(8) <= 160 * 1024) {
     if (invit_lds(8) > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_invit_lds<8>), "k_invit_lds<8>");
-    hipLaunchKernelGGL((k_invit_lds<8>), dim3((want + 7) / 8), dim3(8), invit_lds(8), s, m, want, L.d, L.e, values,
+    hipLaunchKernelGGL((k_invit_lds<8>), dim3((want + 7) / 8), dim3(64), invit_lds(8), s, m, want, L.d, L.e, values,
                        L.tnorm, L.f, L.Z);
   } else if (invit_lds(4) <= 160 * 1024) {
     allow_full_lds(reinterpret_cast<const void*>(&k_invit_lds<4>), "k_invit_lds<4>");
-    hipLaunchKernelGGL((k_invit_lds<4>), dim3((want + 3) / 4), dim3(4), invit_lds(4), s, m, want, L.d, L.e, values,
+    hipLaunchKernelGGL((k_invit_lds<4>), dim3((want + 3) / 4), dim3(64), invit_lds(4), s, m, want, L.d, L.e, values,
                        L.tnorm, L.f, L.Z);
   } else {
     hipLaunchKernelGGL(k_invit, dim3((want + 63) / 64), dim3(64), size_t(2 * m) * 8, s, m, want, L.d, L.e, values,
