@@ -558,7 +558,7 @@ static void order_sticks(StickPlan& p, std::vector<std::pair<int, int>>& sticks)
   p.lines = std::move(lines);
 }
 
-StickPlan build_stick_plan(const System& s) {
+StickPlan build_stick_plan(const System& s, bool paired) {
   StickPlan p{};
   p.n0 = s.dims[0];
   p.n1 = s.dims[1];
@@ -599,7 +599,7 @@ StickPlan build_stick_plan(const System& s) {
   while (p.T > 1 && !fft_fits(p.T, p.rx)) p.T /= 2;
   if (!fft_fits(p.T, p.rx)) fail(BD_ERR_INVALID_PARAMETER, "x FFT does not fit a workgroup");
   // The paired x pass where it is built for the length (it reads rows in twos).
-  if (s.nrep > 1) p.xshape = stick_shape(p.n0);
+  if (paired && s.nrep > 1) p.xshape = stick_shape(p.n0);
   if (p.xshape.on) p.T = p.xshape.tile;
   p.chunk = 16;
   while (p.chunk > 1 && !fft_fits(p.chunk, p.rz)) p.chunk /= 2;
@@ -919,7 +919,35 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
     d_work.alloc(size_t(Gemm::tn_work(nproj, cap, n)));
   }
   const int pairs = slots(cap);
-  d_sticks.alloc(size_t(pairs) * plan.n0 * plan.Spad);
+  int spad = plan.Spad;
+  if (!kb && precision == BD_FP32_HX && (plan.xshape.on || pair.on)) {
+    dplan = build_stick_plan(s, false);
+    // (Planes beyond one workgroup's passes take the paired pass.)
+    plain_density = fft_fits(dplan.Z, dplan.ry) && plane_lds(dplan, elem) <= lds_max;
+  }
+  if (plain_density) {
+    // Large planes: 512 threads and the longest row chunk, as the shape search
+    // picks there (the bits do not depend on the shape).
+    if (dplan.n1 * dplan.n2 >= 64 * 64 && fft_fits_threads(dplan.Z, dplan.ry, 512))
+      for (int c = dplan.n1; c > dplan.chunk; --c) {
+        StickPlan wide = dplan;
+        wide.chunk = c;
+        if (!fft_fits_threads(c, dplan.rz, 512) || plane_lds(wide, elem) > 80 * 1024) continue;
+        dplan.chunk = c;
+        plain_threads = 512;
+        break;
+      }
+    spad = std::max(spad, dplan.Spad);
+    d_dtile_off.alloc(dplan.tile_off.size());
+    d_dtile_off.upload(dplan.tile_off.data(), dplan.tile_off.size(), stream);
+    d_dentries.alloc(dplan.entries.size());
+    d_dentries.upload(dplan.entries.data(), dplan.entries.size(), stream);
+    d_ddst.alloc(dplan.stick_dst.size());
+    d_ddst.upload(dplan.stick_dst.data(), dplan.stick_dst.size(), stream);
+    d_dyz.alloc(dplan.stick_yz.size());
+    d_dyz.upload(dplan.stick_yz.data(), dplan.stick_yz.size(), stream);
+  }
+  d_sticks.alloc(size_t(pairs) * plan.n0 * spad);
   if (paired() && pair.split > 1) d_sticks2.alloc(size_t(pairs) * plan.n0 * plan.Spad);
   // Planes that do not fit one workgroup go through the split pass.
   if (!fft_fits(plan.Z, plan.ry) || plane_lds(plan, elem) > lds_max) enable_split(0);
@@ -1129,15 +1157,25 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
   const int pairs = slots(m);
   const size_t e = sizeof(c2<F>);
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
-  columns_to_sticks<F>(x, ldx, m);
   const int groups = std::min(pairs, kDensityGroups);
+  if (plain_density)
+    hipLaunchKernelGGL(k_stick_inverse<F>, dim3(dplan.ntiles, pairs), dim3(kThreads), stick_lds(dplan, e), stream, x,
+                       ldx, m, dplan.n0, dplan.T, dplan.Spad, d_dtile_off.p, d_dentries.p, d_ddst.p, d_roots.p,
+                       dplan.rx, sticks);
+  else
+    columns_to_sticks<F>(x, ldx, m);
   // Warm start: keep the pairs' real-space fields (Gamma, fused plane pass).
   c2<F>* keep = kept_on ? reinterpret_cast<c2<F>*>(d_kept.p) : nullptr;
   kept_valid = keep != nullptr;
   kept_x = x;
   kept_ldx = ldx;
   kept_m = m;
-  if (pair.on) {
+  if (plain_density) {
+    const auto plane = plain_threads == 512 ? &k_plane<1, F, 512> : &k_plane<1, F, 256>;
+    hipLaunchKernelGGL(plane, dim3(dplan.n0, groups), dim3(plain_threads), plane_lds(dplan, e), stream, sticks, dplan.n0,
+                       dplan.n1, dplan.n2, dplan.Spad, dplan.Z, dplan.chunk, d_dyz.p, d_zc.p, d_roots.p, dplan.ry,
+                       dplan.rz, nullptr, pairs, w, 1.0 / sys->volume, d_rho_part.p, keep);
+  } else if (pair.on) {
     PairArgs<F> a = pair_args<F>(pairs);
     a.kept_out = keep;
     a.weights = w;

@@ -138,6 +138,15 @@ struct GammaOp {
   DevBuf<PlaneLine> d_lines;
   PairShape pair;  // the paired plane pass (plane.hpp), where it applies
   DevBuf<c2<double>> d_sticks2;  // its output sticks where planes go by row parity
+  // BD_FP32_HX at Gamma: the band density stays on the radix passes, whose FP32
+  // rounding it keeps (a density is a sum of squares and shows the transforms'
+  // rounding in full, ~1e-7; H·X shows ~1e-8 of it).
+  bool plain_density = false;
+  int plain_threads = 256;
+  StickPlan dplan;
+  DevBuf<int> d_dtile_off, d_ddst;
+  DevBuf<int4> d_dentries;
+  DevBuf<int2> d_dyz;
   DevBuf<c2<double>> d_roots;  // [n0 | n1 | n2]
   DevBuf<double> d_kinetic, d_potential, d_proj, d_blockd;
   DevBuf<float> d_potential32;  // mixed tier: V(r) in float
@@ -224,7 +233,7 @@ void fused_launch(const GammaOp& op, const FusedShape& f, size_t lds, const KWor
                   int count, int total, hipStream_t s);
 bool fft_fits_threads(int nlines, const RadixPlan& rp, int threads);
 
-StickPlan build_stick_plan(const System& s);
+StickPlan build_stick_plan(const System& s, bool paired = true);
 StickPlan build_k_stick_plan(const System& s, const KBasis& kb, int nproj, size_t elem);
 RadixPlan radix_plan(int n, bool big);
 
