@@ -29,6 +29,7 @@
 #include <string>
 
 #include "common.hpp"
+#include "coop_exchange.hpp"
 #include "eigen.hpp"
 #include "gemm.hpp"
 #include "wave.hpp"
@@ -796,8 +797,9 @@ __global__ __launch_bounds__(256) void k_td_update(int m, double* __restrict__ A
 // words at agent scope): a reader polls the words until both carry the tag,
 // with no separate flag and no cache flush. Parts and columns alternate
 // between two slots by the parity of k (a worker reaches step k + 2 only
-// after every worker has read step k), and the slots are cleared before the
-// launch, so a tag is never stale. The workers are blocks 0 .. nw-1, spread
+// after every worker has read step k: each publishes in every step,
+// coop_exchanged), and the slots are cleared before the launch, so a tag is
+// never stale. The workers are blocks 0 .. nw-1, spread
 // over the XCDs by the round-robin dispatch. Every wait is bounded: a worker
 // that polls a word more than `spins` times (at once when spins < 0), or
 // sees another worker's abort, sets *info = -1 and every worker leaves (the
@@ -947,6 +949,8 @@ __global__ __launch_bounds__(kCT) void k_td_coop(int m, int nw, double* __restri
         if (has2) ll_put(yb + 2 * (me + (lc + 2 * NWV) * nw), a2, tag);
       }
     }
+    // (No column left: the word of the last one says that this worker is here.)
+    if (lc0 >= ncl && tid == 0) ll_put(yb + 2 * (me + (ncl - 1) * nw), 0.0, tag);
     if ((k + 2) % nw == me) {
       const double* col = Al + int64_t((k + 2 - me) / nw) * m;
       for (int r = k + 1 + tid; r < m; r += kCT) ll_put(cb + 2 * r, col[r], tag);
@@ -987,6 +991,9 @@ __global__ __launch_bounds__(kCT) void k_td_coop(int m, int nw, double* __restri
           s += yw[i] * vv[i];
         }
       }
+      double behind;
+      for (int r = m - nw + tid; ok && r <= k; r += kCT)
+        if (coop_exchanged(m, nw, k, r)) ok = ll_get(yb + 2 * r, tag, &behind, spins, info);
     }
     if (!ok) go = 0;
     s = coop_sum(s, red);
@@ -1157,7 +1164,8 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, int steps, d
         if (lane + 64 * t < m) Al[int64_t(k / nw) * m + lane + 64 * t] = v[t];
     }
   };
-  // y_j = A[:, j].v of the own columns j > k, published by one lane each.
+  // y_j = A[:, j].v of the own columns j > k, published by one lane each (and
+  // a word for a last column behind k, coop_exchanged).
   auto products = [&](int k, uint64_t* yb) {
     double s[C];
 #pragma unroll
@@ -1172,7 +1180,7 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, int steps, d
 #pragma unroll
     for (int ci = 1; ci < C; ++ci) mine = lane == ci ? s[ci] : mine;
     const int j = me + (wave + NWV * lane) * nw;
-    if (lane < C && j > k && j < m) ll_put(yb + 2 * j, mine, uint32_t(k + 1));
+    if (lane < C && j < m && coop_exchanged(m, nw, k, j)) ll_put(yb + 2 * j, mine, uint32_t(k + 1));
   };
   reflector(0, c2);
   int k = 0;
@@ -1238,6 +1246,9 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, int steps, d
         if (tries > spins) ok = false;
         if ((tries & 63) == 63 && __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) ok = false;
       }
+      double behind;
+      for (int r = m - nw + tid; ok && r <= k; r += kCT)
+        if (coop_exchanged(m, nw, k, r)) ok = ll_get(yb + 2 * r, tag, &behind, spins, info);
     }
     if (!ok) go[k & 1] = 0;
     __syncthreads();
@@ -2385,6 +2396,7 @@ std::atomic<int> coop_spins{1 << 21};
 int coop_worker_count(int m) {
   int w = coop_workers.load();
   if (w < 0) w = std::min(32, std::max(8, m / 10));
+  w = std::min(w, m);  // (a column each)
   if (w == 0 || m < 3 || m < coop_from.load() || m > coop_to.load() || m > kCoopRd * kCT) return 0;
   for (int nw = w; nw <= 32; ++nw)
     if (coop_lds(m, nw) <= 160 * 1024) return nw;
