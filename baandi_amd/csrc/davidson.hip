@@ -302,6 +302,7 @@ struct Solver {
 
   Solver(GammaOp& op_, DavidsonWork& w_, const bd_davidson_options& o_, const double* diag_)
       : op(op_), w(w_), s(op_.stream), n(w_.n), nb(w_.nb), cap(w_.cap), o(o_), diag(diag_) {
+    w.fw.gemm.sums = op.gemm.sums;
     V = w.V.p;
     HV = w.HV.p;
     X = w.X.p;
@@ -420,11 +421,12 @@ struct Solver {
     int bad = 0;
     for (int attempt = 0; attempt < 2; ++attempt) {
       transpose(s, m, m, w.T.p, cap, w.Tt.p, m);
-      gemm_nn(s, m, m, m, 1.0, w.H.p, cap, w.Tt.p, m, 0.0, w.small3.p, m);  // H_r T^T
-      gemm_nn(s, m, m, m, 1.0, w.T.p, cap, w.small3.p, m, 0.0, w.A.p, m);   // A
+      op.gemm.nn64(s, m, m, m, 1.0, w.H.p, cap, w.Tt.p, m, 0.0, w.small3.p, m);  // H_r T^T
+      op.gemm.nn64(s, m, m, m, 1.0, w.T.p, cap, w.small3.p, m, 0.0, w.A.p, m);   // A
       symmetrize(s, m, w.A.p, m);
-      sym_eigen_lowest(s, m, nb, w.A.p, m, w.vals.p, w.Y.p, m, w.eigw.p, w.info, attempt == 0);
-      gemm_nn(s, m, nb, m, 1.0, w.Tt.p, m, w.Y.p, m, 0.0, w.C.p, m);  // C
+      sym_eigen_lowest(s, m, nb, w.A.p, m, w.vals.p, w.Y.p, m, w.eigw.p, w.info, attempt == 0,
+                       op.gemm.sums);
+      op.gemm.nn64(s, m, nb, m, 1.0, w.Tt.p, m, w.Y.p, m, 0.0, w.C.p, m);  // C
       read(0, w.vals.p, size_t(nb));
       read_flag(0, w.info);
       sync();
@@ -586,8 +588,8 @@ struct Solver {
   int repair(int m, int k) {
     rec.repairs += 1;
     // Coordinates of the Ritz block in the whitened basis: C <- T S C.
-    gemm_nn(s, m, nb, m, 1.0, w.S.p, cap, w.C.p, m, 0.0, w.small2.p, m);
-    gemm_nn(s, m, nb, m, 1.0, w.T.p, cap, w.small2.p, m, 0.0, w.C.p, m);
+    op.gemm.nn64(s, m, nb, m, 1.0, w.S.p, cap, w.C.p, m, 0.0, w.small2.p, m);
+    op.gemm.nn64(s, m, nb, m, 1.0, w.T.p, cap, w.small2.p, m, 0.0, w.C.p, m);
     transpose(s, m, m, w.T.p, cap, w.small1.p, m);  // T^T
     op.gemm.nn(s, n, m, m, 1.0, V, n, w.small1.p, m, 0.0, X, n);
     op.gemm.nn(s, n, m, m, 1.0, HV, n, w.small1.p, m, 0.0, HX, n);
@@ -603,10 +605,10 @@ struct Solver {
     for (int j = 0; j < k; ++j) {
       double* ej = E + int64_t(j) * n;
       for (int pass = 0; pass < 2 && kept > 0; ++pass) {
-        gemm_tn(s, kept, 1, n, 1.0, E, n, ej, n, 0.0, w.small1.p, kept, w.gwork.p);
-        gemm_nn(s, n, 1, kept, -1.0, E, n, w.small1.p, kept, 1.0, ej, n);
+        op.gemm.tn64(s, kept, 1, n, 1.0, E, n, ej, n, 0.0, w.small1.p, kept, w.gwork.p);
+        op.gemm.nn64(s, n, 1, kept, -1.0, E, n, w.small1.p, kept, 1.0, ej, n);
       }
-      gemm_tn(s, 1, 1, n, 1.0, ej, n, ej, n, 0.0, w.small1.p, 1, w.gwork.p);
+      op.gemm.tn64(s, 1, 1, n, 1.0, ej, n, ej, n, 0.0, w.small1.p, 1, w.gwork.p);
       double nn2 = 0.0;
       down(&nn2, w.small1.p, 1);
       const double nrm = std::sqrt(nn2);
@@ -1423,7 +1425,7 @@ struct BlockGraph {
     hipStream_t s = op.stream;
     op.gemm.tn(s, nb, nb, n, 1.0, src, n, src, n, 0.0, G.p, nb, gwork.p);
     symmetrize(s, nb, G.p, nb);
-    sym_eigen_lowest(s, nb, nb, G.p, nb, lam.p, U.p, nb, eigw.p, info + 1);
+    sym_eigen_lowest(s, nb, nb, G.p, nb, lam.p, U.p, nb, eigw.p, info + 1, true, op.gemm.sums);
     hipLaunchKernelGGL(k_canon, dim3(1, nb), dim3(64), 0, s, U.p, lam.p, nb, Tc.p, dropped);
     op.gemm.nn(s, n, nb, nb, 1.0, src, n, Tc.p, nb, 0.0, dst, n);
   }
@@ -1435,7 +1437,7 @@ struct BlockGraph {
     symmetrize(s, m, A.p, m);
     hipLaunchKernelGGL(k_lift_dropped, dim3(unsigned((nb + 255) / 256)), dim3(256), 0, s, A.p, int64_t(m), m - nb,
                        dropped, nb, 1e6);
-    sym_eigen_lowest(s, m, nb, A.p, m, theta.p, Y.p, m, eigw.p, info);
+    sym_eigen_lowest(s, m, nb, A.p, m, theta.p, Y.p, m, eigw.p, info, true, op.gemm.sums);
     op.gemm.nn(s, n, nb, m, 1.0, V.p, n, Y.p, m, 0.0, X.p, n);
     op.gemm.nn(s, n, nb, m, 1.0, HV.p, n, Y.p, m, 0.0, HX.p, n);
   }

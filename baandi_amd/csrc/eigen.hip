@@ -1835,6 +1835,75 @@ __global__ __launch_bounds__(256) void k_bisect(int m, int want, const double* _
   }
 }
 
+// Sums::chain: the counts by the ratios q_i = p_i / p_{i-1}, a division a row on
+// the chain.
+__device__ __forceinline__ int sturm_ratios(int m, const double* ds, const double* e2, double x, double pivmin) {
+  double q = ds[0] - x;
+  if (fabs(q) <= pivmin) q = -pivmin;
+  int c = q < 0.0 ? 1 : 0;
+  for (int i = 1; i < m; ++i) {
+    q = ds[i] - x - e2[i - 1] / q;
+    if (fabs(q) <= pivmin) q = -pivmin;
+    c += q < 0.0 ? 1 : 0;
+  }
+  return c;
+}
+
+__global__ __launch_bounds__(256) void k_bisect_ratios(int m, int want, const double* __restrict__ d,
+                                                       const double* __restrict__ e, double* __restrict__ values,
+                                                       double* __restrict__ tnorm_out) {
+  extern __shared__ double sh[];
+  double* ds = sh;
+  double* e2 = sh + m;
+  double* ea = sh + 2 * m;
+  for (int i = threadIdx.x; i < m; i += blockDim.x) {
+    ds[i] = d[i];
+    const double v = i + 1 < m ? e[i] : 0.0;
+    e2[i] = v * v;
+    ea[i] = fabs(v);
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int j = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (j >= want) return;  // whole waves leave together; no barrier follows
+  double gl = INFINITY, gu = -INFINITY, emax2 = 0.0;
+  for (int i = lane; i < m; i += 64) {
+    const double r = (i > 0 ? ea[i - 1] : 0.0) + ea[i];
+    gl = fmin(gl, ds[i] - r);
+    gu = fmax(gu, ds[i] + r);
+    emax2 = fmax(emax2, e2[i]);
+  }
+  gl = wave_min(gl);
+  gu = wave_max(gu);
+  emax2 = wave_max(emax2);
+  const double tnorm = fmax(fabs(gl), fabs(gu));
+  const double pivmin = DBL_MIN * fmax(1.0, emax2);
+  const double pad = 2.1 * tnorm * DBL_EPSILON * m + 4.2 * pivmin;
+  double lo = gl - pad, hi = gu + pad;
+  // Invariant: count(lo) <= j < count(hi). 64 points per step shrink the
+  // bracket 65x; the cap bounds the loop.
+  for (int it = 0; it < 48; ++it) {
+    const double width = hi - lo;
+    if (width <= 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + pivmin) break;
+    const double xl = lo + width * (double(lane + 1) / 65.0);
+    const int c = sturm_ratios(m, ds, e2, xl, pivmin);
+    const unsigned long long above = __ballot(c >= j + 1);
+    if (above == 0ull) {
+      lo = __shfl(xl, 63, 64);
+    } else {
+      const int f = __ffsll(static_cast<long long>(above)) - 1;
+      const double nhi = __shfl(xl, f, 64);
+      const double nlo = __shfl(xl, f > 0 ? f - 1 : 0, 64);
+      hi = nhi;
+      if (f > 0) lo = nlo;
+    }
+  }
+  if (lane == 0) {
+    values[j] = 0.5 * (lo + hi);
+    if (j == 0) tnorm_out[0] = tnorm;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // 3. Inverse iteration. Per eigenvector j the LU of (T - lambda_j I) with
 // partial pivoting: U has the reciprocal diagonal U0i and two superdiagonals
@@ -2450,10 +2519,10 @@ void tridiag_multi(hipStream_t s, int m, double* A, int64_t lda, const EigenLayo
 }
 
 void tridiag_vectors(hipStream_t s, int m, int want, const EigenLayout& L, double* values, double* Ysc, int64_t ldy,
-                     int* info);
+                     int* info, Sums sums);
 
 void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, double* values, double* Y,
-                      int64_t ldy, double* work, int* info, bool blocked) {
+                      int64_t ldy, double* work, int* info, bool blocked, Sums sums) {
   if (m <= 0 || want <= 0 || want > m || lda < m || ldy < m || lda * m >= (int64_t(1) << 31))
     fail(BD_ERR_INVALID_PARAMETER, "sym_eigen_lowest: shape");
   auto bt_lds = [m](int ch) { return size_t((4 + ch) * m + ch) * 8; };
@@ -2463,13 +2532,14 @@ void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, do
   const EigenLayout L = eigen_layout(m, want, work);
   hipLaunchKernelGGL(k_zero_i, dim3(1), dim3(64), 0, s, info, 1);
   const size_t panel_lds = tridiag_panel_lds(m);
-  const bool automatic = blocked && coop_workers.load() < 0;
+  const bool chain = sums == Sums::chain;
+  const bool automatic = blocked && !chain && coop_workers.load() < 0;
   const int nw = blocked && !(automatic && m <= kOneMax) ? coop_worker_count(m) : 0;
   if (m >= 3 && m >= multi_from.load()) {
     tridiag_multi(s, m, A, lda, L, L.td);
   } else if (nw > 0) {
     zero_doubles(s, reinterpret_cast<double*>(L.words), coop_words(m));
-    if (const CoopReg reg = coop_reg_kernel(m, nw)) {
+    if (const CoopReg reg = chain ? nullptr : coop_reg_kernel(m, nw)) {
       // The last kOneMax rows in one workgroup, where a step costs less than
       // the exchange between several (2.7 us).
       const int steps = automatic ? m - kOneMax : m - 2;
@@ -2492,7 +2562,7 @@ void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, do
   } else {
     tridiag_unblocked(s, m, A, lda, L);
   }
-  tridiag_vectors(s, m, want, L, values, Y, ldy, info);
+  tridiag_vectors(s, m, want, L, values, Y, ldy, info, sums);
   if (m <= 320) {
     hipLaunchKernelGGL(k_back_transform_reg<5>, dim3((want + 3) / 4), dim3(256), bt_reg_lds(m), s, m, want, A, lda,
                        L.tau, L.Ytmp, int64_t(m));
@@ -2517,10 +2587,14 @@ void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, do
 // orthonormal eigenvectors in L.Ytmp (m x want, ld m); Ysc (m x want, ld
 // ldy) is scratch for the cluster Gram-Schmidt output.
 void tridiag_vectors(hipStream_t s, int m, int want, const EigenLayout& L, double* values, double* Ysc, int64_t ldy,
-                     int* info) {
+                     int* info, Sums sums) {
   double* Y = Ysc;
-  hipLaunchKernelGGL(k_bisect, dim3((want + 3) / 4), dim3(256), bisect_lds(m), s, m, want, L.d, L.e, values,
-                     L.tnorm);
+  if (sums == Sums::chain)
+    hipLaunchKernelGGL(k_bisect_ratios, dim3((want + 3) / 4), dim3(256), size_t(3 * m) * 8, s, m, want, L.d, L.e,
+                       values, L.tnorm);
+  else
+    hipLaunchKernelGGL(k_bisect, dim3((want + 3) / 4), dim3(256), bisect_lds(m), s, m, want, L.d, L.e, values,
+                       L.tnorm);
   auto invit_lds = [m](int v) { return size_t(2 * m + 5 * int64_t(m) * v) * 8 + size_t(m) * v; };
   if (invit_lds(8) <= 160 * 1024) {
     if (invit_lds(8) > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_invit_lds<8>), "k_invit_lds<8>");
@@ -2537,9 +2611,9 @@ void tridiag_vectors(hipStream_t s, int m, int want, const EigenLayout& L, doubl
   hipLaunchKernelGGL(k_cluster_gs, dim3((want + 3) / 4), dim3(256), 0, s, m, want, values, L.tnorm, L.f, L.Z, Y, ldy,
                      info);
   // Loewdin step: Y <- Y (3 I - Y^T Y) / 2.
-  gemm_tn(s, want, want, m, 1.0, Y, ldy, Y, ldy, 0.0, L.G, want, L.gwork);
+  gemm_tn(s, want, want, m, 1.0, Y, ldy, Y, ldy, 0.0, L.G, want, L.gwork, sums);
   hipLaunchKernelGGL(k_loewdin_factor, dim3((want + 255) / 256, want), dim3(256), 0, s, want, L.G);
-  gemm_nn(s, m, want, want, 1.0, Y, ldy, L.G, want, 0.0, L.Ytmp, m);
+  gemm_nn(s, m, want, want, 1.0, Y, ldy, L.G, want, 0.0, L.Ytmp, m, sums);
 }
 
 // Lowest `want` eigenpairs of the complex Hermitian A (m x m, both triangles,
@@ -2565,7 +2639,7 @@ void herm_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, d
   if (zt_lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_zhe_tridiag), "k_zhe_tridiag");
   hipLaunchKernelGGL(k_zhe_tridiag, dim3(1), dim3(kZT), zt_lds, s, m, Ac, lda, L.d, L.e, tc);
   // The real stage's scratch is Y itself (m x want doubles fit its 2 ldy x want).
-  tridiag_vectors(s, m, want, L, values, Y, int64_t(m), info);
+  tridiag_vectors(s, m, want, L, values, Y, int64_t(m), info, Sums::fast);
   if (zb_lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(&k_zback_transform), "k_zback_transform");
   hipLaunchKernelGGL(k_zback_transform, dim3((want + 3) / 4), dim3(256), zb_lds, s, m, want, Ac, lda, tc, L.Ytmp,
                      int64_t(m), reinterpret_cast<double2*>(Y), ldy);

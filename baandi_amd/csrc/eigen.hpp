@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "gemm.hpp"
+
 namespace bd {
 
 // Lets launches of kernel `fn` ask for up to the whole 160 KB of LDS (set once
@@ -20,9 +22,11 @@ int64_t sym_eigen_work(int m, int want);
 // (device, `want`) ascending; Y (m x want, ldy) orthonormal eigenvectors.
 // *info (device) is set to 0, or to 1 + j when vector j could not be made
 // orthogonal to its cluster. `blocked` selects the panel tridiagonalisation
-// where it fits (else the one-step kernel).
+// where it fits (else the one-step kernel). Sums::chain keeps, beside its
+// products, the tridiagonalisations whose sums run over a workgroup's threads
+// and the Sturm counts by ratios (GammaOp::keeps_rounding).
 void sym_eigen_lowest(hipStream_t s, int m, int want, double* A, int64_t lda, double* values, double* Y,
-                      int64_t ldy, double* work, int* info, bool blocked = true);
+                      int64_t ldy, double* work, int* info, bool blocked = true, Sums sums = Sums::fast);
 // The same for a complex Hermitian A (both triangles, interleaved (re, im),
 // ld lda complex entries): Y complex m x want (ld ldy complex entries); the
 // same workspace size.
@@ -41,6 +45,7 @@ struct FactorWork {
   // complex factor, whose extension checks only the pivots and finiteness
   // (crates/dft-numerics/src/linalg.rs:277-340).
   int growth_guard = 1;
+  Gemm gemm;  // its FP64 products
 };
 
 // Extend T = L^{-1} of S (both cap x cap, ld cap, lower triangular T with a

@@ -19,9 +19,9 @@ struct c2 {
   T x, y;
 };
 
-// The transforms' arithmetic is written out with its fused multiply-adds, and
-// the compiler adds none of its own (fp contract(off)): the same line has the
-// same bits in every kernel that transforms it.
+// The paired passes' arithmetic is written out with its fused multiply-adds,
+// and the compiler adds none of its own (fp contract(off)): the same line has
+// the same bits in every one of their kernels.
 template <typename T>
 __host__ __device__ __forceinline__ T fma_of(T a, T b, T c) {
   if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
@@ -239,8 +239,10 @@ __host__ __device__ __forceinline__ void dft(c2<T>* v) {
 }
 
 // The same transforms of 2, 3, 4, 5, 8 and 9 points with the products and sums
-// left to the compiler's contraction: the arithmetic of the FP32 radix passes,
-// kept as they are where results in FP32 are compared with earlier ones.
+// left to the compiler's contraction: the arithmetic of the radix passes
+// (stockham_pass). The mixed tier's solves run on them (system potentials
+// included) and turn any other rounding into another result at the scale of
+// their thresholds (GammaOp::keeps_rounding), so it does not change.
 namespace plain {
 template <typename T>
 __device__ __forceinline__ c2<T> cadd(c2<T> a, c2<T> b) { return {a.x + b.x, a.y + b.y}; }
@@ -370,13 +372,11 @@ __device__ __forceinline__ void stockham_pass(c2<T>* lds, int nlines, int lstrid
         if (r > 0) {
           c2<T> w = roots[jm * r * ts];
           if (INV) w.y = -w.y;
-          if constexpr (sizeof(T) == 4) a = plain::cmul(a, w);
-          else a = cmul(a, w);
+          a = plain::cmul(a, w);
         }
         v[k][r] = a;
       }
-      if constexpr (sizeof(T) == 4) plain::dft<R, INV>(v[k]);
-      else dft<R, INV>(v[k]);
+      plain::dft<R, INV>(v[k]);
     }
   }
   __syncthreads();

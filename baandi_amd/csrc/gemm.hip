@@ -125,11 +125,54 @@ TnPlan tn_plan(int64_t M, int64_t N, int64_t K) {
   }
   return best;
 }
+
+// Sums::chain: the tiles that fill the chip at the mixed tier's products (m x m
+// and n x m; bits do not depend on the tile).
+template <typename F>
+void with_chain_tile(int64_t M, int64_t N, const F& f) {
+  if (tiles_of({2, 4}, M, N) >= 256) return f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+  return f(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+}
+
+// Sums::chain: at most 512 workgroups' worth of 64 x 64 tiles and 256 chunks,
+// 256 k at least in each.
+int64_t chain_chunk(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t splits = std::min<int64_t>(
+      {std::max<int64_t>(1, 512 / tiles), std::max<int64_t>(1, K / 256), int64_t(256)});
+  return ((K + splits - 1) / splits + gemm64::TK - 1) / gemm64::TK * gemm64::TK;
+}
+
+template <bool TA>
+void launch_chain(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
+                  const double* B, int64_t ldb, double beta, double* C, int64_t ldc) {
+  with_chain_tile(M, N, [&](auto rb, auto nb) {
+    constexpr int RB = decltype(rb)::value, NB = decltype(nb)::value;
+    const int64_t tiles_n = (N + 16 * NB - 1) / (16 * NB), total = tiles_of({RB, NB}, M, N);
+    hipLaunchKernelGGL((gemm64::k_gemm_nn<RB, NB, TA, true>), dim3(xcd_grid(total)), dim3(256), 0, s, M, N, K,
+                       int(tiles_n), int(total), alpha, A, lda, B, ldb, beta, C, ldc);
+  });
+}
+
+void chain_tn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
+              const double* B, int64_t ldb, double beta, double* C, int64_t ldc, double* work) {
+  const int64_t chunk = chain_chunk(M, N, K), used = chunk > 0 ? (K + chunk - 1) / chunk : 1;
+  if (used <= 1) return launch_chain<true>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  with_chain_tile(M, N, [&](auto rb, auto nb) {
+    constexpr int RB = decltype(rb)::value, NB = decltype(nb)::value;
+    const int64_t tiles_m = (M + 64 * RB - 1) / (64 * RB), tiles = tiles_of({RB, NB}, M, N), total = tiles * used;
+    hipLaunchKernelGGL((gemm64::k_gemm_tn<RB, NB, true>), dim3(xcd_grid(total)), dim3(256), 0, s, M, N, K, chunk,
+                       int(tiles_m), int(tiles), int(total), A, lda, B, ldb, work);
+  });
+  hipLaunchKernelGGL(gemm64::k_gemm_reduce<true>, dim3(unsigned((M * N + 63) / 64)), dim3(256), 0, s, M, N, int(used),
+                     alpha, work, beta, C, ldc);
+}
 }  // namespace
 
-void gemm_nn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
-             int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc) {
+void gemm_nn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A, int64_t lda,
+             const double* B, int64_t ldb, double beta, double* C, int64_t ldc, Sums sums) {
   if (M <= 0 || N <= 0) return;
+  if (sums == Sums::chain) return launch_chain<false>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
   if (short_product(M, N, K)) return launch_short<false>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
   const int64_t slices = (K + gemm64::TK - 1) / gemm64::TK;
   const TileShape* best = &kTiles[0];
@@ -143,8 +186,9 @@ void gemm_nn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const
   });
 }
 
-// Monotone in M and N at a fixed K, and never below max_splits M N, so one
-// buffer serves every call up to its sizing shape.
+// Monotone in M, N and K, and never below max_splits M N (nor the chunks of
+// Sums::chain: at most 512 of 4096 values, K / 256 M N), so one buffer serves
+// every call up to its sizing shape.
 int64_t gemm_tn_work(int64_t M, int64_t N, int64_t K) {
   const int64_t few = std::max<int64_t>(1, std::min<int64_t>(K / 256, 8));
   if (K < 1024) return few * M * N;
@@ -153,8 +197,9 @@ int64_t gemm_tn_work(int64_t M, int64_t N, int64_t K) {
 
 void gemm_tn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
              int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc,
-             double* work) {
+             double* work, Sums sums) {
   if (M <= 0 || N <= 0) return;
+  if (sums == Sums::chain) return chain_tn(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, work);
   if (short_product(M, N, K)) return launch_short<true>(s, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
   const TnPlan p = tn_plan(M, N, K);
   with_tile(p.tile, [&](auto rb, auto nb) {
@@ -164,7 +209,7 @@ void gemm_tn(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const
     hipLaunchKernelGGL((gemm64::k_gemm_tn<RB, NB>), dim3(xcd_grid(total)), dim3(256), 0, s, M, N, K, p.chunk,
                        int(tiles_m), int(tiles), int(total), A, lda, B, ldb, work);
   });
-  hipLaunchKernelGGL(gemm64::k_gemm_reduce, dim3(unsigned((M * N + 63) / 64)), dim3(256), 0, s, M, N, p.splits, alpha,
+  hipLaunchKernelGGL(gemm64::k_gemm_reduce<>, dim3(unsigned((M * N + 63) / 64)), dim3(256), 0, s, M, N, p.splits, alpha,
                      work, beta, C, ldc);
 }
 

@@ -14,6 +14,10 @@
 // Global loads run D slices (16 k each) ahead in registers, the B stages are
 // double buffered, and one barrier a slice is left.
 //
+// CHAIN (Sums::chain): lane l's pair is k = l / 16 and l / 16 + 4, so that the two
+// MFMAs take four ascending k each and every result is one ascending chain;
+// the loads are then of 8 bytes.
+//
 // Bound: FP64 MFMA issue at the large shapes, the latency of a slice at the
 // small ones. Measured against 64 x 64 tiles with both operands through LDS
 // one slice ahead: A^T B of 2560 x 1126 x 191711 35.8 -> 19.3 ms (57 TFLOP/s),
@@ -53,7 +57,7 @@ struct Tile {
 // A: row i, index k at A[i + k lda] (TA = false) or A[k + i lda] (TA = true);
 // B: k, column j at B[k + j ldb]. Rows past M and columns past N repeat the
 // last one (their results are not stored); k past kend counts as zero.
-template <int RB, int NB, bool TA>
+template <int RB, int NB, bool TA, bool CHAIN = false>
 __device__ __forceinline__ void tile_product(int64_t M, int64_t N, int64_t kbeg, int64_t kend, int64_t row0,
                                              int64_t col0, const double* __restrict__ A, int64_t lda,
                                              const double* __restrict__ B, int64_t ldb,
@@ -62,6 +66,8 @@ __device__ __forceinline__ void tile_product(int64_t M, int64_t N, int64_t kbeg,
   constexpr int D = T::depth, BW = T::bwave;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
+  constexpr int step = CHAIN ? 4 : 1;       // a lane's k: first and first + step
+  const int first = CHAIN ? lg : 2 * lg;
 #pragma unroll
   for (int r = 0; r < RB; ++r)
 #pragma unroll
@@ -70,32 +76,33 @@ __device__ __forceinline__ void tile_product(int64_t M, int64_t N, int64_t kbeg,
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
     const int64_t i = min(row0 + (wave * RB + r) * 16 + li, M - 1);
-    pa[r] = TA ? A + i * lda + 2 * lg : A + i + 2 * lg * lda;
+    pa[r] = TA ? A + i * lda + first : A + i + first * lda;
   }
   // Fragment f = wave + 4 u of a slice: column block f / 2, k half f % 2.
   const double* pb[BW];
 #pragma unroll
   for (int u = 0; u < BW; ++u) {
     const int f = min(wave + 4 * u, T::bfrags - 1);
-    pb[u] = B + min(col0 + (f >> 1) * 16 + li, N - 1) * ldb + (f & 1) * 8 + 2 * lg;
+    pb[u] = B + min(col0 + (f >> 1) * 16 + li, N - 1) * ldb + (f & 1) * 8 + first;
   }
+  auto along_k = [](const double* p) {  // the pair where k is contiguous
+    if (CHAIN) return f64x2{p[0], p[step]};
+    const Pair8 v = *reinterpret_cast<const Pair8*>(p);
+    return f64x2{v.x, v.y};
+  };
   f64x2 ra[D][RB][2], rb[D][BW];
   auto fetch = [&](f64x2 (&a)[RB][2], f64x2 (&b)[BW], int64_t k0) {
 #pragma unroll
-    for (int u = 0; u < BW; ++u) {
-      const Pair8 v = *reinterpret_cast<const Pair8*>(pb[u] + k0);
-      b[u] = f64x2{v.x, v.y};
-    }
+    for (int u = 0; u < BW; ++u) b[u] = along_k(pb[u] + k0);
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (TA) {
-          const Pair8 v = *reinterpret_cast<const Pair8*>(pa[r] + k0 + 8 * h);
-          a[r][h] = f64x2{v.x, v.y};
+          a[r][h] = along_k(pa[r] + k0 + 8 * h);
         } else {
           const double* p = pa[r] + (k0 + 8 * h) * lda;
-          a[r][h] = f64x2{p[0], p[lda]};
+          a[r][h] = f64x2{p[0], p[step * lda]};
         }
       }
   };
@@ -148,16 +155,16 @@ __device__ __forceinline__ void tile_product(int64_t M, int64_t N, int64_t kbeg,
 #pragma unroll
     for (int u = 0; u < BW; ++u) {
       const int f = min(wave + 4 * u, T::bfrags - 1);
-      const int64_t k = k0 + (f & 1) * 8 + 2 * lg;
-      b[u] = f64x2{k < kend ? pb[u][k0] : 0.0, k + 1 < kend ? pb[u][k0 + 1] : 0.0};
+      const int64_t k = k0 + (f & 1) * 8 + first;
+      b[u] = f64x2{k < kend ? pb[u][k0] : 0.0, k + step < kend ? pb[u][k0 + step] : 0.0};
     }
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int64_t k = k0 + 8 * h + 2 * lg;
+        const int64_t k = k0 + 8 * h + first;
         const double* p = TA ? pa[r] + k0 + 8 * h : pa[r] + (k0 + 8 * h) * lda;
-        a[r][h] = f64x2{k < kend ? p[0] : 0.0, k + 1 < kend ? p[TA ? 1 : lda] : 0.0};
+        a[r][h] = f64x2{k < kend ? p[0] : 0.0, k + step < kend ? p[TA ? step : step * lda] : 0.0};
       }
     const int stage = int(full) & 1;
     stash(b, stage);
@@ -175,8 +182,8 @@ __device__ __forceinline__ int xcd_index(int total) {
   return (int(blockIdx.x) % kXcds) * per_xcd + int(blockIdx.x) / kXcds;
 }
 
-// NN: C = alpha A B + beta C.
-template <int RB, int NB>
+// C = alpha A B + beta C (TA: A^T), the whole k range in one workgroup.
+template <int RB, int NB, bool TA = false, bool CHAIN = false>
 __global__ __launch_bounds__(256, (Tile<RB, NB>::waves)) void k_gemm_nn(int64_t M, int64_t N, int64_t K, int tiles_n,
                                                                       int total, double alpha,
                                                                       const double* __restrict__ A, int64_t lda,
@@ -188,7 +195,7 @@ __global__ __launch_bounds__(256, (Tile<RB, NB>::waves)) void k_gemm_nn(int64_t 
   if (logical >= total) return;
   const int64_t row0 = int64_t(logical / tiles_n) * (64 * RB), col0 = int64_t(logical % tiles_n) * (16 * NB);
   f64x4 acc[RB][NB];
-  tile_product<RB, NB, false>(M, N, 0, K, row0, col0, A, lda, B, ldb, Bs, acc);
+  tile_product<RB, NB, TA, CHAIN>(M, N, 0, K, row0, col0, A, lda, B, ldb, Bs, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -207,7 +214,7 @@ __global__ __launch_bounds__(256, (Tile<RB, NB>::waves)) void k_gemm_nn(int64_t 
 }
 
 // TN partial: part[s] (M x N) = sum over k in chunk s of A[k, i] B[k, j].
-template <int RB, int NB>
+template <int RB, int NB, bool CHAIN = false>
 __global__ __launch_bounds__(256, (Tile<RB, NB>::waves)) void k_gemm_tn(int64_t M, int64_t N, int64_t K, int64_t chunk,
                                                                       int tiles_m, int tiles, int total,
                                                                       const double* __restrict__ A, int64_t lda,
@@ -220,7 +227,7 @@ __global__ __launch_bounds__(256, (Tile<RB, NB>::waves)) void k_gemm_tn(int64_t 
   const int64_t row0 = int64_t(tile % tiles_m) * (64 * RB), col0 = int64_t(tile / tiles_m) * (16 * NB);
   const int64_t kbeg = int64_t(kc) * chunk, kend = min(K, kbeg + chunk);
   f64x4 acc[RB][NB];
-  tile_product<RB, NB, true>(M, N, kbeg, kend, row0, col0, A, lda, B, ldb, Bs, acc);
+  tile_product<RB, NB, true, CHAIN>(M, N, kbeg, kend, row0, col0, A, lda, B, ldb, Bs, acc);
   double* out = part + int64_t(kc) * M * N;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -322,14 +329,16 @@ __global__ __launch_bounds__(256) void k_gemm_short(int64_t M, int64_t N, int64_
 }
 
 // C = alpha * (the partial sums in chunk order) + beta * C. Four threads an
-// element, a quarter of the chunks each (eight loads in flight).
+// element, a quarter of the chunks each (eight loads in flight); CHAIN: one
+// thread an element, all the chunks in order.
+template <bool CHAIN = false>
 __global__ __launch_bounds__(256) void k_gemm_reduce(int64_t M, int64_t N, int splits, double alpha,
                                                      const double* __restrict__ part, double beta,
                                                      double* __restrict__ C, int64_t ldc) {
   __shared__ double sum[4][64];
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
   const int64_t e = int64_t(blockIdx.x) * 64 + lane, total = M * N;
-  const int per = (splits + 3) / 4, end = min(splits, (q + 1) * per);
+  const int per = CHAIN ? splits : (splits + 3) / 4, end = min(splits, (q + 1) * per);
   double s = 0.0;
   if (e < total) {
     int p = q * per;
@@ -345,7 +354,7 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(int64_t M, int64_t N, int s
   sum[q][lane] = s;
   __syncthreads();
   if (q != 0 || e >= total) return;
-  s = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
+  if (!CHAIN) s = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
   double* c = C + e % M + (e / M) * ldc;
   *c = beta == 0.0 ? alpha * s : alpha * s + beta * *c;
 }

@@ -558,7 +558,7 @@ static void order_sticks(StickPlan& p, std::vector<std::pair<int, int>>& sticks)
   p.lines = std::move(lines);
 }
 
-StickPlan build_stick_plan(const System& s, bool paired) {
+StickPlan build_stick_plan(const System& s, bool paired, size_t elem) {
   StickPlan p{};
   p.n0 = s.dims[0];
   p.n1 = s.dims[1];
@@ -580,16 +580,19 @@ StickPlan build_stick_plan(const System& s, bool paired) {
       keys.insert({c, b});
     }
   std::vector<std::pair<int, int>> sticks(keys.begin(), keys.end());
-  order_sticks(p, sticks);
-  p.S = int(sticks.size());
-  std::map<std::pair<int, int>, int> index;
-  for (int i = 0; i < p.S; ++i) index[sticks[i]] = i;
   std::set<int> zs;
   for (auto& k : sticks) zs.insert(k.first);
   p.z_of_zc.assign(zs.begin(), zs.end());
   p.Z = int(p.z_of_zc.size());
   std::map<int, int> zc_of;
   for (int i = 0; i < p.Z; ++i) zc_of[p.z_of_zc[i]] = i;
+  // The paired x pass where it is built for the length (it reads rows in twos).
+  if (paired && s.nrep > 1) p.xshape = stick_shape(p.n0);
+  const bool by_line = p.xshape.on || (paired && pair_shape(p.n1, p.n2, p.Z, elem).on);
+  if (by_line) order_sticks(p, sticks);
+  p.S = int(sticks.size());
+  std::map<std::pair<int, int>, int> index;
+  for (int i = 0; i < p.S; ++i) index[sticks[i]] = i;
   // Tile size: the largest power of two <= 32 whose x transform fits a workgroup.
   // Radix-9/8 passes only where the batches fit as with radices 2-5.
   if (!fft_fits(32, p.rx)) p.rx = radix_plan(p.n0, false);
@@ -598,16 +601,15 @@ StickPlan build_stick_plan(const System& s, bool paired) {
   p.T = 32;
   while (p.T > 1 && !fft_fits(p.T, p.rx)) p.T /= 2;
   if (!fft_fits(p.T, p.rx)) fail(BD_ERR_INVALID_PARAMETER, "x FFT does not fit a workgroup");
-  // The paired x pass where it is built for the length (it reads rows in twos).
-  if (paired && s.nrep > 1) p.xshape = stick_shape(p.n0);
   if (p.xshape.on) p.T = p.xshape.tile;
   p.chunk = 16;
   while (p.chunk > 1 && !fft_fits(p.chunk, p.rz)) p.chunk /= 2;
   p.chunk = std::min(p.chunk, p.n1);
   // Mirror units (stick + its inversion partner) packed whole into tiles, so
-  // +G and -G of every representative share a tile.
-  // (the mirrors after the sticks they belong to, so that a wavefront's slots
-  // are neighbours in the stick buffer).
+  // +G and -G of every representative share a tile. Without a paired pass the
+  // stick buffer holds the slots in order; with one it holds the sticks line by
+  // line, and in a tile the mirrors come after the sticks they belong to, so
+  // that a wavefront's slots are neighbours in the buffer.
   std::vector<int> tile_of(p.S, -1), slot_of(p.S, -1);
   std::vector<std::vector<std::pair<int, int>>> units(1);
   int tile = 0, used = 0;
@@ -631,21 +633,25 @@ StickPlan build_stick_plan(const System& s, bool paired) {
   }
   for (const auto& in_tile : units) {
     int slot = 0;
-    for (const auto& u : in_tile) slot_of[u.first] = slot++;
+    for (const auto& u : in_tile) {
+      slot_of[u.first] = slot++;
+      if (!by_line && u.second != u.first) slot_of[u.second] = slot++;
+    }
     for (const auto& u : in_tile)
-      if (u.second != u.first) slot_of[u.second] = slot++;
+      if (by_line && u.second != u.first) slot_of[u.second] = slot++;
   }
   p.ntiles = tile + 1;
   p.Spad = p.ntiles * p.T;
   p.stick_yz.assign(p.Spad, make_int2(-1, -1));
   p.stick_dst.assign(p.Spad, -1);
   for (int i = 0; i < p.S; ++i) {
-    p.stick_yz[i] = make_int2(sticks[i].second, zc_of[sticks[i].first]);
-    p.stick_dst[tile_of[i] * p.T + slot_of[i]] = i;
+    const int slot = tile_of[i] * p.T + slot_of[i], at = by_line ? i : slot;
+    p.stick_yz[at] = make_int2(sticks[i].second, zc_of[sticks[i].first]);
+    p.stick_dst[slot] = at;
   }
-  int pads = p.S;  // the padding slots behind the sticks
-  for (int& d : p.stick_dst)
-    if (d < 0) d = pads++;
+  int pads = p.S;  // by line: the padding slots behind the sticks
+  for (int slot = 0; slot < p.Spad; ++slot)
+    if (p.stick_dst[slot] < 0) p.stick_dst[slot] = by_line ? pads++ : slot;
   // Representative entries grouped by tile.
   std::vector<std::vector<int4>> per(p.ntiles);
   const StickShape& sh = p.xshape;
@@ -865,9 +871,10 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   capacity = cap;
   precision = prec;
   gemm.bf16x3 = prec == BD_MIXED;
+  if (keeps_rounding()) gemm.sums = Sums::chain;
   nproj = kb ? 2 * s.nproj : s.nproj;
   const size_t elem = fft32() ? sizeof(c2<float>) : sizeof(c2<double>);
-  plan = kb ? build_k_stick_plan(s, *kb, int(nproj), elem) : build_stick_plan(s);
+  plan = kb ? build_k_stick_plan(s, *kb, int(nproj), elem) : build_stick_plan(s, !keeps_rounding(), elem);
   size_t lds_max = size_t(prop.sharedMemPerBlock);
   if (stick_lds(plan, elem) > lds_max) fail(BD_ERR_INVALID_PARAMETER, "x FFT tile exceeds the device LDS");
   if (fft32()) allow_lds<float>(plan);
@@ -921,7 +928,7 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   const int pairs = slots(cap);
   int spad = plan.Spad;
   if (!kb && precision == BD_FP32_HX && (plan.xshape.on || pair.on)) {
-    dplan = build_stick_plan(s, false);
+    dplan = build_stick_plan(s, false, elem);
     // (Planes beyond one workgroup's passes take the paired pass.)
     plain_density = fft_fits(dplan.Z, dplan.ry) && plane_lds(dplan, elem) <= lds_max;
   }

@@ -125,6 +125,14 @@ struct GammaOp {
   // The FFT stages (sticks, planes, the potential) run in FP32 in every mode
   // but FP64; the GEMMs are BF16x3 only in BD_MIXED.
   bool fft32() const { return precision != BD_FP64; }
+  // The mixed tier at Gamma keeps the rounding of the radix passes and of
+  // products summed in one chain (and with it the solver its factorisations and
+  // counts, Sums::chain). Its solves stop at Ritz changes just above the BF16x3
+  // noise, and a change of rounding anywhere redraws that noise within three
+  // products: a band stops an iteration earlier or later, and the density moves
+  // by 5e-4 to 4e-2 (16 to 64 atoms). A stored calculation is to come out again,
+  // so this tier does not follow a faster kernel with another order of sums.
+  bool keeps_rounding() const { return !kb && precision == BD_MIXED; }
   int64_t nproj;
   hipStream_t stream = nullptr;
   StickPlan plan;
@@ -233,7 +241,8 @@ void fused_launch(const GammaOp& op, const FusedShape& f, size_t lds, const KWor
                   int count, int total, hipStream_t s);
 bool fft_fits_threads(int nlines, const RadixPlan& rp, int threads);
 
-StickPlan build_stick_plan(const System& s, bool paired = true);
+// paired: with the paired passes where they are built (elem = sizeof(c2<F>)).
+StickPlan build_stick_plan(const System& s, bool paired, size_t elem);
 StickPlan build_k_stick_plan(const System& s, const KBasis& kb, int nproj, size_t elem);
 RadixPlan radix_plan(int n, bool big);
 

@@ -52,15 +52,16 @@ __global__ void k_copy_block(int k, const double* __restrict__ S, int64_t lds, d
 // already set by an earlier block of the same border leaves the block
 // untouched; min_ratio keeps the minimum over the blocks.
 //
-// G = M D M^T with M unit lower: column l sits in the registers of wave
-// l mod 16 (lane i owns row i, and i + 64 past 64 rows), and a step passes one column
-// through LDS: one barrier, one division. The pivots are tested together at
-// the end (a failed one only spoils later columns, which nobody then reads).
-// M^{-1} by forward substitution, a wave's columns side by side so that their
-// chains (a lane read and the update) overlap; L^{-1} = D^{-1/2} M^{-1}.
-// Bound by the chain of steps. k = 80: 51 us, k = 20: 7; 98 and 16 with the
-// block as a packed triangle in LDS, two divisions a step and one column at a
-// time in the substitution.
+// G = L L^T: column l of the elimination sits in the registers of wave l mod 16
+// (lane i owns row i, and i + 64 past 64 rows), and a step passes one column
+// through LDS: one barrier, one division (by the pivot d_j; L's column is the
+// passed one over sqrt(d_j), formed for all columns at the end). The pivots are
+// tested together then, too (a failed one only spoils later columns, which
+// nobody reads). L^{-1} by forward substitution, a wave's columns side by side
+// so that their chains (a lane read, a product and the update) overlap.
+// Bound by the chain of steps. k = 80: 55 us, k = 20: 8; 98 and 16, with the
+// same bits, with the block as a packed triangle in LDS, two divisions a step
+// and one column at a time in the substitution.
 template <int NC>
 __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __restrict__ G,
                                                       const double* __restrict__ sdiag, int64_t sstride,
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
   const int ldm = k + 1;
   double* M = sh;                        // k columns of ldm
   double* pass = M + int64_t(k) * ldm;   // two slots of k: the column of a step
-  double* dv = pass + 2 * k;             // k: the pivots
+  double* dv = pass + 2 * k;             // k: the pivots, then 1 / sqrt of them
   double a[NC][R];
   int row[R];  // this lane's rows, the last one's for those past it
 #pragma unroll
@@ -111,11 +112,11 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
       for (int c = jc; c < NC; ++c) alj[c] = col[min(wave + nw * c, k - 1)];
       const double inv_d = 1.0 / dj;
 #pragma unroll
-      for (int t = 0; t < R; ++t) mine[t] *= inv_d;
+      for (int c = jc; c < NC; ++c) alj[c] *= inv_d;
 #pragma unroll
       for (int c = jc; c < NC; ++c)
 #pragma unroll
-        for (int t = 0; t < R; ++t) a[c][t] = fma(-alj[c], mine[t], a[c][t]);
+        for (int t = 0; t < R; ++t) a[c][t] = fma(-mine[t], alj[c], a[c][t]);
       if (wave == jw) {
 #pragma unroll
         for (int t = 0; t < R; ++t) {
@@ -145,7 +146,15 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
     if (failed) flag[0] = 1;
   }
   if (failed) return;  // every wave found the same: uniform exit
-  double x[NC][R], ml[R];  // (M is zero up to the diagonal)
+  // M = L below the diagonal.
+  for (int l = wave; l < k; l += nw) {
+    const double sd = sqrt(dv[l]);
+    for (int i = l + 1 + lane; i < k; i += 64) M[i + int64_t(l) * ldm] /= sd;
+  }
+  __syncthreads();
+  for (int l = tid; l < k; l += kCT) dv[l] = 1.0 / sqrt(dv[l]);
+  __syncthreads();
+  double x[NC][R], ml[R], rl = dv[0];  // (M is zero up to the diagonal)
 #pragma unroll
   for (int t = 0; t < R; ++t) {
     ml[t] = M[row[t]];
@@ -159,21 +168,23 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
       double next[R];
 #pragma unroll
       for (int t = 0; t < R; ++t) next[t] = M[row[t] + int64_t(min(l + 1, k - 1)) * ldm];
+      const double next_rl = dv[min(l + 1, k - 1)];
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        const double xl = read_lane(x[c][tl], l - 64 * tl);
+        const double xl = read_lane(x[c][tl], l - 64 * tl) * rl;
 #pragma unroll
         for (int t = 0; t < R; ++t) x[c][t] = fma(-ml[t], xl, x[c][t]);
       }
 #pragma unroll
       for (int t = 0; t < R; ++t) ml[t] = next[t];
+      rl = next_rl;
     }
   }
 #pragma unroll
   for (int t = 0; t < R; ++t) {
     const int i = lane + 64 * t;
     if (i >= k) continue;
-    const double rs = 1.0 / sqrt(dv[i]);
+    const double rs = dv[i];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int l = wave + nw * c;
@@ -272,10 +283,10 @@ constexpr int kFactorSplit = 96;
 // W = T11 S12, G = S22 - W^T W, T22 = chol(G)^{-1}, T21 = -T22 W^T T11.
 void extend_block(hipStream_t s, const double* S, double* T, int cap, int from, int to, const FactorWork& fw) {
   const int k = to - from;
-  if (from > 0) gemm_nn(s, from, k, from, 1.0, T, cap, S + int64_t(from) * cap, cap, 0.0, fw.W, from);
+  if (from > 0) fw.gemm.nn64(s, from, k, from, 1.0, T, cap, S + int64_t(from) * cap, cap, 0.0, fw.W, from);
   hipLaunchKernelGGL(k_copy_block, dim3((k + 255) / 256, k), dim3(256), 0, s, k,
                      S + from + int64_t(from) * cap, int64_t(cap), fw.G);
-  if (from > 0) gemm_tn(s, k, k, from, -1.0, fw.W, from, fw.W, from, 1.0, fw.G, k, fw.gwork);
+  if (from > 0) fw.gemm.tn64(s, k, k, from, -1.0, fw.W, from, fw.W, from, 1.0, fw.G, k, fw.gwork);
   double* T22 = T + from + int64_t(from) * cap;
   const size_t lds = (size_t(k) * (k + 1) + 3 * size_t(k)) * 8;
   if (k > kFactorBlock || lds > 160 * 1024) fail(BD_ERR_INVALID_PARAMETER, "inverse Cholesky block too large");
@@ -284,8 +295,8 @@ void extend_block(hipStream_t s, const double* S, double* T, int cap, int from, 
   hipLaunchKernelGGL(chol, dim3(1), dim3(kCT), lds, s, k, fw.G, S + from + int64_t(from) * cap,
                      int64_t(cap) + 1, T22, int64_t(cap), fw.flag, fw.min_ratio);
   if (from > 0) {
-    gemm_tn(s, k, from, from, 1.0, fw.W, from, T, cap, 0.0, fw.U, k, fw.gwork);         // U = W^T T11
-    gemm_nn(s, k, from, k, -1.0, T22, cap, fw.U, k, 0.0, T + from, cap);                  // T21 = -T22 U
+    fw.gemm.tn64(s, k, from, from, 1.0, fw.W, from, T, cap, 0.0, fw.U, k, fw.gwork);  // U = W^T T11
+    fw.gemm.nn64(s, k, from, k, -1.0, T22, cap, fw.U, k, 0.0, T + from, cap);          // T21 = -T22 U
   }
   hipLaunchKernelGGL(k_growth_guard, dim3((k + 3) / 4), dim3(256), 0, s, S, T, cap, from, to, fw.growth_guard,
                      fw.flag);
