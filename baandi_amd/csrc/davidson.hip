@@ -362,7 +362,7 @@ struct Solver {
   // synchronisation.
   void queue_apply(const double* src, int k, double* dst) {
     BD_HIP(hipEventRecord(ev0, s));
-    op.apply(src, n, k, dst, n);
+    op.solve_apply(src, n, k, dst, n);
     BD_HIP(hipEventRecord(ev1, s));
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, s, w.flag);
     hipLaunchKernelGGL(k_finite, dim3(256), dim3(256), 0, s, dst, n * k, w.flag);
@@ -1468,7 +1468,7 @@ struct BlockGraph {
   // The iteration's device work (captured once, then replayed).
   void enqueue() {
     before_apply();
-    op.apply(V.p + n * nb, n, nb, HV.p + n * nb, n);
+    op.solve_apply(V.p + n * nb, n, nb, HV.p + n * nb, n);
     ritz(m2);
   }
 
@@ -1480,7 +1480,7 @@ struct BlockGraph {
 
   void start(const double* x0, int64_t ldx0) {
     start_before_apply(x0, ldx0);
-    op.apply(V.p, n, nb, HV.p, n);
+    op.solve_apply(V.p, n, nb, HV.p, n);
     ritz(nb);
     check();
   }

@@ -874,8 +874,15 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   if (keeps_rounding()) gemm.sums = Sums::chain;
   nproj = kb ? 2 * s.nproj : s.nproj;
   const size_t elem = fft32() ? sizeof(c2<float>) : sizeof(c2<double>);
-  plan = kb ? build_k_stick_plan(s, *kb, int(nproj), elem) : build_stick_plan(s, !keeps_rounding(), elem);
+  plan = kb ? build_k_stick_plan(s, *kb, int(nproj), elem) : build_stick_plan(s, true, elem);
   size_t lds_max = size_t(prop.sharedMemPerBlock);
+  if (!kb && fft32() && (plan.xshape.on || (!plan.lines.empty() && pair_shape(plan.n1, plan.n2, plan.Z, elem).on))) {
+    dplan = build_stick_plan(s, false, elem);
+    // (FP32 densities beyond one workgroup's passes take the paired pass; a
+    // mixed operator then has the radix passes alone.)
+    plain = fft_fits(dplan.Z, dplan.ry) && plane_lds(dplan, elem) <= lds_max;
+    if (keeps_rounding() && !plain) plan = dplan;
+  }
   if (stick_lds(plan, elem) > lds_max) fail(BD_ERR_INVALID_PARAMETER, "x FFT tile exceeds the device LDS");
   if (fft32()) allow_lds<float>(plan);
   else allow_lds<double>(plan);
@@ -927,12 +934,7 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   }
   const int pairs = slots(cap);
   int spad = plan.Spad;
-  if (!kb && precision == BD_FP32_HX && (plan.xshape.on || pair.on)) {
-    dplan = build_stick_plan(s, false, elem);
-    // (Planes beyond one workgroup's passes take the paired pass.)
-    plain_density = fft_fits(dplan.Z, dplan.ry) && plane_lds(dplan, elem) <= lds_max;
-  }
-  if (plain_density) {
+  if (plain) {
     // Large planes: 512 threads and the longest row chunk, as the shape search
     // picks there (the bits do not depend on the shape).
     if (dplan.n1 * dplan.n2 >= 64 * 64 && fft_fits_threads(dplan.Z, dplan.ry, 512))
@@ -1125,6 +1127,33 @@ void GammaOp::sticks_to_columns(const double* x, int64_t ldx, double* y, int64_t
   }
 }
 
+// X -> sticks, and H·X's local part, on the radix passes' own plan.
+void GammaOp::plain_to_sticks(const double* x, int64_t ldx, int m) {
+  const StickPlan& p = dplan;
+  hipLaunchKernelGGL(k_stick_inverse<float>, dim3(p.ntiles, slots(m)), dim3(kThreads), stick_lds(p, sizeof(c2<float>)),
+                     stream, x, ldx, m, p.n0, p.T, p.Spad, d_dtile_off.p, d_dentries.p, d_ddst.p, d_roots.p, p.rx,
+                     reinterpret_cast<c2<float>*>(d_sticks.p));
+}
+
+void GammaOp::plain_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
+  const StickPlan& p = dplan;
+  const int pairs = slots(m);
+  const size_t e = sizeof(c2<float>);
+  c2<float>* sticks = reinterpret_cast<c2<float>*>(d_sticks.p);
+  if (profiling) BD_HIP(hipEventRecord(ev[0], stream));
+  plain_to_sticks(x, ldx, m);
+  if (profiling) BD_HIP(hipEventRecord(ev[1], stream));
+  const auto plane = plain_threads == 512 ? &k_plane<0, float, 512> : &k_plane<0, float, 256>;
+  hipLaunchKernelGGL(plane, dim3(pairs, p.n0), dim3(plain_threads), plane_lds(p, e), stream, sticks, p.n0, p.n1, p.n2,
+                     p.Spad, p.Z, p.chunk, d_dyz.p, d_zc.p, d_roots.p, p.ry, p.rz, d_potential32.p, pairs, nullptr,
+                     0.0, nullptr, nullptr);
+  if (profiling) BD_HIP(hipEventRecord(ev[2], stream));
+  hipLaunchKernelGGL(k_stick_forward<float>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x, ldx, y,
+                     ldy, m, p.n0, p.T, p.Spad, d_dtile_off.p, d_dentries.p, d_ddst.p, d_roots.p, p.rx, sticks,
+                     d_kinetic.p, 1.0 / double(N), 0);
+  if (profiling) BD_HIP(hipEventRecord(ev[3], stream));
+}
+
 template <typename F>
 void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
   const StickPlan& p = plan;
@@ -1165,19 +1194,15 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
   const size_t e = sizeof(c2<F>);
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
   const int groups = std::min(pairs, kDensityGroups);
-  if (plain_density)
-    hipLaunchKernelGGL(k_stick_inverse<F>, dim3(dplan.ntiles, pairs), dim3(kThreads), stick_lds(dplan, e), stream, x,
-                       ldx, m, dplan.n0, dplan.T, dplan.Spad, d_dtile_off.p, d_dentries.p, d_ddst.p, d_roots.p,
-                       dplan.rx, sticks);
-  else
-    columns_to_sticks<F>(x, ldx, m);
+  if (plain_density()) plain_to_sticks(x, ldx, m);
+  else columns_to_sticks<F>(x, ldx, m);
   // Warm start: keep the pairs' real-space fields (Gamma, fused plane pass).
   c2<F>* keep = kept_on ? reinterpret_cast<c2<F>*>(d_kept.p) : nullptr;
   kept_valid = keep != nullptr;
   kept_x = x;
   kept_ldx = ldx;
   kept_m = m;
-  if (plain_density) {
+  if (plain_density()) {
     const auto plane = plain_threads == 512 ? &k_plane<1, F, 512> : &k_plane<1, F, 256>;
     hipLaunchKernelGGL(plane, dim3(dplan.n0, groups), dim3(plain_threads), plane_lds(dplan, e), stream, sticks, dplan.n0,
                        dplan.n1, dplan.n2, dplan.Spad, dplan.Z, dplan.chunk, d_dyz.p, d_zc.p, d_roots.p, dplan.ry,
@@ -1261,7 +1286,7 @@ void GammaOp::projections(const double* x, int64_t ldx, int m) {
   gemm.tn(stream, nproj, m, n, 1.0, d_proj.p, n, x, ldx, 0.0, d_q.p, nproj, d_work.p);
 }
 
-void GammaOp::apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) {
+void GammaOp::apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy, bool solve) {
   if (m < 0 || m > capacity) fail(BD_ERR_INVALID_PARAMETER, "column count exceeds capacity");
   if (ldx < n || ldy < n) fail(BD_ERR_INVALID_PARAMETER, "leading dimension smaller than rows");
   if (!has_potential) fail(BD_ERR_INVALID_PARAMETER, "no potential installed");
@@ -1286,7 +1311,8 @@ void GammaOp::apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy)
     BD_HIP(hipGetLastError());
     return;
   }
-  if (fft32()) local_apply<float>(x, ldx, m, y, ldy);
+  if (solve && plain_solve()) plain_apply(x, ldx, m, y, ldy);
+  else if (fft32()) local_apply<float>(x, ldx, m, y, ldy);
   else local_apply<double>(x, ldx, m, y, ldy);
   if (nproj > 0) {
     projections(x, ldx, m);

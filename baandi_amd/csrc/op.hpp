@@ -125,13 +125,14 @@ struct GammaOp {
   // The FFT stages (sticks, planes, the potential) run in FP32 in every mode
   // but FP64; the GEMMs are BF16x3 only in BD_MIXED.
   bool fft32() const { return precision != BD_FP64; }
-  // The mixed tier at Gamma keeps the rounding of the radix passes and of
-  // products summed in one chain (and with it the solver its factorisations and
-  // counts, Sums::chain). Its solves stop at Ritz changes just above the BF16x3
-  // noise, and a change of rounding anywhere redraws that noise within three
-  // products: a band stops an iteration earlier or later, and the density moves
-  // by 5e-4 to 4e-2 (16 to 64 atoms). A stored calculation is to come out again,
-  // so this tier does not follow a faster kernel with another order of sums.
+  // The mixed tier's solves at Gamma keep the rounding of the radix passes
+  // (solve_apply) and of products summed in one chain, with the factorisations
+  // and counts that go with it (Sums::chain). They stop at Ritz changes just
+  // above the BF16x3 noise, and a change of rounding anywhere redraws that noise
+  // within three products: a band stops an iteration earlier or later, and the
+  // density moves by 5e-4 (64 atoms) to 4e-2 (16 atoms). The same potential and
+  // start are to give the same solve, so these do not follow a faster kernel
+  // with another order of sums; a single H·X, which moves by 1e-7, does.
   bool keeps_rounding() const { return !kb && precision == BD_MIXED; }
   int64_t nproj;
   hipStream_t stream = nullptr;
@@ -146,10 +147,14 @@ struct GammaOp {
   DevBuf<PlaneLine> d_lines;
   PairShape pair;  // the paired plane pass (plane.hpp), where it applies
   DevBuf<c2<double>> d_sticks2;  // its output sticks where planes go by row parity
-  // BD_FP32_HX at Gamma: the band density stays on the radix passes, whose FP32
-  // rounding it keeps (a density is a sum of squares and shows the transforms'
-  // rounding in full, ~1e-7; H·X shows ~1e-8 of it).
-  bool plain_density = false;
+  // FP32 transforms at Gamma where paired passes are built: the radix passes'
+  // own plan beside them. BD_MIXED solves run on it (keeps_rounding), and so do
+  // BD_FP32_HX band densities, whose rounding it keeps (a density is a sum of
+  // squares and shows the transforms' rounding in full, ~1e-7; H·X shows ~1e-8
+  // of it).
+  bool plain = false;
+  bool plain_density() const { return plain && precision == BD_FP32_HX; }
+  bool plain_solve() const { return plain && keeps_rounding(); }
   int plain_threads = 256;
   StickPlan dplan;
   DevBuf<int> d_dtile_off, d_ddst;
@@ -216,12 +221,16 @@ struct GammaOp {
   int slots(int m) const { return kb ? m : (m + 1) / 2; }
   ~GammaOp();
   void set_potential_dev(const double* v, uint64_t epoch);
-  void apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy);
+  void apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy, bool solve = false);
+  // H·X inside a solve (keeps_rounding).
+  void solve_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy) { apply(x, ldx, m, y, ldy, true); }
   void band_density(const double* x, int64_t ldx, int m, const double* w, double* rho, bool accumulate = false);
   void projections(const double* x, int64_t ldx, int m);  // d_q = P^T X
   void refresh_potential32();
   template <typename F>
   void local_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy);
+  void plain_to_sticks(const double* x, int64_t ldx, int m);
+  void plain_apply(const double* x, int64_t ldx, int m, double* y, int64_t ldy);
   size_t plane_lds_bytes(int chunk) const;
   template <typename F>
   void density(const double* x, int64_t ldx, int m, const double* w, double* rho, bool accumulate = false);
