@@ -1752,9 +1752,11 @@ __global__ __launch_bounds__(256) void k_zback_transform(int m, int want, const 
 // division (m = 320, 160 values: 160 -> 52 us, a wave and 9 or 10 passes of 64
 // points each). The rounding is that of an exact count for entries a few
 // ulps away, as with ratios. T is scaled to a norm below one by a power of
-// two; minors are rescaled every 8 rows; e^2 is at least kTinyE2, far below
-// what moves an eigenvalue, so that a zero minor (x an eigenvalue of a leading
-// block) gives the next one its sign instead of zeroing the rest.
+// two; minors are rescaled every 8 rows by the larger of the last two; e^2 is at
+// least kTinyE2, far below what moves an eigenvalue, so that a zero minor (x an
+// eigenvalue of a leading block) gives the next one its sign instead of zeroing
+// the rest. (Rows d_i = x in a run leave 0 and kTinyE2^(k/2) in turn: 1e-240
+// after 8 rows, which the next 8 would lose unscaled.)
 constexpr double kTinyE2 = 1e-60;
 constexpr int kSturmRows = 8;
 
@@ -1773,7 +1775,7 @@ __device__ __forceinline__ int sturm_count(int chunks, const double2* rows, doub
       p = fma(t[i].x - x, p, -u);
       c += int(unsigned(__double2hiint(p) ^ __double2hiint(pp)) >> 31);
     }
-    const int ex = -max(__builtin_amdgcn_frexp_exp(p), __builtin_amdgcn_frexp_exp(pp));
+    const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(p), fabs(pp)));
     p = ldexp(p, ex);
     pp = ldexp(pp, ex);
   }
