@@ -288,8 +288,8 @@ typedef struct {
 
 typedef struct {
   int32_t iterations;
-  int32_t h_calls;
-  int32_t h_columns;
+  int32_t h_calls;   /* H applications of the method and their columns (a product dropped */
+  int32_t h_columns; /* with a rejected border is not among them, its time is in seconds_apply) */
   int32_t repairs;
   int32_t restarts;
   int32_t all_converged;
