@@ -769,22 +769,26 @@ size_t GammaOp::elem_bytes() const { return fft32() ? sizeof(c2<float>) : sizeof
 // A (threads, chunk) shape of the plane pass: the fused k_plane holds the
 // whole Z x n1 plane; the split pass holds zb z-lines (y transforms) or a
 // chunk of y rows (z transforms) at a time.
-bool GammaOp::plane_shape_valid(int threads, int chunk) const {
-  const StickPlan& p = plan;
+bool GammaOp::plane_shape_valid(const StickPlan& p, int threads, int chunk) const {
   const size_t e = elem_bytes(), lim = 160 * 1024;
   if ((threads != 256 && threads != 512) || chunk < 1 || chunk > p.n1) return false;
   if (!fft_fits_threads(chunk, p.rz, threads)) return false;
   if (p.zb > 0)
     return fft_fits_threads(p.zb, p.ry, threads) && size_t(p.zb * p.n1 + p.n1) * e <= lim &&
            size_t(chunk * p.n2 + p.n2) * e <= lim;
-  return fft_fits_threads(p.Z, p.ry, threads) && plane_lds_bytes(chunk) <= lim;
+  return fft_fits_threads(p.Z, p.ry, threads) && plane_lds_bytes(chunk) <= lim;  // (Z, n1, n2: any plan's)
 }
 
 // Switch to the split plane pass with zb z-lines per y batch (0: the largest
-// that fits), and size its plane buffer: up to ~2 GiB of pairs per batch, at
-// least kDensityGroups pairs (or all).
+// that fits). (Ops on the paired pass move no plane through HBM.)
 void GammaOp::enable_split(int zb) {
-  const StickPlan& p = plan;
+  split_plan(plan, zb, !paired());
+  plane_threads = 256;
+}
+
+// The split pass of plan p, and its plane buffer: up to ~2 GiB of pairs per
+// batch, at least kDensityGroups pairs (or all).
+void GammaOp::split_plan(StickPlan& p, int zb, bool buffer) {
   const size_t e = elem_bytes(), lim = 160 * 1024;
   auto fits = [&](int z) {
     return z >= 1 && z <= p.Z && fft_fits_threads(z, p.ry, 256) && size_t(z * p.n1 + p.n1) * e <= lim;
@@ -798,19 +802,17 @@ void GammaOp::enable_split(int zb) {
   const int pairs = slots(capacity);
   int batch = int(std::max<size_t>(1, (size_t(2) << 30) / plane));
   batch = std::min(pairs, std::max(batch, kDensityGroups));
-  // (Ops on the paired pass move no plane through HBM.)
-  if (!paired() && d_planes.n < (size_t(batch) * plane + 15) / 16) {
+  if (buffer && d_planes.n < (size_t(batch) * plane + 15) / 16) {
     DevBuf<c2<double>> fresh;
     fresh.alloc((size_t(batch) * plane + 15) / 16);
     std::swap(d_planes.p, fresh.p);
     std::swap(d_planes.n, fresh.n);
   }
-  plan.zb = zb;
+  p.zb = zb;
   plane_batch = batch;
-  plane_threads = 256;
-  int c = std::min(plan.chunk, p.n1);
-  while (c > 1 && !plane_shape_valid(256, c)) --c;
-  plan.chunk = c;
+  int c = std::min(p.chunk, p.n1);
+  while (c > 1 && !plane_shape_valid(p, 256, c)) --c;
+  p.chunk = c;
 }
 
 // The k kernels move a coefficient's (Re, Im) as one 16-byte access.
@@ -878,10 +880,11 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   size_t lds_max = size_t(prop.sharedMemPerBlock);
   if (!kb && fft32() && (plan.xshape.on || (!plan.lines.empty() && pair_shape(plan.n1, plan.n2, plan.Z, elem).on))) {
     dplan = build_stick_plan(s, false, elem);
-    // (FP32 densities beyond one workgroup's passes take the paired pass; a
-    // mixed operator then has the radix passes alone.)
-    plain = fft_fits(dplan.Z, dplan.ry) && plane_lds(dplan, elem) <= lds_max;
-    if (keeps_rounding() && !plain) plan = dplan;
+    // Planes beyond one workgroup's passes: mixed solves split them, FP32
+    // densities take the paired pass.
+    if (!fft_fits(dplan.Z, dplan.ry) || plane_lds(dplan, elem) > lds_max) plain_split = keeps_rounding();
+    else plain = true;
+    plain = plain || plain_split;
   }
   if (stick_lds(plan, elem) > lds_max) fail(BD_ERR_INVALID_PARAMETER, "x FFT tile exceeds the device LDS");
   if (fft32()) allow_lds<float>(plan);
@@ -934,10 +937,11 @@ GammaOp::GammaOp(const System& s, const KBasis* k, int cap, int prec) : sys(&s),
   }
   const int pairs = slots(cap);
   int spad = plan.Spad;
+  if (plain_split) split_plan(dplan, 0, true);
   if (plain) {
     // Large planes: 512 threads and the longest row chunk, as the shape search
     // picks there (the bits do not depend on the shape).
-    if (dplan.n1 * dplan.n2 >= 64 * 64 && fft_fits_threads(dplan.Z, dplan.ry, 512))
+    if (!plain_split && dplan.n1 * dplan.n2 >= 64 * 64 && fft_fits_threads(dplan.Z, dplan.ry, 512))
       for (int c = dplan.n1; c > dplan.chunk; --c) {
         StickPlan wide = dplan;
         wide.chunk = c;
@@ -1023,8 +1027,8 @@ void GammaOp::refresh_potential32() {
 // MODE 0 transforms the sticks in place with V(r); MODE 1 sums the band
 // density into kDensityGroups-style group partials at rho_part.
 template <int MODE, typename F, int NT>
-void GammaOp::split_pass(int pairs, const F* pot, const double* w, double* rho_part) {
-  const StickPlan& p = plan;
+void GammaOp::split_pass(const StickPlan& p, const int2* yz, int pairs, const F* pot, const double* w,
+                         double* rho_part) {
   const size_t e = sizeof(c2<F>);
   c2<F>* sticks = reinterpret_cast<c2<F>*>(d_sticks.p);
   c2<F>* planes = reinterpret_cast<c2<F>*>(d_planes.p);
@@ -1034,12 +1038,12 @@ void GammaOp::split_pass(int pairs, const F* pot, const double* w, double* rho_p
   for (int t0 = 0; t0 < pairs; t0 += plane_batch) {
     const int bp = std::min(plane_batch, pairs - t0);
     hipLaunchKernelGGL((k_plane_y<true, F, NT>), dim3(bp, p.n0, zbatches), dim3(NT), ly, stream, sticks, p.n0, p.n1,
-                       p.Spad, p.Z, p.zb, d_stick_yz.p, d_roots.p, p.ry, t0, planes);
+                       p.Spad, p.Z, p.zb, yz, d_roots.p, p.ry, t0, planes);
     if (MODE == 0) {
       hipLaunchKernelGGL((k_plane_z<0, F, NT>), dim3(bp, p.n0, ychunks), dim3(NT), lz, stream, planes, p.n0, p.n1,
                          p.n2, p.Z, p.chunk, d_zc.p, d_roots.p, p.rz, pot, bp, t0, pairs, nullptr, 0.0, 0, nullptr);
       hipLaunchKernelGGL((k_plane_y<false, F, NT>), dim3(bp, p.n0, zbatches), dim3(NT), ly, stream, sticks, p.n0,
-                         p.n1, p.Spad, p.Z, p.zb, d_stick_yz.p, d_roots.p, p.ry, t0, planes);
+                         p.n1, p.Spad, p.Z, p.zb, yz, d_roots.p, p.ry, t0, planes);
     } else {
       hipLaunchKernelGGL((k_plane_z<1, F, NT>), dim3(p.n0, ychunks, groups), dim3(NT), lz, stream, planes, p.n0,
                          p.n1, p.n2, p.Z, p.chunk, d_zc.p, d_roots.p, p.rz, nullptr, bp, t0, pairs, w,
@@ -1143,10 +1147,14 @@ void GammaOp::plain_apply(const double* x, int64_t ldx, int m, double* y, int64_
   if (profiling) BD_HIP(hipEventRecord(ev[0], stream));
   plain_to_sticks(x, ldx, m);
   if (profiling) BD_HIP(hipEventRecord(ev[1], stream));
-  const auto plane = plain_threads == 512 ? &k_plane<0, float, 512> : &k_plane<0, float, 256>;
-  hipLaunchKernelGGL(plane, dim3(pairs, p.n0), dim3(plain_threads), plane_lds(p, e), stream, sticks, p.n0, p.n1, p.n2,
-                     p.Spad, p.Z, p.chunk, d_dyz.p, d_zc.p, d_roots.p, p.ry, p.rz, d_potential32.p, pairs, nullptr,
-                     0.0, nullptr, nullptr);
+  if (plain_split) {
+    split_pass<0, float, 256>(p, d_dyz.p, pairs, d_potential32.p, nullptr, nullptr);
+  } else {
+    const auto plane = plain_threads == 512 ? &k_plane<0, float, 512> : &k_plane<0, float, 256>;
+    hipLaunchKernelGGL(plane, dim3(pairs, p.n0), dim3(plain_threads), plane_lds(p, e), stream, sticks, p.n0, p.n1,
+                       p.n2, p.Spad, p.Z, p.chunk, d_dyz.p, d_zc.p, d_roots.p, p.ry, p.rz, d_potential32.p, pairs,
+                       nullptr, 0.0, nullptr, nullptr);
+  }
   if (profiling) BD_HIP(hipEventRecord(ev[2], stream));
   hipLaunchKernelGGL(k_stick_forward<float>, dim3(p.ntiles, pairs), dim3(kThreads), stick_lds(p, e), stream, x, ldx, y,
                      ldy, m, p.n0, p.T, p.Spad, d_dtile_off.p, d_dentries.p, d_ddst.p, d_roots.p, p.rx, sticks,
@@ -1171,8 +1179,8 @@ void GammaOp::local_apply(const double* x, int64_t ldx, int m, double* y, int64_
     pair_launch<F>(stream, pair, 0, a, 1);
     sticks = a.out;
   } else if (p.zb > 0) {
-    if (plane_threads == 512) split_pass<0, F, 512>(pairs, pot, nullptr, nullptr);
-    else split_pass<0, F, 256>(pairs, pot, nullptr, nullptr);
+    if (plane_threads == 512) split_pass<0, F, 512>(p, d_stick_yz.p, pairs, pot, nullptr, nullptr);
+    else split_pass<0, F, 256>(p, d_stick_yz.p, pairs, pot, nullptr, nullptr);
   } else if (plane_threads == 512) {
     hipLaunchKernelGGL((k_plane<0, F, 512>), dim3(pairs, p.n0), dim3(512), plane_lds(p, e), stream, sticks, p.n0,
                        p.n1, p.n2, p.Spad, p.Z, p.chunk, d_stick_yz.p, d_zc.p, d_roots.p, p.ry, p.rz, pot, pairs,
@@ -1214,8 +1222,8 @@ void GammaOp::density(const double* x, int64_t ldx, int m, const double* w, doub
     a.rho = d_rho_part.p;
     pair_launch<F>(stream, pair, 1, a, groups);
   } else if (p.zb > 0) {
-    if (plane_threads == 512) split_pass<1, F, 512>(pairs, nullptr, w, d_rho_part.p);
-    else split_pass<1, F, 256>(pairs, nullptr, w, d_rho_part.p);
+    if (plane_threads == 512) split_pass<1, F, 512>(p, d_stick_yz.p, pairs, nullptr, w, d_rho_part.p);
+    else split_pass<1, F, 256>(p, d_stick_yz.p, pairs, nullptr, w, d_rho_part.p);
   } else if (plane_threads == 512)
     hipLaunchKernelGGL((k_plane<1, F, 512>), dim3(p.n0, groups), dim3(512), plane_lds(p, e), stream, sticks, p.n0,
                        p.n1, p.n2, p.Spad, p.Z, p.chunk, d_stick_yz.p, d_zc.p, d_roots.p, p.ry, p.rz, nullptr,

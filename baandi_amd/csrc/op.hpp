@@ -155,6 +155,7 @@ struct GammaOp {
   bool plain = false;
   bool plain_density() const { return plain && precision == BD_FP32_HX; }
   bool plain_solve() const { return plain && keeps_rounding(); }
+  bool plain_split = false;
   int plain_threads = 256;
   StickPlan dplan;
   DevBuf<int> d_dtile_off, d_ddst;
@@ -179,10 +180,12 @@ struct GammaOp {
   DevBuf<c2<double>> d_planes;
   int plane_batch = 0;
   size_t elem_bytes() const;
-  bool plane_shape_valid(int threads, int chunk) const;
+  bool plane_shape_valid(const StickPlan& p, int threads, int chunk) const;
+  bool plane_shape_valid(int threads, int chunk) const { return plane_shape_valid(plan, threads, chunk); }
   void enable_split(int zb);
+  void split_plan(StickPlan& p, int zb, bool buffer);
   template <int MODE, typename F, int NT>
-  void split_pass(int pairs, const F* pot, const double* w, double* rho_part);
+  void split_pass(const StickPlan& p, const int2* yz, int pairs, const F* pot, const double* w, double* rho_part);
   // Warm start (KeptHx): real-space pair fields of the last band density,
   // [pair][N] of the op's precision, and the columns they belong to.
   DevBuf<c2<double>> d_kept;
