@@ -53,8 +53,9 @@ def si64():
 
 
 def test_si64_hx_every_plane_shape(si64):
-    """Si64 H·X on 32 columns for each plane-kernel shape, against the oracle;
-    all shapes give the same bits."""
+    """Si64 H·X on 32 columns against the oracle, whatever plane-kernel shape is
+    set: the paired pass takes none of them (test_gpu_radix_passes.py runs the
+    shapes, on planes without a paired kernel)."""
     from oracle.hamiltonian import apply_orc
     torch, system, orc, op, pot = si64
     plan = op.plan_info()

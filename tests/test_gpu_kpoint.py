@@ -285,7 +285,8 @@ def _random_blocks(ops, m, seed):
 
 @pytest.mark.parametrize("betas", [False, True])
 def test_fused_matches_three_stage(betas):
-    """The fused one-workgroup-per-column kernel against the three-stage
+    """The one-workgroup-per-column kernel (here the paired one; the radix-pass
+    kernel's turn is in test_gpu_radix_passes.py) against the three-stage
     stick/plane path on the Al cell (25^3 grid): bit for bit without
     projectors (same per-line FFT arithmetic); with projectors the nonlocal
     sums differ in order only."""
@@ -334,6 +335,8 @@ def test_batch_apply_bitwise_equals_per_k():
 
 
 def test_autotuned_shape_is_bitwise_neutral():
+    """On the paired kernel, which takes no shape: the current one is timed and
+    stays (test_gpu_radix_passes.py tunes the radix-pass kernel)."""
     import torch
     system, ops = _al_ops(capacity=16)
     op = ops[0]
@@ -445,8 +448,9 @@ def test_graph_iteration_bitwise_equals_eager(kind):
 
 
 def test_plane_autotune_is_bitwise_neutral():
-    """Gamma op: the tuned k_plane shape (threads, rows per z chunk) gives the
-    same H·X bits as the default, FP64 and mixed."""
+    """Gamma op on the paired pass: tuning the k_plane shape (threads, rows per z
+    chunk), which it does not take, leaves the H·X bits, FP64 and mixed
+    (test_gpu_radix_passes.py tunes planes without a paired kernel)."""
     import torch
     from baandi_amd import lib as L
     from baandi_amd.hamiltonian import GammaSystem, DistributedRealHamiltonian

@@ -93,3 +93,35 @@ def test_plane_pass(n1, n2, precision):
     print(f"[plane] {n1}x{n2} {precision}: H·X {err:.1e} density {derr:.1e} kept {kerr:.1e} (bound {bound:.1e})",
           flush=True)
     assert err < bound and derr < bound and kerr < bound
+
+
+@pytest.mark.parametrize("n1,n2", PLANES)
+def test_mixed_density(n1, n2):
+    """The FP32 paired density (the mixed tier's; FP32 H·X operators keep the
+    radix passes for theirs) and the kept-field apply from its fields: bounds as
+    above."""
+    import torch
+    from baandi_amd import lib as L
+    from baandi_amd.hamiltonian import DistributedRealHamiltonian
+    from kernel_tables import paired_planes
+    assert (n1, n2) in paired_planes()
+    s = _cell(n1, n2)
+    g = torch.Generator(device="cuda").manual_seed(n1 * 1000 + n2)
+    x = torch.randn(3, s.n, generator=g, device="cuda", dtype=torch.float64)
+    x /= x.norm(dim=1, keepdim=True)
+    v = torch.randn(int(np.prod(s.dims)), generator=g, device="cuda", dtype=torch.float64)
+    op = DistributedRealHamiltonian(s, capacity=3, precision=L.BD_MIXED)
+    op.set_owned_potential(v)
+    psi, ref = _reference(torch, s, x, v)
+    kept = op.plane_split() == 0
+    if kept:
+        op.keep_fields(True)
+    w = np.array([2.0, 0.5, 1.0])
+    rho, z = torch.full_like(v, float("nan")), torch.zeros_like(x)
+    op.band_density_sum(x, w, rho)
+    want = (torch.from_numpy(w).cuda().view(-1, 1, 1, 1) * psi * psi).sum(dim=0).reshape(-1) / s.volume
+    bound = 100.0 * 2.0 ** -24
+    assert float((rho - want).norm() / want.norm()) < bound
+    if kept:
+        op.apply_kept(x, v, z)
+        assert float((z - ref).norm() / ref.norm()) < bound

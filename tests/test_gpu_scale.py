@@ -1,11 +1,11 @@
 """The pieces that carry the path to the Si512 cell and the SCF glue, on
 MI355X through the C ABI:
 
-* the split plane pass (planes that do not fit one workgroup's LDS go
-  through HBM): forced on small cells it gives the bits of the one-workgroup
-  plane kernel for H·X and the band density, and matches the oracle; on the
-  Si512 cell (144^3, picked automatically) H·X matches the oracle's C++
-  restatement (oracle/cpu_hx.cpp, pinned to the NumPy oracle on small cells);
+* the split-plane setting of operators on the paired pass: accepted, read back
+  and without effect on H·X and the band density (test_gpu_radix_passes.py runs
+  the split pass itself, on planes without a paired kernel); on the Si512 cell
+  (144^3, planes by row parity) H·X matches the oracle's C++ restatement
+  (oracle/cpu_hx.cpp, pinned to the NumPy oracle on small cells);
 * the tridiagonalisation across the chip (large subspaces, up to Si512's
   2252) against LAPACK, also forced on small and degenerate matrices;
 * the warm start (KeptHx): H_old X + dV X from the kept real-space fields
@@ -47,9 +47,9 @@ def _apply(op, x):
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_split_plane_pass_equals_fused(precision):
-    """Si2 at 20 Ry (24^3, Z = 11) and Si8 at 6 Ha: the split pass with 1, 3
-    and Z z-lines per batch against the one-workgroup plane kernel, bit for
-    bit, for H·X and for the band density."""
+    """Si2 at 20 Ry (24^3, Z = 11) and Si8 at 6 Ha, whose planes have a paired
+    kernel: set to split passes of 1, 3 and Z z-lines per batch, H·X and the
+    band density stay the paired pass's, bit for bit."""
     import torch
     from baandi_amd import lib as L
     from baandi_amd.hamiltonian import GammaSystem
@@ -122,8 +122,9 @@ def test_device_setup_matches_host(cell):
 
 def test_si512_hx_matches_cpu_restatement():
     """The Si512 cell (4x4x4 cells, 30 Ry, 144^3 grid, 2560 projectors): its
-    144 x Z planes exceed one workgroup's LDS in FP64, so the op runs the
-    split pass; H·X on 4 columns against the oracle's C++ restatement."""
+    144 x Z planes exceed one workgroup's LDS in FP64, so the op is set to the
+    split pass and runs the paired one by row parity; H·X on 4 columns against
+    the oracle's C++ restatement."""
     import time
     from baandi_amd import workloads as W
     from oracle.cpu_hx import CpuHamiltonian
