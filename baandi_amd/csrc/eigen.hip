@@ -4,11 +4,19 @@
 // pairs are formed, which is all the Davidson step reads.
 //
 //  1. Householder tridiagonalisation (Golub & Van Loan, Matrix Computations,
-//     4th ed., Alg. 8.3.1) in one 1024-thread workgroup: the matrix stays in
-//     the L2 of one XCD, and each step updates the trailing block and
-//     multiplies it by the next reflector in a single pass.
-//  2. Sturm-sequence bisection (Barth, Martin & Wilkinson 1967), one wave per
-//     eigenvalue with 64-point multisection per step.
+//     4th ed., Alg. 8.3.1), by size:
+//       3 <= m <= 128      k_td_one, one workgroup with its columns in registers
+//       m <= 640           k_td_coop_reg, cooperating workgroups, columns in
+//                          registers; the last 128 rows by k_td_one
+//       m <= ~736          k_td_coop, cooperating workgroups, columns in LDS (of
+//                          at most 32); also for Sums::chain from m = 128
+//       m >= 1026          k_td_column, k_td_symv, k_td_update across the chip
+//       otherwise          k_tridiag_panel (panels of 8 reflectors, one
+//                          workgroup; Sums::chain below 128) where its LDS fits
+//                          (m <= 523), else k_tridiag, one step at a time
+//     Each keeps the trailing block exactly symmetric.
+//  2. Sturm-sequence bisection (Givens 1954; Barth, Martin & Wilkinson 1967),
+//     one wave per eigenvalue with 64-point multisection per step.
 //  3. Inverse iteration with a partially pivoted tridiagonal LU (the scheme
 //     of LAPACK dlagtf/dlagts/dstein), one lane per eigenvector.
 //  4. Two passes of classical Gram-Schmidt inside clusters of close

@@ -3,7 +3,7 @@
 // the lengths of plane_kernels.hpp and stick.hip whose columns fit the LDS).
 // The column's sticks stay in LDS; a wavefront transforms sticks and then
 // whole y-z planes by itself, in its own plane buffer, so the workgroup meets
-// five times a column where one workgroup-wide pass per radix
+// four times a column where one workgroup-wide pass per radix
 // (k_hpsi_fused) met some twenty times every few planes. The arithmetic of a
 // line, V and the kinetic term are those of the paired stick/plane path: the
 // local part has its bits. One launch covers every column of every k point of

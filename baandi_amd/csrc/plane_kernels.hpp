@@ -370,10 +370,12 @@ __global__ __launch_bounds__(64 * kMaxWaves, waves_per_simd<F>(ya, A)) void k_pl
 
 // The planes the kernels are built for, as X(split, ya, yb, A, B) with
 // n1 = split ya yb and n2 = A B: the larger radix outside (A, ya), the radix
-// whose z transform runs twice around V inside (B). Equal axes at the
-// 2,3,5-smooth lengths that are a product of two radices; 128^2 and 144^2
-// also by row parity (FP64 planes beyond one workgroup's LDS); and the axes of
-// supercells one, two and three cells long at 30 to 36 points a cell.
+// whose z transform runs twice around V inside (B). Equal axes of 15 to 48, 54,
+// 60, 64, 72, 80, 90, 96, 108, 120, 128 and 144 points; 128^2 and 144^2 also by
+// row parity (FP64 planes beyond one workgroup's LDS); and unequal axes of
+// supercells one, two and three cells long at 30, 32 and 36 points a cell. A
+// kernel is compiled for each plane, mode and type: other planes (50, 75, 81,
+// 100, 135 points, other unequal axes) run the pass-per-radix kernels.
 #define BD_PLANES(X)                                                                                  \
   X(1, 5, 3, 5, 3) X(1, 5, 4, 5, 4) X(1, 6, 4, 6, 4) X(1, 5, 5, 5, 5) X(1, 9, 3, 9, 3)                \
   X(1, 6, 5, 6, 5) X(1, 8, 4, 8, 4) X(1, 6, 6, 6, 6) X(1, 8, 5, 8, 5) X(1, 9, 5, 9, 5)                \

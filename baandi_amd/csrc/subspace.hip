@@ -267,9 +267,15 @@ __global__ void k_zero_flag(int* flag, double* min_ratio) {
 }
 }  // namespace
 
-// The split-K GEMMs above use at most max(1, K/256) chunks of an M x N tile
-// with M, N, K <= cap.
-int64_t factor_gwork(int cap) { return int64_t(cap < 256 ? 1 : cap / 256) * cap * cap; }
+// Partial sums of the products above (M, N, K <= cap): up to K = 1023 at most
+// max(1, K / 256) copies of an M x N block; beyond, up to eight copies or 2^21
+// values (max_splits of gemm.hip), of which cap / 256 >= 4 copies of cap x cap
+// hold either. gemm_tn_work is monotone, so its value at cap covers them all.
+int64_t factor_gwork(int cap) {
+  const int64_t size = int64_t(cap < 256 ? 1 : cap / 256) * cap * cap;
+  if (size < gemm_tn_work(cap, cap, cap)) fail(BD_ERR_APPLICATION, "factor workspace below its products' partial sums");
+  return size;
+}
 
 namespace {
 // Widest border block k_chol_inv_lds holds: its rows live in the kInvRows

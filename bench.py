@@ -8,8 +8,8 @@ a = 20.52 Bohr, Gamma, 30 Ry, 160 bands, 128 occupied, synthetic Z=4
 pseudopotential, seeded N(0,1) start) to dr2 < 1e-8 Ry, with all inputs
 already resident on the GPU. Prints one JSON line.
 
-The roofline object covers the dominant H·X kernel (k_plane: y/z transforms
-with the V(r) multiply), timed with HIP events on the operator's stream over
+The roofline object covers the dominant H·X kernel (k_plane_pair: y/z transforms
+with the V(r) multiply), its compulsory bytes over its time, timed with HIP events on the operator's stream over
 the timed region. The CPU baseline times the oracle's C++ FP64 H·X (all host
 threads, and one) on a bounded sample of the same Si64 columns. Side legs
 (untimed by the step clock): the subspace GEMMs, the Al 6x6x6 k-point SCF,
@@ -31,25 +31,18 @@ sys.path.insert(0, ROOT)
 os.environ["GPU_MAX_HW_QUEUES"] = "16"
 
 HBM_PEAK_GBS = 8000.0
-# Measured HBM bytes per pair of k_plane at Si64 FP64 (autotuned 512-thread shape):
-# rocprofv3 FETCH_SIZE (x2.000, the 256 MiB copy calibration) + WRITE_SIZE (x1.000)
-# of an 80-pair launch, 204066.0 KiB / 80 pairs (profiles/k_plane_si64_fp64.txt).
-PLANE_TRAFFIC_BYTES_PER_PAIR = 204066.0 * 1024 / 80
+# Measured HBM bytes per pair of k_plane_pair at Si64 FP64: rocprofv3 FETCH_SIZE
+# (56773.5 KiB, x2.000, the 256 MiB copy calibration) + WRITE_SIZE (89820.0 KiB,
+# x1.000) of an 80-pair launch (profiles/measured_workloads.txt).
+PLANE_TRAFFIC_BYTES_PER_PAIR = 203367.0 * 1024 / 80
 METRIC = "Si64 SCF wall-time to 1e-8 Ha/atom: mixed+learned vs plain FP64, 1 MI355X"
 
 
-def plane_bytes_model(plan, pairs, c=16, r=8):
-    """Algorithmic bytes of the y and z stages of the 3-pass pencil model
-    (per pair 4 c (Z n1 n0 + N) + r N for V), for `pairs` pairs."""
-    n0, n1, n2, Z = plan["n0"], plan["n1"], plan["n2"], plan["z_planes"]
-    N = n0 * n1 * n2
-    return pairs * (4 * c * (Z * n1 * n0 + N) + r * N)
-
-
-def fused_bytes(plan, pairs, c=16, r=8):
-    """Compulsory HBM bytes of k_plane as built: sticks in and out, V once."""
+def plane_bytes(plan, pairs, launches=1, c=16, r=8):
+    """Compulsory HBM bytes of the plane pass, whose planes stay in LDS: the
+    sticks in and out, V once a launch."""
     n0, n1, n2 = plan["n0"], plan["n1"], plan["n2"]
-    return 2 * c * pairs * n0 * plan["sticks"] + r * n0 * n1 * n2
+    return 2 * c * pairs * n0 * plan["sticks"] + launches * r * n0 * n1 * n2
 
 
 def cpu_baseline(system, columns=160, reps=3):
@@ -269,7 +262,7 @@ def si512_leg(iterations=2, reps=2):
     """Si512 (4x4x4 conventional cells, displaced N(0, 0.03 Bohr), Gamma,
     30 Ry, 1126 bands, 1024 occupied) at the potential of the Gaussian start
     density: the set-up with its atom loops on the GPU, the H·X of the full
-    1126-column block (split plane pass, 144^3 grid) in FP64 and in the mixed
+    1126-column block (144^3 grid, planes by row parity) in FP64 and in the mixed
     tier, and `iterations` FP64 Davidson iterations from a seeded start
     (subspace up to 2252), each timed."""
     import numpy as np
@@ -312,12 +305,12 @@ def si512_leg(iterations=2, reps=2):
         plan = op.plan_info()
         plane_ms = st["plane"] / reps
         c = 16 if prec == L.BD_FP64 else 8
-        model = plane_bytes_model(plan, st["pairs"] / reps, c=c, r=c // 2)
+        moved = plane_bytes(plan, st["pairs"] / reps, c=c, r=c // 2)
         entry = {"hx_ms": round(ms, 2), "columns": bands, "plane_split_z_lines": op.plane_split(),
                  "stage_ms": {k: round(v / reps, 3) for k, v in st.items()
                               if k not in ("applies", "pairs", "columns")},
-                 "plane_model_GBs": round(model / (plane_ms * 1e-3) / 1e9, 1) if plane_ms > 0 else None,
-                 "plane_frac_hbm": round(model / (plane_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if plane_ms > 0 else None}
+                 "plane_compulsory_GBs": round(moved / (plane_ms * 1e-3) / 1e9, 1) if plane_ms > 0 else None,
+                 "plane_frac_hbm": round(moved / (plane_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if plane_ms > 0 else None}
         if ref_y is None:
             ref_y = y.clone()
             entry["plan"] = plan
@@ -506,9 +499,8 @@ def main():
     plan = last["plan"]
     launches = st["applies"]
     plane_ms = st["plane"]
-    achieved = plane_bytes_model(plan, st["pairs"]) / (plane_ms * 1e-3) / 1e9 if plane_ms > 0 else 0.0
-    fused = fused_bytes(plan, st["pairs"]) / (plane_ms * 1e-3) / 1e9 if plane_ms > 0 else 0.0
-    per_launch_bytes = plane_bytes_model(plan, st["pairs"] / max(launches, 1))
+    moved = plane_bytes(plan, st["pairs"], launches)
+    achieved = moved / (plane_ms * 1e-3) / 1e9 if plane_ms > 0 else 0.0
     ms_per_step = 1e3 * sum(walls) / len(walls)
     out = {
         "metric": METRIC,
@@ -539,17 +531,17 @@ def main():
         "breakdown_s": {k: round(v, 4) for k, v in last["totals"].items() if k.endswith("_s")},
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_plane",
+            "kernel": "k_plane_pair",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": round(PLANE_TRAFFIC_BYTES_PER_PAIR * st["pairs"] / max(launches, 1)),
-            "model": "3-pass pencil model, y+z stages: 4*16*(Z*n1*n0+N)+8*N bytes per pair",
-            "bytes_per_launch_avg": per_launch_bytes,
+            "model": "compulsory: 2*16*n0*S bytes a pair (sticks in and out) + 8*N a launch (V); the kernel is "
+                     "bound by LDS and FP64 issue, not by these bytes",
+            "bytes_per_launch_avg": moved / max(launches, 1),
             "avg_launch_ms": round(plane_ms / max(launches, 1), 4),
             "launches": launches,
-            "fused_compulsory_GBs": round(fused, 1),
         },
     }
     out["subspace_gemms"] = gemm_leg()

@@ -223,17 +223,20 @@ bd_status bd_k_batch_apply_dev(bd_k_batch* batch, const double* const* x_dev, co
                                const int32_t* m, double* const* y_dev, const int64_t* ldy);
 /* Launch-shape autotuner of the fused kernel: times every valid (threads,
  * sticks per x-FFT batch, rows per z-FFT batch, y-z planes per pass) on m
- * columns, reps launches each, keeps the fastest.
+ * columns, reps launches each, keeps the fastest. Gamma ops: the plane
+ * kernel's (threads, rows a z chunk) instead. Ops on a paired kernel take no
+ * shape: the current one is timed and stays.
  * out5: threads, xlines, zrows, xplanes, microseconds per launch. */
 bd_status bd_gamma_op_autotune(bd_gamma_op* op, int32_t m, int32_t reps, double* out5);
 /* Read (set = 0) or set the fused shape (threads, xlines, zrows, xplanes);
- * threads = 0 selects the three-stage path. */
+ * threads = 0 selects the three-stage path. Cubes with a paired column kernel
+ * (BD_CUBES of csrc/kpair.hip) run it at any other shape. */
 bd_status bd_gamma_op_fused_shape(bd_gamma_op* op, int32_t* inout4, int32_t set);
 /* Read (set = 0) or set the plane kernel's shape on the stick/plane path
  * (threads 256 or 512, y rows per z-FFT chunk); set accepts the shapes the
  * autotuner may pick. All shapes give the same bits. Gamma ops whose plane has
- * a kernel of the paired pass (both lengths a product of two radices) run that
- * one whatever the shape says. */
+ * a kernel of the paired pass (the list BD_PLANES of csrc/plane_kernels.hpp)
+ * run that one whatever the shape says. */
 bd_status bd_gamma_op_plane_shape(bd_gamma_op* op, int32_t* inout2, int32_t set);
 /* Read (set = 0) or set the plane pass: 0 = one workgroup per y-z plane
  * (only where the Z x n1 plane fits the LDS), zb > 0 = the split pass, which
@@ -474,10 +477,11 @@ bd_status bd_herm_eigen_dev(int32_t m, int32_t want, double* A, int64_t lda, dou
 bd_status bd_sym_eigen_multi_from(int32_t* inout, int32_t set);
 /* Read (set = 0) or set {workers, from, to, spins} of the cooperative
  * tridiagonalisation: for from <= m <= to (and below the multi_from size) the
- * matrix is split by columns over the LDS of `workers` workgroups (more
- * where the columns do not fit, at most 32; -1: m/10 clamped to 8..32),
- * which pass each reflector and each product through tagged words in device
- * memory; workers = 0 keeps the one-workgroup panel kernel. A worker that
+ * matrix is split by columns over `workers` workgroups (more where the columns
+ * do not fit, at most 32; -1: m/10 clamped to 8..32, and up to 128 rows, as
+ * well as the last 128 of a larger matrix, in one workgroup), which pass the
+ * products and the column two ahead through tagged words in device memory;
+ * workers = 0 keeps the one-workgroup panel kernel. A worker that
  * polls a word more than `spins` times (at once when spins < 0) abandons the
  * solve, which then fails like any eigensolve (the Davidson redoes it with
  * the one-step kernel). Default {-1, 128, 1025, 2097152}. */
