@@ -1135,6 +1135,10 @@ __global__ __launch_bounds__(kCT) void k_td_coop_reg(int m, int nw, int steps, d
     c2[t] = entry(r, 0);
     c1[t] = entry(r, 1);
   }
+  // A is read before this wave publishes anything: with one step (m = 129) the
+  // owners write the trailing columns into A right after the first exchange,
+  // and column 1's loads are not waited for until then.
+  __threadfence();
   double tk = 0.0;
   // Reflector k from `col` (column k as of step k - 1): v (zero up to row k),
   // tau; d, e and tau by one wave, the owner keeps v for the end.
