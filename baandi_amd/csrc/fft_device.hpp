@@ -19,9 +19,9 @@ struct c2 {
   T x, y;
 };
 
-// The paired passes' arithmetic is written out with its fused multiply-adds,
-// and the compiler adds none of its own (fp contract(off)): the same line has
-// the same bits in every one of their kernels.
+// The transforms' arithmetic is written out with its fused multiply-adds, and
+// the compiler adds none of its own (fp contract(off)): the same line has the
+// same bits in every kernel that transforms it. (Not so in `plain` below.)
 template <typename T>
 __host__ __device__ __forceinline__ T fma_of(T a, T b, T c) {
   if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
@@ -239,10 +239,10 @@ __host__ __device__ __forceinline__ void dft(c2<T>* v) {
 }
 
 // The same transforms of 2, 3, 4, 5, 8 and 9 points with the products and sums
-// left to the compiler's contraction: the arithmetic of the radix passes
-// (stockham_pass). The mixed tier's solves run on them (system potentials
-// included) and turn any other rounding into another result at the scale of
-// their thresholds (GammaOp::keeps_rounding), so it does not change.
+// left to the compiler's contraction: the arithmetic of the FP32 radix passes and
+// of the FP64 field transforms (the potentials). The mixed tier's solves run on
+// these and turn any other rounding into another result at the scale of their
+// thresholds (GammaOp::keeps_rounding), so it does not change.
 namespace plain {
 template <typename T>
 __device__ __forceinline__ c2<T> cadd(c2<T> a, c2<T> b) { return {a.x + b.x, a.y + b.y}; }
@@ -348,8 +348,8 @@ __device__ __forceinline__ void dft(c2<T>* v) {
 
 // One in-place Stockham pass (radix R, Ns = product of earlier radices).
 // `roots[k]` = e^{-2 pi i k/n} (forward); the inverse conjugates. A workgroup
-// of NT threads holds pass_mb(R, NT) butterflies per thread.
-template <int R, bool INV, typename T, int NT>
+// of NT threads holds pass_mb(R, NT) butterflies per thread. PLAIN: `plain`.
+template <int R, bool INV, typename T, int NT, bool PLAIN>
 __device__ __forceinline__ void stockham_pass(c2<T>* lds, int nlines, int lstride, int estride,
                                               int n, int Ns, const c2<T>* roots) {
   static_assert(NT == 256 || NT == 512, "workgroups of 256 or 512 threads");
@@ -372,11 +372,13 @@ __device__ __forceinline__ void stockham_pass(c2<T>* lds, int nlines, int lstrid
         if (r > 0) {
           c2<T> w = roots[jm * r * ts];
           if (INV) w.y = -w.y;
-          a = plain::cmul(a, w);
+          if constexpr (PLAIN) a = plain::cmul(a, w);
+          else a = cmul(a, w);
         }
         v[k][r] = a;
       }
-      plain::dft<R, INV>(v[k]);
+      if constexpr (PLAIN) plain::dft<R, INV>(v[k]);
+      else dft<R, INV>(v[k]);
     }
   }
   __syncthreads();
@@ -397,18 +399,18 @@ __device__ __forceinline__ void stockham_pass(c2<T>* lds, int nlines, int lstrid
 
 // Full 1D transform of every line by a workgroup of NT threads (blockDim.x
 // == NT). The caller synchronises before the call; the call ends synchronised.
-template <bool INV, typename T, int NT = 256>
+template <bool INV, typename T, int NT = 256, bool PLAIN = sizeof(T) == 4>
 __device__ void lds_fft(c2<T>* lds, int nlines, int lstride, int estride, const RadixPlan& rp,
                         const c2<T>* roots) {
   int Ns = 1;
   for (int p = 0; p < rp.count; ++p) {
     const int R = rp.radix[p];
-    if (R == 8) stockham_pass<8, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
-    else if (R == 9) stockham_pass<9, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
-    else if (R == 4) stockham_pass<4, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
-    else if (R == 2) stockham_pass<2, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
-    else if (R == 3) stockham_pass<3, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
-    else stockham_pass<5, INV, T, NT>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    if (R == 8) stockham_pass<8, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    else if (R == 9) stockham_pass<9, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    else if (R == 4) stockham_pass<4, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    else if (R == 2) stockham_pass<2, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    else if (R == 3) stockham_pass<3, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
+    else stockham_pass<5, INV, T, NT, PLAIN>(lds, nlines, lstride, estride, rp.n, Ns, roots);
     Ns *= R;
   }
 }

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kFT) void k_grid_fft(c2<double>* __restrict__ g, in
     L[b * n + i] = b < nb ? g[base + b * bstride + i * step] : c2<double>{0.0, 0.0};
   }
   __syncthreads();
-  lds_fft<INV, double, kFT>(L, B, n, 1, rp, rt);
+  lds_fft<INV, double, kFT, true>(L, B, n, 1, rp, rt);
   for (int e = threadIdx.x; e < nb * n; e += blockDim.x) {
     const int i = e / nb, b = e - i * nb;
     g[base + b * bstride + i * step] = L[b * n + i];

@@ -52,17 +52,18 @@ __global__ void k_copy_block(int k, const double* __restrict__ S, int64_t lds, d
 // already set by an earlier block of the same border leaves the block
 // untouched; min_ratio keeps the minimum over the blocks.
 //
-// G = L L^T: column l of the elimination sits in the registers of wave l mod 16
-// (lane i owns row i, and i + 64 past 64 rows), and a step passes one column
-// through LDS: one barrier, one division (by the pivot d_j; L's column is the
-// passed one over sqrt(d_j), formed for all columns at the end). The pivots are
-// tested together then, too (a failed one only spoils later columns, which
-// nobody reads). L^{-1} by forward substitution, a wave's columns side by side
-// so that their chains (a lane read, a product and the update) overlap.
-// Bound by the chain of steps. k = 80: 55 us, k = 20: 8; 98 and 16, with the
-// same bits, with the block as a packed triangle in LDS, two divisions a step
-// and one column at a time in the substitution.
-template <int NC>
+// G = M D M^T with M unit lower: column l sits in the registers of wave
+// l mod 16 (lane i owns row i, and i + 64 past 64 rows), and a step passes one column
+// through LDS: one barrier, one division. The pivots are tested together at
+// the end (a failed one only spoils later columns, which nobody then reads).
+// M^{-1} by forward substitution, a wave's columns side by side so that their
+// chains (a lane read and the update) overlap; L^{-1} = D^{-1/2} M^{-1}.
+// CHAIN (Sums::chain, GammaOp::keeps_rounding): the rounding of G = L L^T, L's
+// columns those of the elimination over sqrt(d_j), the substitution on L.
+// Bound by the chain of steps. k = 80: 51 us, k = 20: 7 (CHAIN 60 and 8); 98 and
+// 16, with CHAIN's bits, with the block as a packed triangle in LDS, two
+// divisions a step and one column at a time in the substitution.
+template <int NC, bool CHAIN>
 __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __restrict__ G,
                                                       const double* __restrict__ sdiag, int64_t sstride,
                                                       double* __restrict__ T22, int64_t ldt, int* __restrict__ flag,
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
   const int ldm = k + 1;
   double* M = sh;                        // k columns of ldm
   double* pass = M + int64_t(k) * ldm;   // two slots of k: the column of a step
-  double* dv = pass + 2 * k;             // k: the pivots, then 1 / sqrt of them
+  double* dv = pass + 2 * k;             // k: the pivots (CHAIN: then 1 / sqrt of them)
   double a[NC][R];
   int row[R];  // this lane's rows, the last one's for those past it
 #pragma unroll
@@ -111,8 +112,13 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
 #pragma unroll
       for (int c = jc; c < NC; ++c) alj[c] = col[min(wave + nw * c, k - 1)];
       const double inv_d = 1.0 / dj;
+      if (CHAIN) {
 #pragma unroll
-      for (int c = jc; c < NC; ++c) alj[c] *= inv_d;
+        for (int c = jc; c < NC; ++c) alj[c] *= inv_d;
+      } else {
+#pragma unroll
+        for (int t = 0; t < R; ++t) mine[t] *= inv_d;
+      }
 #pragma unroll
       for (int c = jc; c < NC; ++c)
 #pragma unroll
@@ -146,15 +152,16 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
     if (failed) flag[0] = 1;
   }
   if (failed) return;  // every wave found the same: uniform exit
-  // M = L below the diagonal.
-  for (int l = wave; l < k; l += nw) {
-    const double sd = sqrt(dv[l]);
-    for (int i = l + 1 + lane; i < k; i += 64) M[i + int64_t(l) * ldm] /= sd;
+  if (CHAIN) {  // M = L below the diagonal
+    for (int l = wave; l < k; l += nw) {
+      const double sd = sqrt(dv[l]);
+      for (int i = l + 1 + lane; i < k; i += 64) M[i + int64_t(l) * ldm] /= sd;
+    }
+    __syncthreads();
+    for (int l = tid; l < k; l += kCT) dv[l] = 1.0 / sqrt(dv[l]);
+    __syncthreads();
   }
-  __syncthreads();
-  for (int l = tid; l < k; l += kCT) dv[l] = 1.0 / sqrt(dv[l]);
-  __syncthreads();
-  double x[NC][R], ml[R], rl = dv[0];  // (M is zero up to the diagonal)
+  double x[NC][R], ml[R], rl = CHAIN ? dv[0] : 1.0;  // (M is zero up to the diagonal)
 #pragma unroll
   for (int t = 0; t < R; ++t) {
     ml[t] = M[row[t]];
@@ -168,10 +175,10 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
       double next[R];
 #pragma unroll
       for (int t = 0; t < R; ++t) next[t] = M[row[t] + int64_t(min(l + 1, k - 1)) * ldm];
-      const double next_rl = dv[min(l + 1, k - 1)];
+      const double next_rl = CHAIN ? dv[min(l + 1, k - 1)] : 1.0;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        const double xl = read_lane(x[c][tl], l - 64 * tl) * rl;
+        const double xl = CHAIN ? read_lane(x[c][tl], l - 64 * tl) * rl : read_lane(x[c][tl], l - 64 * tl);
 #pragma unroll
         for (int t = 0; t < R; ++t) x[c][t] = fma(-ml[t], xl, x[c][t]);
       }
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
   for (int t = 0; t < R; ++t) {
     const int i = lane + 64 * t;
     if (i >= k) continue;
-    const double rs = dv[i];
+    const double rs = CHAIN ? dv[i] : 1.0 / sqrt(dv[i]);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int l = wave + nw * c;
@@ -194,16 +201,17 @@ __global__ __launch_bounds__(kCT) void k_chol_inv_lds(int k, const double* __res
 }
 
 typedef void (*CholInv)(int, const double*, const double*, int64_t, double*, int64_t, int*, double*);
+template <bool CHAIN>
 CholInv chol_inv_kernel(int k) {
   switch ((k * 64 + kCT - 1) / kCT) {  // columns a wave
-    case 1: return &k_chol_inv_lds<1>;
-    case 2: return &k_chol_inv_lds<2>;
-    case 3: return &k_chol_inv_lds<3>;
-    case 4: return &k_chol_inv_lds<4>;
-    case 5: return &k_chol_inv_lds<5>;
-    case 6: return &k_chol_inv_lds<6>;
-    case 7: return &k_chol_inv_lds<7>;
-    case 8: return &k_chol_inv_lds<8>;
+    case 1: return &k_chol_inv_lds<1, CHAIN>;
+    case 2: return &k_chol_inv_lds<2, CHAIN>;
+    case 3: return &k_chol_inv_lds<3, CHAIN>;
+    case 4: return &k_chol_inv_lds<4, CHAIN>;
+    case 5: return &k_chol_inv_lds<5, CHAIN>;
+    case 6: return &k_chol_inv_lds<6, CHAIN>;
+    case 7: return &k_chol_inv_lds<7, CHAIN>;
+    case 8: return &k_chol_inv_lds<8, CHAIN>;
   }
   return nullptr;
 }
@@ -296,7 +304,7 @@ void extend_block(hipStream_t s, const double* S, double* T, int cap, int from, 
   double* T22 = T + from + int64_t(from) * cap;
   const size_t lds = (size_t(k) * (k + 1) + 3 * size_t(k)) * 8;
   if (k > kFactorBlock || lds > 160 * 1024) fail(BD_ERR_INVALID_PARAMETER, "inverse Cholesky block too large");
-  const CholInv chol = chol_inv_kernel(k);
+  const CholInv chol = fw.gemm.sums == Sums::chain ? chol_inv_kernel<true>(k) : chol_inv_kernel<false>(k);
   if (lds > 64 * 1024) allow_full_lds(reinterpret_cast<const void*>(chol), "k_chol_inv_lds");
   hipLaunchKernelGGL(chol, dim3(1), dim3(kCT), lds, s, k, fw.G, S + from + int64_t(from) * cap,
                      int64_t(cap) + 1, T22, int64_t(cap), fw.flag, fw.min_ratio);
